@@ -300,33 +300,32 @@ hipError_t launch_combine(const AttnArgs & a, hipStream_t st, hipEvent_t ev0, hi
 // segments 0 .. pos / a.seg in order: each output is a function of its position and the store only, whatever the
 // chunking of the prefill.
 
-// 32 values of scale block b (dims 32 b .. 32 b + 31) of one staged row of B bits -> 16 fp16 pairs fp16_rn(d q), the
-// same values as the decode operands (kfrag)
+// 32 values of scale block b (dims 32 b .. 32 b + 31) of one staged row of B bits -> 16 fp16 pairs fp16_rn(d q) in
+// pair order (pair i of word w: o[4 w + i]), the same values as the decode operands (kfrag)
 template <int B>
 __device__ __forceinline__ void dequant_block(const uint8_t * row, uint16_t sc, int b, half2v (&o)[16]) {
     const half2v d2 = as_h2((unsigned) sc * 0x10001u);
-    constexpr float bias = B == 8 ? 1152.f : (float) (1024 + (1 << (B - 1)));
-    const half2v b2 = {(_Float16) -bias, (_Float16) -bias};
+    unsigned W[B == 8 ? 8 : 4], H[3] = {0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < (B == 8 ? 2 : 1); i++) {
+        const uint4 x = reinterpret_cast<const uint4 *>(row + (B == 8 ? 32 : 16) * b)[i];
+        W[4 * i] = x.x;
+        W[4 * i + 1] = x.y;
+        W[4 * i + 2] = x.z;
+        W[4 * i + 3] = x.w;
+    }
+    if constexpr (B < 8) {
+        constexpr int HB = B - 4;
+#pragma unroll
+        for (int i = 0; i < HB; i++) H[i] = reinterpret_cast<const unsigned *>(row + 128 + 4 * HB * b)[i];
+    }
 #pragma unroll
     for (int w = 0; w < 4; w++) {
-        unsigned lo, hi;
-        if constexpr (B == 8) {
-            const uint2 x = *reinterpret_cast<const uint2 *>(row + 32 * b + 8 * w);
-            lo = x.x ^ 0x80808080u;
-            hi = x.y ^ 0x80808080u;
-        } else {
-            constexpr int HB = B - 4;
-            const int word = 4 * b + w;
-            const unsigned W = *reinterpret_cast<const unsigned *>(row + 4 * word);
-            unsigned H = 0;
+        unsigned p[4];
+        if constexpr (B == 8) q8_pairs(W[2 * w], W[2 * w + 1], p);
+        else code_pairs<B>(W[w], hi_dword<B - 4>(H, w), hi_part<B - 4>(w), p);
 #pragma unroll
-            for (int k = 0; k < HB; k++) H |= (unsigned) row[128 + word * HB + k] << (8 * k);
-            word_codes<B>(W, H, lo, hi);
-        }
-        o[4 * w] = (as_h2(perm_b32(lo, C64, 0x00050004u)) + b2) * d2;
-        o[4 * w + 1] = (as_h2(perm_b32(lo, C64, 0x00070006u)) + b2) * d2;
-        o[4 * w + 2] = (as_h2(perm_b32(hi, C64, 0x00050004u)) + b2) * d2;
-        o[4 * w + 3] = (as_h2(perm_b32(hi, C64, 0x00070006u)) + b2) * d2;
+        for (int i = 0; i < 4; i++) o[4 * w + i] = pair_operand(p[i], i < 2 ? CodeBias<B>::lo : CodeBias<B>::hi, d2);
     }
 }
 
@@ -488,9 +487,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             float v[4] = {x.x, x.y, x.z, x.w};
             if (a.qnw) qk_prep(v, a.qnw, a.rope + (size_t) (a.n0 + t) * 32);
             if (a.krot) fwht256_w64(v);
-            o0[0] = (_Float16) (v[0] * 0.0625f);
-            o0[1] = (_Float16) (v[1] * 0.0625f);
-            o1[0] = (_Float16) (v[2] * 0.0625f);
+            o0[0] = (_Float16) (v[0] * 0.0625f); // (pair order, as the K rows of the fp16 tile)
+            o0[1] = (_Float16) (v[2] * 0.0625f);
+            o1[0] = (_Float16) (v[1] * 0.0625f);
             o1[1] = (_Float16) (v[3] * 0.0625f);
         }
         *reinterpret_cast<uint2 *>(qs + rl * SK_LD + 4 * lane) = make_uint2(as_u(o0), as_u(o1));
@@ -623,7 +622,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
             for (int j = 0; j < 4; j++)
                 *reinterpret_cast<float4 *>(dst + 32 * db + 8 * j + 4 * hf) =
-                    make_float4(O[db][4 * j], O[db][4 * j + 1], O[db][4 * j + 2], O[db][4 * j + 3]);
+                    make_float4(O[db][4 * j], O[db][4 * j + 2], O[db][4 * j + 1], O[db][4 * j + 3]); // (V's dims are in pair order)
     }
 }
 

@@ -15,9 +15,9 @@
 //                 section below).  Two 16-position subtiles.
 //   softmax       lane (n, quarter q) owns the scores of its row at positions 4q..4q+3 and 16+4q..16+4q+3: 8 values,
 //                 max / sum across the 4 quarters by v_permlane16/32_swap; exp2 in log2 units.
-//   O += P V      the MFMA's K as 16 positions x 2 adjacent dims: A = two adjacent dims of one position of V,
+//   O += P V      the MFMA's K as 16 positions x 2 dims: A = one pair of dims of one position of V,
 //                 B = P in the (row, dim parity) column pairs.
-// Dequantization happens in registers with the 0x6400 magic (kv_dev.h): fp16 values half_rn(d q), the reference's
+// Dequantization happens in registers with the fp16 magic pairs (kv_codes.h): fp16 values half_rn(d q), the reference's
 // operands (q8_to_f16 qwen38_mk.cu:2336, qn_to_f16 :2458).  The arithmetic of a row follows attn_core_t
 // (qwen38_mk.cu:2757-3080): S in fp32 from fp16 operands, masked positions -> -inf, P rounded to fp16, O in fp32.
 //
@@ -31,7 +31,6 @@
 namespace qkv {
 
 constexpr float LOG2E = 1.4426950408889634f;
-constexpr unsigned C64 = 0x64646464u;
 
 // The page table is read through the constant address space (no kernel writes it during a launch): a scalar load,
 // which waits on lgkmcnt only, never on the tile copies in flight.  Its latency under a full HBM stream is of the order
@@ -114,48 +113,42 @@ __device__ __forceinline__ void load_ksub(KSub<B> & k, const uint8_t * row, cons
     k.s = *reinterpret_cast<const unsigned *>(sc + 2 * q);
 }
 
-// the high-bit field of word ks (HB * 8 bits)
+// the dword of h and the part of it that hold word ks's high field (code_pairs)
 template <int HB>
-__device__ __forceinline__ unsigned hi_field(const unsigned * h, int ks) {
-    if constexpr (HB == 1) return (h[ks >> 2] >> (8 * (ks & 3))) & 0xffu;
-    if constexpr (HB == 2) return (h[ks >> 1] >> (16 * (ks & 1))) & 0xffffu;
-    if constexpr (HB == 3) {
+__device__ __forceinline__ unsigned hi_dword(const unsigned * h, int ks) {
+    if constexpr (HB == 1) return h[ks >> 2];
+    if constexpr (HB == 2) return h[ks >> 1];
+    if constexpr (HB == 3) { // the 24 bits from bit 24 ks (garbage above)
         const int bit = 24 * ks, dw = bit >> 5, sh = bit & 31;
         unsigned x = h[dw] >> sh;
         if (sh > 8) x |= h[dw + 1] << (32 - sh);
-        return x & 0xffffffu;
+        return x;
     }
     return 0u;
 }
+template <int HB>
+__device__ __forceinline__ constexpr int hi_part(int ks) { return HB == 1 ? ks & 3 : ks & 1; }
 
-// fp16 A fragment of K step ks: values 8 ks .. 8 ks + 7 of the lane's row quarter, natural order
-template <int B>
+// where a K / V format's masks go (code_pairs)
+template <int KB, int VB>
+__device__ __forceinline__ constexpr bool mask_sc() {
+    return KB != 6 && VB != 6;
+}
+
+// fp16 A fragment of K step ks: values 8 ks .. 8 ks + 7 of the lane's row quarter, in pair order (pair_at)
+template <int B, bool SC>
 __device__ __forceinline__ half8 kfrag(const KSub<B> & k, int ks) {
-    unsigned lo, hi;
-    float bias;
-    if constexpr (B == 8) {
-        lo = k.d[2 * ks] ^ 0x80808080u; // signed q -> q + 128
-        hi = k.d[2 * ks + 1] ^ 0x80808080u;
-        bias = 1152.f;
-    } else {
-        word_codes<B>(k.d[ks], hi_field<B - 4>(k.h, ks), lo, hi);
-        bias = (float) (1024 + (1 << (B - 1)));
-    }
-    const half2v b2 = {(_Float16) -bias, (_Float16) -bias};
+    unsigned p[4];
+    if constexpr (B == 8) q8_pairs(k.d[2 * ks], k.d[2 * ks + 1], p);
+    else code_pairs<B, SC>(k.d[ks], hi_dword<B - 4>(k.h, ks), hi_part<B - 4>(ks), p);
     const half2v d2 = splat_h(k.s, ks >= 4);
-    const half2v p0 = (as_h2(perm_b32(lo, C64, 0x00050004u)) + b2) * d2;
-    const half2v p1 = (as_h2(perm_b32(lo, C64, 0x00070006u)) + b2) * d2;
-    const half2v p2 = (as_h2(perm_b32(hi, C64, 0x00050004u)) + b2) * d2;
-    const half2v p3 = (as_h2(perm_b32(hi, C64, 0x00070006u)) + b2) * d2;
     half8 r;
-    r[0] = p0[0];
-    r[1] = p0[1];
-    r[2] = p1[0];
-    r[3] = p1[1];
-    r[4] = p2[0];
-    r[5] = p2[1];
-    r[6] = p3[0];
-    r[7] = p3[1];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const half2v x = pair_operand(p[i], i < 2 ? CodeBias<B>::lo : CodeBias<B>::hi, d2);
+        r[2 * i] = x[0];
+        r[2 * i + 1] = x[1];
+    }
     return r;
 }
 
@@ -194,45 +187,12 @@ __device__ __forceinline__ void load_vpos(VRaw<B> & v, int j, const uint8_t * ro
     v.s[j] = sc[m >> 1];
 }
 
-// code bytes of the lane's 16 dims for position j: c[a] byte b = biased code of dim 16 m + 4 a + b
-template <int B>
-__device__ __forceinline__ void vcodes(const VRaw<B> & v, int j, unsigned (&c)[4]) {
-    if constexpr (B == 8) {
-#pragma unroll
-        for (int a = 0; a < 4; a++) c[a] = v.d[j][a];
-    } else {
-        constexpr int HB = B - 4;
-        unsigned h0 = 0, h1 = 0;
-        if constexpr (HB == 1) {
-            h0 = v.h[j][0] & 0xffu;
-            h1 = (v.h[j][0] >> 8) & 0xffu;
-        } else if constexpr (HB == 2) {
-            h0 = v.h[j][0] & 0xffffu;
-            h1 = v.h[j][0] >> 16;
-        } else if constexpr (HB == 3) {
-            h0 = v.h[j][0] & 0xffffffu;
-            h1 = (v.h[j][0] >> 24) | (v.h[j][1] << 8);
-        }
-        word_codes<B>(v.d[j][0], h0, c[0], c[1]);
-        word_codes<B>(v.d[j][1], h1, c[2], c[3]);
-    }
-}
-
-// the code bytes of nibble word w (0, 1) of the lane's 16 dims for position j: c[0] byte b = dim 16 m + 8 w + b,
-// c[1] byte b = dim 16 m + 8 w + 4 + b (biased codes; q8: the signed bytes)
-template <int B>
-__device__ __forceinline__ void vcodes_word(const VRaw<B> & v, int j, int w, unsigned (&c)[2]) {
-    if constexpr (B == 8) {
-        c[0] = v.d[j][2 * w];
-        c[1] = v.d[j][2 * w + 1];
-    } else {
-        constexpr int HB = B - 4;
-        unsigned hw = 0;
-        if constexpr (HB == 1) hw = (v.h[j][0] >> (8 * w)) & 0xffu;
-        else if constexpr (HB == 2) hw = w ? v.h[j][0] >> 16 : v.h[j][0] & 0xffffu;
-        else if constexpr (HB == 3) hw = w ? (v.h[j][0] >> 24) | (v.h[j][1] << 8) : v.h[j][0] & 0xffffffu;
-        word_codes<B>(v.d[j][w], hw, c[0], c[1]);
-    }
+// the magic pairs of word w (0, 1) of the lane's 16 dims for position j: pair i, element e = dim 16 m + 8 w + pair_at(i, e)
+template <int B, bool SC>
+__device__ __forceinline__ void vpairs(const VRaw<B> & v, int j, int w, unsigned (&p)[4]) {
+    if constexpr (B == 8) q8_pairs(v.d[j][2 * w], v.d[j][2 * w + 1], p);
+    else if constexpr (B == 7) code_pairs<B, SC>(v.d[j][w], w ? (v.h[j][0] >> 24) | (v.h[j][1] << 8) : v.h[j][0], 0, p);
+    else code_pairs<B, SC>(v.d[j][w], B == 4 ? 0u : v.h[j][0], w, p);
 }
 
 // ------------------------------------------------------------------------------------------------ tile staging
@@ -322,6 +282,13 @@ __device__ __forceinline__ f32x4 gload16(const void * g) {
     return r;
 }
 __device__ __forceinline__ void pin_after(f32x4 & x) { asm volatile("" : "+v"(x)); }
+// a wave-uniform pointer as a scalar
+template <typename P>
+__device__ __forceinline__ P * uniform_ptr(P * p) {
+    const unsigned long long x = (unsigned long long) p;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned) x), hi = __builtin_amdgcn_readfirstlane((unsigned) (x >> 32));
+    return reinterpret_cast<P *>(((unsigned long long) hi << 32) | lo);
+}
 struct TileSrc {
     const uint8_t * k;
     const uint16_t * ks;
@@ -466,14 +433,14 @@ __device__ __forceinline__ void read_v(RawTile<KB, VB> & r, const uint8_t * st, 
 //   S^T = K Q^T   column n of Q^T is query row 8 h + n / 2 (each score is computed in lanes n and n ^ 1), so lane
 //                 (n, q) owns its row's scores at positions 4 q + e and 16 + 4 q + e (e = 0..3);
 //   O += P V      the MFMA's K = 32 is 16 positions x (e = 0, 1):
-//                 O[row][16 m + 2 b + e'] = sum_{p, e} A[m][(p, e)] B[(p, e)][(row, e')],
-//                 A = V[p][16 m + 2 b + e],  B = P[p][row] if e = e' else 0,
-//                 so an A register holds two adjacent dims of one position: a byte pair of the position's code word
-//                 and one scale per register, shared by every row group.
+//                 O[row][dim(m, b, e')] = sum_{p, e} A[m][(p, e)] B[(p, e)][(row, e')],
+//                 A = V[p][dim(m, b, e)],  B = P[p][row] if e = e' else 0,
+//                 dim(m, b, e) = 16 m + 8 (b / 4) + pair_at(b % 4, e): an A register holds one pair of one position's
+//                 code word (kv_codes.h) and one scale, shared by every row group.
 // A row's arithmetic does not depend on its group or on T, so the partials are bitwise T-invariant.
 template <int NP>
 struct WaveState {
-    f32x4 acc[NP][8]; // group h, block b, element i -> dim 16 (4 q + i) + 2 b + (n & 1) of row 8 h + n / 2
+    f32x4 acc[NP][8]; // group h, block b, element i -> dim(4 q + i, b, n & 1) of row 8 h + n / 2 (above)
     float m[NP], l[NP];
     int lim[NP];      // last visible position of the lane's row (-1: padding row)
     int lim_min;      // last position visible to every real row (L - T), wave-uniform
@@ -495,6 +462,35 @@ struct NoHook {
     __device__ void operator()(A &&...) const {}
 };
 
+// O += P V (block b = pair b % 4 of nibble word b / 4 of the lane's 16 dims)
+template <int NP, int VB, bool SC>
+__device__ __forceinline__ void tile_pv(f32x4 (&acc)[NP][8], const VRaw<VB> & v, const half8 (&pb)[NP][2]) {
+    half2v dv[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) dv[j] = as_h2((v.s[j] & 0xffffu) * 0x10001u);
+#pragma unroll
+    for (int G = 0; G < 2; G++) // (one position group at a time: half the unpacked codes live)
+#pragma unroll
+        for (int W = 0; W < 2; W++) {
+            unsigned c[4][4];
+#pragma unroll
+            for (int jj = 0; jj < 4; jj++) vpairs<VB, SC>(v, 4 * G + jj, W, c[jj]);
+#pragma unroll
+            for (int bb = 0; bb < 4; bb++) {
+                const int b = 4 * W + bb;
+                half8 va;
+#pragma unroll
+                for (int jj = 0; jj < 4; jj++) {
+                    const half2v x = pair_operand(c[jj][bb], bb < 2 ? CodeBias<VB>::lo : CodeBias<VB>::hi, dv[4 * G + jj]);
+                    va[2 * jj] = x[0];
+                    va[2 * jj + 1] = x[1];
+                }
+#pragma unroll
+                for (int h = 0; h < NP; h++) acc[h][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pb[h][G], acc[h][b], 0, 0, 0);
+            }
+        }
+}
+
 // LATE_V: raw.v is unset on entry; load_v(raw, n, q) reads the V operands from the stage after the scores, and after_v()
 // (which refills the stage) runs once they are in registers -- K and V are never live together next to the state
 template <int NP, int KB, int VB, bool LATE_V = false, typename FV = NoHook, typename FA = NoHook>
@@ -509,8 +505,8 @@ __device__ __forceinline__ void compute_tile(WaveState<NP> & st, const half8 * s
     for (int h = 0; h < NP; h++) s[h][0] = s[h][1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < 8; ks++) {
-        const half8 a0 = kfrag<KB>(raw.k0, ks);
-        const half8 a1 = kfrag<KB>(raw.k1, ks);
+        const half8 a0 = kfrag<KB, mask_sc<KB, VB>()>(raw.k0, ks);
+        const half8 a1 = kfrag<KB, mask_sc<KB, VB>()>(raw.k1, ks);
 #pragma unroll
         for (int h = 0; h < NP; h++) {
             const half8 b = NP == 1 ? st.qf[ks] : sQ[qchunk(8 * h + (n >> 1), 8 * q + ks)];
@@ -598,84 +594,77 @@ __device__ __forceinline__ void compute_tile(WaveState<NP> & st, const half8 * s
         lds_drain();
         after_v();
     }
-    // ---- O += P V: block b = dims 16 m + 2 b, + 1 of the lane's V row m (nibble word b / 4, values 2 (b % 4), + 1)
-    half2v dv[8];
-#pragma unroll
-    for (int j = 0; j < 8; j++) dv[j] = as_h2((raw.v.s[j] & 0xffffu) * 0x10001u);
-    constexpr unsigned QX = VB == 8 ? 0x80808080u : 0u; // q8: signed byte -> byte + 128
-    constexpr float VBIAS = VB == 8 ? 1152.f : (float) (1024 + (1 << (VB - 1)));
-    const half2v vb2 = {(_Float16) -VBIAS, (_Float16) -VBIAS};
-#pragma unroll
-    for (int w = 0; w < 2; w++) {
-        unsigned c[8][2];
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            vcodes_word<VB>(raw.v, j, w, c[j]);
-            c[j][0] ^= QX;
-            c[j][1] ^= QX;
-        }
-#pragma unroll
-        for (int bb = 0; bb < 4; bb++) {
-            const int b = 4 * w + bb;
-            const unsigned sel = (bb & 1) ? 0x00070006u : 0x00050004u;
-#pragma unroll
-            for (int G = 0; G < 2; G++) {
-                half8 va;
-#pragma unroll
-                for (int jj = 0; jj < 4; jj++) {
-                    const int j = 4 * G + jj;
-                    const half2v x = (as_h2(perm_b32(c[j][bb >> 1], C64, sel)) + vb2) * dv[j];
-                    va[2 * jj] = x[0];
-                    va[2 * jj + 1] = x[1];
-                }
-#pragma unroll
-                for (int h = 0; h < NP; h++) st.acc[h][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pb[h][G], st.acc[h][b], 0, 0, 0);
-            }
-        }
-    }
+    tile_pv<NP, VB, mask_sc<KB, VB>()>(st.acc, raw.v, pb);
 }
 
-// ------------------------------------------------------------------------------------------------ 24-row tile
-// compute_tile for 16 or 24 rows (NP = 2, 3) with each score computed once: the S^T MFMAs take 16 distinct query rows
-// per column block (block 0: rows 0..15, block 1: rows 16..23 and, in lanes 8..15, copies of them), so the online
-// softmax runs over NB = 1 or 2 blocks instead of NP 8-row groups held twice.  The P V operands keep
-// compute_tile's (row, dim parity) column pairs: group h's lane n takes row 8 h + n / 2's fp16 P from the lane that
-// owns that row (ds_bpermute within the lane's 16-lane row).  A row's scores, softmax, P and P V are the same
-// operations on the same values as in compute_tile (an MFMA output element does not depend on its column): bitwise
-// the same partials as k_attn's 24-row kernel.
+// one row group's accumulators of a lane (odd: its dim parity) times e into the row's LDS buffer at its quarter's first
+// dim: blocks 2 k, 2 k + 1 are adjacent dims (pair_at), one 8-byte write
+__device__ __forceinline__ void store_acc(float * o, int odd, float e, const f32x4 (&acc)[8]) {
+#pragma unroll
+    for (int b = 0; b < 8; b += 2)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float2 * const d = reinterpret_cast<float2 *>(o + 16 * i + 8 * (b >> 2) + 4 * ((b >> 1) & 1) + 2 * odd);
+            *d = make_float2(e * acc[b][i], e * acc[b + 1][i]);
+        }
+}
+
+// ------------------------------------------------------------------------------------------------ distinct rows
+// compute_tile for NP = 2 or 3 groups (16 or 24 rows) with each score computed once: the S^T MFMAs take 16
+// distinct query rows per column block (NB = 1 or 2 blocks; NP = 3: block 1 holds rows 16..23, each in two adjacent
+// columns), so the online softmax runs over NB blocks instead of NP 8-row groups held twice.  The P V operands keep
+// compute_tile's (row, dim parity) column pairs: a block's two groups are its even and its odd rows, so a group's lane
+// n takes its row's fp16 P from a neighbouring lane by one DPP move (before: rows 8 h + n / 2 fetched by ds_bpermute,
+// an LDS round trip each).  A row's scores, softmax, P and P V are the same operations on the same values as in
+// compute_tile (an MFMA output element does not depend on its column): bitwise the same partials.
 template <int NP>
 struct RowState {
     static constexpr int NB = (NP + 1) / 2;
-    f32x4 acc[NP][8]; // as WaveState::acc: group h, lane (n, q) -> row 8 h + n / 2
+    f32x4 acc[NP][8]; // as WaveState::acc: group h, lane (n, q) -> row group_row(h, n)
     float m[NB], l[NB];
-    int lim[NB];      // last visible position of the lane's block row 16 H + n (-1: padding)
+    int lim[NB];      // last visible position of the lane's row block_row(H, n) (-1: padding)
     int lim_min;
 };
+// the row of block H's column n, and of group h's lane n (a last odd group has its block to itself)
+template <int NP>
+__device__ __forceinline__ int block_row(int H, int n) {
+    return (NP & 1) && H == NP / 2 ? 16 * H + (n >> 1) : 16 * H + n;
+}
+template <int NP>
+__device__ __forceinline__ int group_row(int h, int n) {
+    return (NP & 1) && h == NP - 1 ? 8 * h + (n >> 1) : 16 * (h >> 1) + 2 * (n >> 1) + (h & 1);
+}
+// the value that group h's lane takes of its block's x
+template <int NP>
+__device__ __forceinline__ unsigned group_val(unsigned x, int h) {
+    if ((NP & 1) && h == NP - 1) return x;
+    return h & 1 ? __builtin_amdgcn_update_dpp(0u, x, 0xF5, 0xf, 0xf, false)  // quad_perm 1,1,3,3
+                 : __builtin_amdgcn_update_dpp(0u, x, 0xA0, 0xf, 0xf, false); // quad_perm 0,0,2,2
+}
 
-// load_v(raw, n, q) reads the V operands after the scores; after_v() runs once they are in registers
-template <int NP, int KB, int VB, typename FV, typename FA = NoHook>
-__device__ __forceinline__ void compute_tile_v(RowState<NP> & st, const half8 * sQ, int p0, RawTile<KB, VB> & raw, FV load_v,
-                                               FA after_v = FA()) {
-    static_assert(NP == 2 || NP == 3, "16 or 24 rows");
-    constexpr int NB = RowState<NP>::NB;
-    // (the lane index stays visible here: its LDS addresses are held across the tile loop, which fits these kernels'
-    // registers and saves ~60 VALU instructions per tile)
-    const int lane = lane_id();
-    const int q = lane >> 4, n = lane & 15;
-    f32x4 s[NB][2];
+// S^T = K Q^T of a tile's two 16-position subtiles: qf(H, ks) is the lane's Q^T operand of block H, K step ks
+template <int NP, int KB, int VB, typename FQ>
+__device__ __forceinline__ void tile_scores(f32x4 (&s)[(NP + 1) / 2][2], const RawTile<KB, VB> & raw, FQ qf) {
+    constexpr int NB = (NP + 1) / 2;
 #pragma unroll
     for (int H = 0; H < NB; H++) s[H][0] = s[H][1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < 8; ks++) {
-        const half8 a0 = kfrag<KB>(raw.k0, ks);
-        const half8 a1 = kfrag<KB>(raw.k1, ks);
+        const half8 a0 = kfrag<KB, mask_sc<KB, VB>()>(raw.k0, ks);
+        const half8 a1 = kfrag<KB, mask_sc<KB, VB>()>(raw.k1, ks);
 #pragma unroll
         for (int H = 0; H < NB; H++) {
-            const half8 b = sQ[qchunk(H ? 16 + (n & 7) : n, 8 * q + ks)];
+            const half8 b = qf(H, ks);
             s[H][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, b, s[H][0], 0, 0, 0);
             s[H][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, b, s[H][1], 0, 0, 0);
         }
     }
+}
+
+// the online softmax of the tile at p0 (st.m, st.l, the rescale of st.acc) and its P operands (lane: column n, quarter q)
+template <int NP>
+__device__ __forceinline__ void tile_softmax(RowState<NP> & st, const f32x4 (&s)[(NP + 1) / 2][2], int p0, int n, int q, half8 (&pb)[NP][2]) {
+    constexpr int NB = RowState<NP>::NB;
     constexpr float RESCALE_LOG2 = 8.f;
     const bool full = __builtin_amdgcn_readfirstlane(p0 + ATP - 1 <= st.lim_min);
     unsigned w[NB][2][2]; // block H, group G, pair k: the lane's fp16 P of positions 16 G + 4 q + 2 k, + 1
@@ -720,7 +709,7 @@ __device__ __forceinline__ void compute_tile_v(RowState<NP> & st, const half8 * 
         st.l[H] = __builtin_fmaf(st.l[H], al, ps);
         st.m[H] = mnew;
         alpha[H] = al;
-        rescale |= al != 1.f && mold != -INFINITY && (H == 0 || n < 8);
+        rescale |= al != 1.f && mold != -INFINITY;
 #pragma unroll
         for (int G = 0; G < 2; G++)
 #pragma unroll
@@ -731,70 +720,48 @@ __device__ __forceinline__ void compute_tile_v(RowState<NP> & st, const half8 * 
                 w[H][G][k] = as_u(x2);
             }
     }
-    // group h's lane n takes row 8 h + n / 2: block h / 2, lane (8 h + n / 2) % 16 of the same 16-lane row
-    const int src[3] = {4 * (16 * q + (n >> 1)), 4 * (16 * q + 8 + (n >> 1)), 4 * (16 * q + (n >> 1))};
     if (__any(rescale)) { // alpha == 1 exactly leaves O unchanged: the skip is exact
 #pragma unroll
         for (int h = 0; h < NP; h++) {
-            const float a = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(src[h], __builtin_bit_cast(int, alpha[h >> 1])));
+            const float a = __builtin_bit_cast(float, group_val<NP>(__builtin_bit_cast(unsigned, alpha[h >> 1]), h));
 #pragma unroll
             for (int b = 0; b < 8; b++) st.acc[h][b] *= a;
         }
     }
     const unsigned odd = n & 1;
     const unsigned sel_lo = odd ? 0x05040c0cu : 0x0c0c0504u, sel_hi = odd ? 0x07060c0cu : 0x0c0c0706u;
-    half8 pb[NP][2];
 #pragma unroll
     for (int h = 0; h < NP; h++)
 #pragma unroll
         for (int G = 0; G < 2; G++)
 #pragma unroll
             for (int k = 0; k < 2; k++) {
-                const unsigned x = (unsigned) __builtin_amdgcn_ds_bpermute(src[h], (int) w[h >> 1][G][k]);
+                const unsigned x = group_val<NP>(w[h >> 1][G][k], h);
                 const half2v y0 = as_h2(perm_b32(x, 0u, sel_lo)), y1 = as_h2(perm_b32(x, 0u, sel_hi));
                 pb[h][G][4 * k] = y0[0];
                 pb[h][G][4 * k + 1] = y0[1];
                 pb[h][G][4 * k + 2] = y1[0];
                 pb[h][G][4 * k + 3] = y1[1];
             }
+}
+
+// one tile of a two-per-CU kernel (16 or 24 rows): load_v(raw, n, q) reads the V operands after the scores; after_v()
+// runs once they are in registers
+template <int NP, int KB, int VB, typename FV, typename FA = NoHook>
+__device__ __forceinline__ void compute_tile_v(RowState<NP> & st, const half8 * sQ, int p0, RawTile<KB, VB> & raw, FV load_v,
+                                               FA after_v = FA()) {
+    // (the lane index stays visible here: its LDS addresses are held across the tile loop, which fits these kernels'
+    // registers and saves ~60 VALU instructions per tile)
+    const int lane = lane_id();
+    const int q = lane >> 4, n = lane & 15;
+    f32x4 s[RowState<NP>::NB][2];
+    tile_scores<NP>(s, raw, [&](int H, int ks) { return sQ[qchunk(block_row<NP>(H, n), 8 * q + ks)]; });
+    half8 pb[NP][2];
+    tile_softmax<NP>(st, s, p0, n, q, pb);
     load_v(raw, n, q);
     lds_drain();
     after_v();
-    // ---- O += P V as compute_tile
-    half2v dv[8];
-#pragma unroll
-    for (int j = 0; j < 8; j++) dv[j] = as_h2((raw.v.s[j] & 0xffffu) * 0x10001u);
-    constexpr unsigned QX = VB == 8 ? 0x80808080u : 0u;
-    constexpr float VBIAS = VB == 8 ? 1152.f : (float) (1024 + (1 << (VB - 1)));
-    const half2v vb2 = {(_Float16) -VBIAS, (_Float16) -VBIAS};
-#pragma unroll
-    for (int wd = 0; wd < 2; wd++) {
-        unsigned c[8][2];
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            vcodes_word<VB>(raw.v, j, wd, c[j]);
-            c[j][0] ^= QX;
-            c[j][1] ^= QX;
-        }
-#pragma unroll
-        for (int bb = 0; bb < 4; bb++) {
-            const int b = 4 * wd + bb;
-            const unsigned sel = (bb & 1) ? 0x00070006u : 0x00050004u;
-#pragma unroll
-            for (int G = 0; G < 2; G++) {
-                half8 va;
-#pragma unroll
-                for (int jj = 0; jj < 4; jj++) {
-                    const int j = 4 * G + jj;
-                    const half2v x = (as_h2(perm_b32(c[j][bb >> 1], C64, sel)) + vb2) * dv[j];
-                    va[2 * jj] = x[0];
-                    va[2 * jj + 1] = x[1];
-                }
-#pragma unroll
-                for (int h = 0; h < NP; h++) st.acc[h][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pb[h][G], st.acc[h][b], 0, 0, 0);
-            }
-        }
-    }
+    tile_pv<NP, VB, mask_sc<KB, VB>()>(st.acc, raw.v, pb);
 }
 
 // The fused append's rows of one wave (mk_kv_append_attend): positions L - T .. L - 1 of segment [c0, c1) whose tile
@@ -1050,9 +1017,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SMALL ? 3 :
                 float v[4] = {qx[j][0], qx[j][1], qx[j][2], qx[j][3]};
                 if (qnw) qk_prep(v, qnw + (size_t) l * HD, rope + (size_t) (L - T + t) * 32);
                 if ((krot >> (layer0 + l)) & 1u) fwht256_w64(v);
-                o0[0] = (_Float16) (v[0] * 0.0625f);
-                o0[1] = (_Float16) (v[1] * 0.0625f);
-                o1[0] = (_Float16) (v[2] * 0.0625f);
+                o0[0] = (_Float16) (v[0] * 0.0625f); // (pair order, as the K operands)
+                o0[1] = (_Float16) (v[2] * 0.0625f);
+                o1[0] = (_Float16) (v[1] * 0.0625f);
                 o1[1] = (_Float16) (v[3] * 0.0625f);
             }
             reinterpret_cast<uint2 *>(sQ + qchunk(r, lane >> 1))[lane & 1] = make_uint2(as_u(o0), as_u(o1));
@@ -1065,8 +1032,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SMALL ? 3 :
             for (int H = 0; H < RowState<NP>::NB; H++) {
                 st.m[H] = -INFINITY;
                 st.l[H] = 0.f;
-                const int row = row0 + 16 * H + n; // (block 1, lanes 8..15: padding)
-                st.lim[H] = (H == 0 || n < 8) && row < R ? L - T + (row - div_m(row, T_m) * T) : -1;
+                const int row = row0 + block_row<NP>(H, n);
+                st.lim[H] = row < R ? L - T + (row - div_m(row, T_m) * T) : -1;
             }
         } else {
 #pragma unroll
@@ -1167,14 +1134,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SMALL ? 3 :
         static_assert(AWAVES * MR * OLD * 4 + 2 * AWAVES * RP * 4 <= SLDS, "merge buffers inside the stages");
         __syncthreads(); // every wave is done with its stage
         if constexpr (DISTINCT) {
-            if (q == 0) { // rows 16 H + n of the blocks
-                s_m[wv * RP + n] = st.m[0];
-                s_l[wv * RP + n] = st.l[0];
-                if constexpr (NP == 3)
-                    if (n < 8) {
-                        s_m[wv * RP + 16 + n] = st.m[RowState<NP>::NB - 1];
-                        s_l[wv * RP + 16 + n] = st.l[RowState<NP>::NB - 1];
-                    }
+            if (q == 0) {
+#pragma unroll
+                for (int H = 0; H < RowState<NP>::NB; H++) { // (a row held in two columns: the same value twice)
+                    s_m[wv * RP + block_row<NP>(H, n)] = st.m[H];
+                    s_l[wv * RP + block_row<NP>(H, n)] = st.l[H];
+                }
             }
         } else if (q == 0 && !(n & 1)) {
 #pragma unroll
@@ -1192,15 +1157,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SMALL ? 3 :
             for (int hh = 0; hh < 2; hh++) {
                 const int h = 2 * ps + hh;
                 if (h < NP) {
-                    const int row = 8 * h + (n >> 1);
+                    const int row = DISTINCT ? group_row<NP>(h, n) : 8 * h + (n >> 1);
                     const float M = fmaxf(fmaxf(s_m[row], s_m[RP + row]), fmaxf(s_m[2 * RP + row], s_m[3 * RP + row]));
                     const float mr = DISTINCT ? s_m[wv * RP + row] : st.m[(DISTINCT ? 0 : h)]; // the wave's own m of the row
                     const float e = mr == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mr - M);
-                    float * o = reinterpret_cast<float *>(smem) + (wv * MR + 8 * hh + (n >> 1)) * OLD + 64 * q + (n & 1);
-#pragma unroll
-                    for (int b = 0; b < 8; b++)
-#pragma unroll
-                        for (int i = 0; i < 4; i++) o[16 * i + 2 * b] = e * st.acc[h][b][i];
+                    store_acc(reinterpret_cast<float *>(smem) + (wv * MR + row - 16 * ps) * OLD + 64 * q, n & 1, e, st.acc[h]);
                 }
             }
             __syncthreads();
@@ -1245,12 +1206,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SMALL ? 3 :
 // free stages during the merge, so an item starts with them on their way.  A row's
 // slices, tile arithmetic and merge order are those of k_attn: bitwise the same partials.
 // APPEND (mk_kv_append_attend): the new rows are stored before an item's first copy, so nothing is started early.
-template <typename P>
-__device__ __forceinline__ P * uniform_ptr(P * p) {
-    const unsigned long long x = (unsigned long long) p;
-    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned) x), hi = __builtin_amdgcn_readfirstlane((unsigned) (x >> 32));
-    return reinterpret_cast<P *>(((unsigned long long) hi << 32) | lo);
-}
 struct ItemGeo {
     int si, seq, L, ws, c0, c1, ntiles, g, l, pbase;
     SideLayout SK, SV;
@@ -1380,9 +1335,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 float v[4] = {qx[j][0], qx[j][1], qx[j][2], qx[j][3]};
                 if (a.qnw) qk_prep(v, a.qnw + (size_t) G.l * HD, a.rope + (size_t) (G.L - T + t) * 32);
                 if ((a.krot >> (a.layer0 + G.l)) & 1u) fwht256_w64(v);
-                o0[0] = (_Float16) (v[0] * 0.0625f);
-                o0[1] = (_Float16) (v[1] * 0.0625f);
-                o1[0] = (_Float16) (v[2] * 0.0625f);
+                o0[0] = (_Float16) (v[0] * 0.0625f); // (pair order, as the K operands)
+                o0[1] = (_Float16) (v[2] * 0.0625f);
+                o1[0] = (_Float16) (v[1] * 0.0625f);
                 o1[1] = (_Float16) (v[3] * 0.0625f);
             }
             reinterpret_cast<uint2 *>(sQ + (r / RP) * RP * (HD / 8) + qchunk(r % RP, lane >> 1))[lane & 1] = make_uint2(as_u(o0), as_u(o1));
@@ -1392,8 +1347,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int H = 0; H < 2; H++) {
             st.m[H] = -INFINITY;
             st.l[H] = 0.f;
-            const int row = row0 + 16 * H + n; // (block 1, lanes 8..15: padding)
-            st.lim[H] = (H == 0 || n < 8) && row < R ? G.L - T + (row - div_m(row, T_m) * T) : -1;
+            const int row = row0 + block_row<NP>(H, n);
+            st.lim[H] = row < R ? G.L - T + (row - div_m(row, T_m) * T) : -1;
         }
 #pragma unroll
         for (int h = 0; h < NP; h++)
@@ -1442,12 +1397,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         float * const s_m = reinterpret_cast<float *>(sQ); // [8][24] (the query rows are read by now)
         float * const s_l = s_m + NW * RP;
         lds_barrier(); // every wave is done with its tiles and the query rows
-        if (q == 0) { // rows 16 H + n of the blocks
-            s_m[wv * RP + n] = st.m[0];
-            s_l[wv * RP + n] = st.l[0];
-            if (n < 8) {
-                s_m[wv * RP + 16 + n] = st.m[1];
-                s_l[wv * RP + 16 + n] = st.l[1];
+        if (q == 0) {
+#pragma unroll
+            for (int H = 0; H < RowState<NP>::NB; H++) { // (a row held in two columns: the same value twice)
+                s_m[wv * RP + block_row<NP>(H, n)] = st.m[H];
+                s_l[wv * RP + block_row<NP>(H, n)] = st.l[H];
             }
         }
         const int th = threadIdx.x / 256, tl = threadIdx.x - 256 * th, wb = AWAVES * th;
@@ -1456,21 +1410,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         lds_barrier();
 #pragma unroll
         for (int h = 0; h < NP; h++) {
+            // pass h's 8 buffer rows are group h's: row group_row(h, 2 j) in buffer row j
             {
-                const int row = 8 * h + (n >> 1);
+                const int row = group_row<NP>(h, n);
                 const float M = fmaxf(fmaxf(s_mw[row], s_mw[RP + row]), fmaxf(s_mw[2 * RP + row], s_mw[3 * RP + row]));
                 const float mr = s_mw[wv % AWAVES * RP + row]; // the wave's own m of the row
                 const float e = mr == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mr - M);
-                float * o = wbuf(wv) + (n >> 1) * OLD + 64 * q + (n & 1);
-#pragma unroll
-                for (int b = 0; b < 8; b++)
-#pragma unroll
-                    for (int k = 0; k < 4; k++) o[16 * k + 2 * b] = e * st.acc[h][b][k];
+                store_acc(wbuf(wv) + (n >> 1) * OLD + 64 * q, n & 1, e, st.acc[h]);
             }
             lds_barrier();
-            const int nrow = min(8, RB - 8 * h);
-            for (int idx = tl; idx < nrow * (HD / 4); idx += 256) {
-                const int r8 = idx / (HD / 4), c4 = idx % (HD / 4);
+            for (int idx = tl; idx < 8 * (HD / 4); idx += 256) {
+                const int r8 = idx / (HD / 4), c4 = idx % (HD / 4), row = group_row<NP>(h, 2 * r8);
+                if (row >= RB) continue;
                 float4 y = *reinterpret_cast<const float4 *>(wbuf(wb) + r8 * OLD + 4 * c4);
 #pragma unroll
                 for (int w = 1; w < AWAVES; w++) {
@@ -1480,7 +1431,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                     y.z += z.z;
                     y.w += z.w;
                 }
-                store_part(a.part + ((size_t) item * R + trow0 + 8 * h + r8) * HD + 4 * c4, y);
+                store_part(a.part + ((size_t) item * R + trow0 + row) * HD + 4 * c4, y);
             }
             if (h + 1 < NP) lds_barrier();
         }

@@ -10,6 +10,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "kv_codes.h"
 #include "kv_layout.h"
 
 namespace qkv {
@@ -299,8 +300,8 @@ __device__ __forceinline__ void store_row(const StoreLayout & S, const SideLayou
 }
 
 // ------------------------------------------------------------------------------------------------ dequantization
-// fp16 operands are built with the 0x6400 magic: the half with bits 0x6400 | n is 1024 + n exactly (n < 1024), so
-// (0x6400 | n) - (1024 + bias) is the integer code exactly and one fp16 multiply by the scale rounds d * q once,
+// fp16 operands are built from magic pairs (kv_codes.h): a half such as 0x6400 | n is 1024 + n exactly (n < 1024), so
+// subtracting 1024 + bias leaves the integer code exactly and one fp16 multiply by the scale rounds d * q once,
 // the same value as the reference's half_rn(d * (float) q) (q8_to_f16 :2336, qn_to_f16 :2458).
 
 __device__ __forceinline__ unsigned perm_b32(unsigned hi_src, unsigned lo_src, unsigned sel) {
@@ -310,36 +311,19 @@ __device__ __forceinline__ unsigned perm_b32(unsigned hi_src, unsigned lo_src, u
 __device__ __forceinline__ half2v as_h2(unsigned x) { return __builtin_bit_cast(half2v, x); }
 __device__ __forceinline__ unsigned as_u(half2v x) { return __builtin_bit_cast(unsigned, x); }
 
-// the hb-bit fields 0..3 of x (field k at bit hb k) moved to bits 4 .. 4+hb-1 of byte k
-template <int HB>
-__device__ __forceinline__ unsigned spread4(unsigned x) {
-    // 24-bit multiplies (full rate): the compiler cannot always prove the operands fit and would otherwise emit the
-    // quarter-rate 32-bit multiply
-    if constexpr (HB == 1) return __umul24((x << 4) & 0xf0u, 0x00204081u) & 0x10101010u; // bit k -> bit 8k + 4
-    if constexpr (HB == 2) {
-        x = __umul24(x & 0xffu, 0x10010u) & 0x00f000f0u; // fields 0,1 at bits 4..7, fields 2,3 at 20..23
-        return __umul24(x, 0x41u) & 0x30303030u;       // field 1 -> 12..13, field 3 -> 28..29
-    }
-    if constexpr (HB == 3) {
-        x &= 0xfffu;
-        x = (x | (x << 10)) & 0x003f003fu;
-        x = (x | (x << 5)) & 0x07070707u;
-        return x << 4;
-    }
-    return 0u;
+// signed code -> fp16 operand of one pair: (p - bias) d, one rounding (see CodeBias)
+__device__ __forceinline__ half2v pair_operand(unsigned p, float bias, half2v d2) {
+    const half2v b2 = {(_Float16) -bias, (_Float16) -bias};
+    return (as_h2(p) + b2) * d2;
 }
-
-// the biased codes n of the 8 values of one nibble word W (+ its high-bit field H): bytes of lo = values 0..3,
-// bytes of hi = values 4..7
-template <int B>
-__device__ __forceinline__ void word_codes(unsigned W, unsigned H, unsigned & lo, unsigned & hi) {
-    constexpr int HB = B - 4;
-    lo = W & 0x0f0f0f0fu;
-    hi = (W >> 4) & 0x0f0f0f0fu;
-    if constexpr (HB > 0) {
-        lo |= spread4<HB>(H);
-        hi |= spread4<HB>(H >> (4 * HB));
-    }
+// the pairs of 8 q8 bytes (two dwords of signed codes), in the packed words' pair order
+__device__ __forceinline__ void q8_pairs(unsigned d0, unsigned d1, unsigned (&p)[4]) {
+    d0 ^= 0x80808080u; // signed q -> q + 128
+    d1 ^= 0x80808080u;
+    p[0] = perm_b32(d0, 0x64646464u, 0x00060004u);
+    p[1] = perm_b32(d0, 0x64646464u, 0x00070005u);
+    p[2] = perm_b32(d1, 0x64646464u, 0x00060004u);
+    p[3] = perm_b32(d1, 0x64646464u, 0x00070005u);
 }
 
 } // namespace qkv
