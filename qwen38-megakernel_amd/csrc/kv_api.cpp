@@ -34,6 +34,13 @@ struct HipError : std::runtime_error {
     } while (0)
 
 constexpr int SLOTS = 17;
+// the prefill's fp16 operand tiles: at most this much for a call over several (layer, kv head) units (a context of 160 k
+// positions of one layer); one unit of a longer context takes what it needs
+constexpr size_t PREFILL_KV16_MAX = 640ull << 20;
+// layers whose fp16 tiles one prefill launch may read: as many as fit the XCDs' L2s together, so that the row blocks of one
+// (layer, kv head, segment) on an XCD share its L2 (two layers of 60,621 positions in one launch: 1,910 us for a 433-token
+// chunk, one at a time 1,590; four layers of 1,111 positions: 307 us together, 330 one at a time)
+constexpr size_t PREFILL_L2 = 32ull << 20;
 constexpr int ATT_BUCKET_ = 640;
 constexpr int ATP_ = 32;
 
@@ -138,6 +145,9 @@ struct Store {
     size_t part_bytes = 0;
     void * ml = nullptr;
     size_t ml_bytes = 0;
+    // prefill: the keys of one or more (layer, kv head) units as fp16 tiles (grown on demand, PREFILL_KV16_MAX)
+    void * kv16 = nullptr;
+    size_t kv16_bytes = 0;
     int max_blocks = 0;
     int occupancy = 0; // decode workgroups per CU: 0 = by launch size, 2 or 3 (launch_attn)
     // 25..48 query rows per kv head: one pass of 8-wave workgroups (1), two batches of 24 rows (0), or by format (2):
@@ -175,6 +185,7 @@ struct Store {
         for (void * p : retired) (void) hipFree(p);
         if (part) (void) hipFree(part);
         if (ml) (void) hipFree(ml);
+        if (kv16) (void) hipFree(kv16);
         if (rope_own) (void) hipFree(rope_own);
     }
     // Workspace buffers a larger call has replaced.  They stay allocated until the store is freed: work already
@@ -744,6 +755,16 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
         }
         hipStream_t st = static_cast<hipStream_t>(stream);
         const size_t esz = dtype ? 2 : 4, krow = (size_t) n_layers * NKV * HD;
+        // The fp16 tiles of every (layer, kv head): when all of them fit the scratch, they are kept from piece to piece
+        // of this call and a piece rewrites only what changed: its own rows, and the rows that the window has moved past
+        // (read as packed rows from now on).  Otherwise each launch holds one layer's heads (as many as fit) and writes
+        // all their tiles.  (One tile to spare: the attention copies tiles in pairs.)
+        const int kv_tiles = (pos + T + ATP_ - 1) / ATP_ + 1;
+        const size_t unit = (size_t) kv_tiles * KV16_TILE, fit = PREFILL_KV16_MAX / unit;
+        const bool keep = (size_t) n_layers * NKV <= fit;
+        const int ng = fit >= 4 ? 4 : fit >= 2 ? 2 : 1;
+        s.grow(s.kv16, s.kv16_bytes, unit * (size_t) (keep ? n_layers * NKV : ng));
+        int ws0 = -1, L0 = 0; // the previous piece's window start and length
         for (int a0 = 0; a0 < T;) {
             const int b = std::min(T, ((pos + a0) / ATT_BUCKET_ + 1) * ATT_BUCKET_ - pos);
             const int n0 = pos + a0, Tp = b - a0;
@@ -758,23 +779,38 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
             p.Tp = Tp;
             p.L = n0 + Tp;
             p.ws = window_start(p.L, s.win);
+            p.T = T;
             p.R = GQA * Tp;
             p.nrb = (p.R + PF2_ROWS - 1) / PF2_ROWS;
             p.seg = pf_seg(p.L);
             p.nseg = (p.L + p.seg - 1) / p.seg;
+            if (keep && ws0 >= 0) { // (ws is a multiple of the tile; L0's tile may be a partial one)
+                p.t0 = (s.kvrc > 0 ? ws0 : L0) / ATP_;
+                p.skip0 = s.kvrc > 0 ? p.ws / ATP_ : 0;
+                p.skip1 = L0 / ATP_;
+            }
+            p.kv_tiles = kv_tiles;
             p.qs = qs;
             p.gs = gs;
             p.rope = qnw ? s.rope : nullptr;
-            s.grow(s.part, s.part_bytes, (size_t) NKV * p.nseg * p.R * HD * sizeof(float));
-            s.grow(s.ml, s.ml_bytes, (size_t) NKV * p.nseg * p.R * sizeof(float2));
-            p.part = static_cast<float *>(s.part);
-            p.ml = static_cast<float2 *>(s.ml);
-            for (int l = 0; l < n_layers; l++) {
-                const int sl = layer0 + l;
-                const size_t trow = (size_t) l * T + a0; // first token row of the piece in this layer's block
+            for (int l = 0; l < s.n_layers; l++) {
+                p.krot |= (unsigned) s.spec.kr[l] << l;
+                p.vrot |= (unsigned) s.spec.vr[l] << l;
+            }
+            for (int l = 0; l < n_layers;) { // consecutive layers with the same K/V bits share their launches
+                const int sl = layer0 + l, kb = s.S.side[sl][0].bits, vb = s.S.side[sl][1].bits;
+                int e = l + 1;
+                while (keep && e < n_layers && (size_t) (e + 1 - l) * NKV * unit <= PREFILL_L2 && s.S.side[layer0 + e][0].bits == kb && s.S.side[layer0 + e][1].bits == vb) e++;
                 p.layer = sl;
-                p.krot = s.spec.kr[sl];
-                p.vrot = s.spec.vr[sl];
+                p.nl = e - l;
+                p.ng = keep ? NKV : ng;
+                const size_t units = (size_t) p.nl * p.ng;
+                s.grow(s.part, s.part_bytes, units * p.nseg * p.R * HD * sizeof(float));
+                s.grow(s.ml, s.ml_bytes, units * p.nseg * p.R * sizeof(float2));
+                p.part = static_cast<float *>(s.part);
+                p.ml = static_cast<float2 *>(s.ml);
+                p.kv16 = static_cast<uint8_t *>(s.kv16) + (keep ? (size_t) l * NKV * unit : 0);
+                const size_t trow = (size_t) l * T + a0; // first token row of the piece in this run's block
                 p.q = q + trow * NH * qs;
                 p.qnw = qnw ? qnw + (size_t) l * HD : nullptr;
                 p.out = out + trow * NH * HD;
@@ -782,8 +818,11 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
                 p.q32a = q32a ? q32a + trow * 192 * 16 : nullptr;
                 p.q32b = q32b ? q32b + trow * 192 * 16 : nullptr;
                 p.q32m = q32m ? q32m + trow * 192 * 4 : nullptr;
-                HCK(launch_prefill(p, s.S.side[sl][0].bits, s.S.side[sl][1].bits, st));
+                for (p.g0 = 0; p.g0 < NKV; p.g0 += p.ng) HCK(launch_prefill(p, kb, vb, st));
+                l = e;
             }
+            ws0 = p.ws;
+            L0 = p.L;
             a0 = b;
         }
         return 0;

@@ -295,10 +295,18 @@ hipError_t launch_combine(const AttnArgs & a, hipStream_t st, hipEvent_t ev0, hi
 
 // ------------------------------------------------------------------------------------------------ prefill
 // Causal attention of one prefill piece (pk_attn8's exact form, prefill_attn.cuh:698-702; pieces and window
-// prefill_host.cu:606-615).  Keys are cut into absolute segments of a.seg positions (a function of the row's bucket); a
-// row's partial for segment k is one online softmax over the segment's tiles in order, and the combine folds the row's
-// segments 0 .. pos / a.seg in order: each output is a function of its position and the store only, whatever the
-// chunking of the prefill.
+// prefill_host.cu:606-615), in three launches over every layer of a run (equal K / V bits):
+//   k_prefill_kv       the piece's keys as fp16 MFMA operands in a scratch buffer (PrefillArgs::kv16), each tile once
+//   k_prefill_attn     the attention over them: no unpacking in its loop
+//   k_prefill_combine  the segments of each row, the output epilogue
+// A piece has up to 30 row blocks of 128 per kv head, and unpacking the stored rows is as much work as a row block's
+// share of the attention: done inside the attention kernel, it took half of every workgroup's waves (16,384-position
+// prompt: 640 TFLOP/s).  Done once, it is a pass over the keys (4 KB written per position) that a piece pays back from
+// the second row block on; one row block alone still gains, its tiles no longer waiting on the unpacking.
+//
+// Keys are cut into absolute segments of a.seg positions (a function of the row's bucket).  Within a segment even and odd
+// tiles are two online softmaxes, merged in that order; the combine folds the row's segments 0 .. pos / a.seg in order:
+// each output is a function of its position and the store only, whatever the chunking of the prefill.
 
 // 32 values of scale block b (dims 32 b .. 32 b + 31) of one staged row of B bits -> 16 fp16 pairs fp16_rn(d q) in
 // pair order (pair i of word w: o[4 w + i]), the same values as the decode operands (kfrag)
@@ -329,23 +337,7 @@ __device__ __forceinline__ void dequant_block(const uint8_t * row, uint16_t sc, 
     }
 }
 
-// fp16 tile layout in LDS: K and V as [32][SK_LD] (row = position; the consumers read V transposed, read_tr16)
-constexpr int SK_LD = HD + 8;
-// V rows 560 bytes apart: the 4 rows that one 16-lane group of a transposed read addresses (32 bytes each) start 32
-// bytes apart in the banks instead of overlapping (528 bytes: 3.6% slower; 576: 4% slower; 592: the same as 560)
-constexpr int SV_LD = HD + 24;
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-// Prefill attention on 32x32x16 MFMAs: workgroup = (128 query rows, kv head, key segment), row block fastest so the
-// workgroups of one segment run side by side; 8 waves.  Waves 0-3 (consumers) hold 32 query
-// rows each and run the MFMAs and the softmax on the fp16 tile of buffer i % 2; waves 4-7 (producers) each copy an
-// 8-position quarter of the tiles (two tiles in flight) and dequantize exactly what they copied into the other
-// buffer.  One barrier per tile hands a buffer over; on each SIMD a producer's VALU work overlaps a consumer's MFMAs.
-constexpr int PQ_REGION = 5120;                           // per producer and stage: K rows 2 KB, V rows 2 KB, scales 1 KB
-constexpr int PQ_STAGES = 2 * 4 * PQ_REGION;              // two stages of the 4 producers
-constexpr int PQ_BUF = ATP * (SK_LD + SV_LD) * 2;        // one fp16 tile: K [32][SK_LD], V [32][SV_LD]
-constexpr int PQ_LDS = PQ_STAGES + 2 * PQ_BUF;
-
 typedef __fp16 f16v4 __attribute__((__vector_size__(4 * sizeof(__fp16))));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 // ds_read_b64_tr_b16 at LDS byte address off: in each group of 16 lanes, lane i receives element i % 4 of the 8-byte
@@ -354,28 +346,18 @@ __device__ __forceinline__ half4 read_tr16(unsigned off) {
     return __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4f16((__attribute__((address_space(3))) f16v4 *) (size_t) off));
 }
 
-// Instruction order for an unrolled chain of N LDS fragment reads each feeding one MFMA: the first D reads, then one
-// MFMA and the next read in turn, then the last D MFMAs (scheduling groups; no effect on the arithmetic).  Left to
-// itself the scheduler reads each fragment just before its MFMA into the same registers, so every MFMA of the chain
-// waits a whole LDS round trip.
-// K: 3 fragments ahead; V: 2 MFMAs ahead (4 transposed reads).  Measured: K 2 ahead 1.3% slower, V 3 or 4 ahead
-// 1.1% and 0.3% slower.
-constexpr int PF_K = 3, PF_V = 2;
-template <int D, int N, int RPM = 1>
-__device__ __forceinline__ void pipeline_reads() {
-    if constexpr (D > 0) {
-        __builtin_amdgcn_sched_group_barrier(0x100, D * RPM, 0); // DS reads
-#pragma unroll
-        for (int i = 0; i < N - D; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // MFMA
-            __builtin_amdgcn_sched_group_barrier(0x100, RPM, 0);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x008, D, 0);
-    }
-}
-static_assert(PQ_LDS >= PF2_ROWS * SK_LD * 2, "query staging inside the tile buffers");
+// One fp16 tile (32 positions) of the scratch, KV16_TILE bytes: 1 KiB fragments in the order the attention kernel reads
+// them, fragment f, lane l at 1024 f + 16 l:
+//   f = ks        (16)  A of S^T = K Q^T, K step ks: position l % 32, dims 16 ks + 8 (l / 32) .. + 7 (pair order)
+//   f = 16 + 2 db + s2  A of O^T += V^T P^T: dim 32 db + l % 32 (pair order), positions 16 s2 + 8 a + 4 (l / 32) + i as
+//                       element 4 a + i
+// Copied to LDS as they are, every fragment read is one conflict-free 16-byte read per lane.
+constexpr int PQ_REGION = 5120;   // per wave: K rows 2 KB, V rows 2 KB, scales 1 KB of 8 positions
+constexpr int SV_LD = HD + 24;    // V rows of the transposing buffer 560 bytes apart: the 4 rows that one 16-lane group of
+                                  // a transposed read addresses start 32 bytes apart in the banks
+constexpr int PKV_LDS = 4 * PQ_REGION + ATP * SV_LD * 2;
 
-// the 8 positions of quarter pw of tile i: one producer wave's copies (5 instructions, always) into its region
+// the 8 positions of quarter pw of a tile: one wave's copies (5 instructions) into its region
 template <int KB, int VB>
 __device__ __forceinline__ void pq_issue(const TileSrc & t, int nq, unsigned lds, int lane) {
     constexpr int KRB = 32 * KB, VRB = 32 * VB; // row bytes
@@ -383,206 +365,214 @@ __device__ __forceinline__ void pq_issue(const TileSrc & t, int nq, unsigned lds
     for (int j = 0; j < 2; j++) {
         int o = 1024 * j + 16 * lane;
         if (o >= nq * KRB) o = nq * KRB - 16;
-        dma16_keep(t.k + o, lds + 1024 * j);
+        dma16(t.k + o, lds + 1024 * j);
     }
 #pragma unroll
     for (int j = 0; j < 2; j++) {
         int o = 1024 * j + 16 * lane;
         if (o >= nq * VRB) o = nq * VRB - 16;
-        dma16_keep(t.v + o, lds + 2048 + 1024 * j);
+        dma16(t.v + o, lds + 2048 + 1024 * j);
     }
     const int r = min(lane & 7, nq - 1);
-    dma16_keep(lane < 8 ? static_cast<const void *>(t.ks + 8 * r) : static_cast<const void *>(t.vs + 8 * r), lds + 4096);
+    dma16(lane < 8 ? static_cast<const void *>(t.ks + 8 * r) : static_cast<const void *>(t.vs + 8 * r), lds + 4096);
 }
 
-// one producer lane: position lane % 8 of its quarter, scale block lane / 8, K and V into the fp16 buffer
+// one lane: position lane % 8 of its wave's quarter, scale block lane / 8: K straight into the tile's fragments, V into
+// the transposing buffer
 template <int KB, int VB>
-__device__ __forceinline__ void pq_dequant(const uint8_t * reg, int pw, int lane, _Float16 * sK, _Float16 * sV) {
+__device__ __forceinline__ void pq_dequant(const uint8_t * reg, int pw, int lane, uint8_t * tile, _Float16 * sV) {
     const int pl = lane & 7, b = lane >> 3, p = 8 * pw + pl;
     const uint16_t * ksc = reinterpret_cast<const uint16_t *>(reg + 4096);
     half2v o[16];
     dequant_block<KB>(reg + pl * 32 * KB, ksc[pl * 8 + b], b, o);
-    uint4 * kd = reinterpret_cast<uint4 *>(sK + p * SK_LD + 32 * b);
 #pragma unroll
-    for (int k = 0; k < 4; k++) kd[k] = make_uint4(as_u(o[4 * k]), as_u(o[4 * k + 1]), as_u(o[4 * k + 2]), as_u(o[4 * k + 3]));
+    for (int k = 0; k < 4; k++)
+        *reinterpret_cast<uint4 *>(tile + 1024 * (2 * b + (k >> 1)) + 16 * (p + 32 * (k & 1))) =
+            make_uint4(as_u(o[4 * k]), as_u(o[4 * k + 1]), as_u(o[4 * k + 2]), as_u(o[4 * k + 3]));
     dequant_block<VB>(reg + 2048 + pl * 32 * VB, ksc[64 + pl * 8 + b], b, o);
     uint4 * vd = reinterpret_cast<uint4 *>(sV + p * SV_LD + 32 * b);
 #pragma unroll
     for (int k = 0; k < 4; k++) vd[k] = make_uint4(as_u(o[4 * k]), as_u(o[4 * k + 1]), as_u(o[4 * k + 2]), as_u(o[4 * k + 3]));
 }
 
+// Tiles a.t0 .. of every (layer, kv head) of the launch: one workgroup of 4 waves per tile, each wave copying 8 positions
+// HBM -> LDS and unpacking what it copied.  HBM-bound: 4 workgroups per CU (38 KiB of LDS each) keep copies in flight.
 template <int KB, int VB>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_prefill3(PrefillArgs a) {
+__global__ __launch_bounds__(256) void k_prefill_kv(PrefillArgs a) {
+    __shared__ __attribute__((aligned(16))) uint8_t smem[PKV_LDS];
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const StoreLayout & S = a.S;
+    const int t = a.t0 + blockIdx.x, u = blockIdx.y, l = u / a.ng, g = a.g0 + u % a.ng;
+    const SideLayout SK = S.side[a.layer + l][0], SV = S.side[a.layer + l][1];
+    if (t >= a.skip0 && t < a.skip1) return;
+    const int p0t = ATP * t, nv = min(ATP, a.L - p0t);
+    const int q0 = min(8 * wv, nv - 1), nq = min(8, nv - q0), p0 = p0t + q0;
+    const bool ring = S.kvrc > 0 && p0t >= a.ws;
+    const TileSrc src = tile_src<KB, VB>(S, SK, SV, g, p0, page_of(S, a.seq, p0), (size_t) (a.seq * NKV + g) * S.kvrc, ring);
+    const unsigned lds = (unsigned) __builtin_amdgcn_readfirstlane(
+        (unsigned) (size_t) (__attribute__((address_space(3))) uint8_t *) smem + wv * PQ_REGION);
+    uint8_t * const tile = a.kv16 + ((size_t) u * a.kv_tiles + t) * KV16_TILE;
+    uint8_t * const reg = smem + wv * PQ_REGION;
+    _Float16 * const sV = reinterpret_cast<_Float16 *>(smem + 4 * PQ_REGION);
+    if (ring) {
+        pq_issue<8, 8>(src, nq, lds, lane);
+        vm_wait<0>();
+        pq_dequant<8, 8>(reg, wv, lane, tile, sV);
+    } else {
+        pq_issue<KB, VB>(src, nq, lds, lane);
+        vm_wait<0>();
+        pq_dequant<KB, VB>(reg, wv, lane, tile, sV);
+    }
+    __syncthreads();
+    // V fragments by two transposed reads of 4 positions each: lane q + 4 j of 16-lane group gr addresses position
+    // 16 s2 + 4 hf + j (+ 8 for the second read), dims 32 db + 16 (gr & 1) + 4 q .. + 3, and lane i of the group receives
+    // dim 32 db + 16 (gr & 1) + i of the 4 positions
+    const int hf = lane >> 5;
+    const unsigned v_lane = (unsigned) (size_t) (const __attribute__((address_space(3))) _Float16 *) sV +
+                            2 * ((4 * hf + ((lane >> 2) & 3)) * SV_LD + 16 * ((lane >> 4) & 1) + 4 * (lane & 3));
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int f = 4 * wv + k, db = f >> 1, s2 = f & 1;
+        const unsigned vo = v_lane + 2 * (16 * s2 * SV_LD + 32 * db);
+        const half8 av = __builtin_shufflevector(read_tr16(vo), read_tr16(vo + 2 * 8 * SV_LD), 0, 1, 2, 3, 4, 5, 6, 7);
+        *reinterpret_cast<half8 *>(tile + 1024 * (16 + f) + 16 * lane) = av;
+    }
+}
+
+// Instruction order for an unrolled chain of N LDS fragment reads each feeding one MFMA: the first D reads, then one
+// MFMA and the next read in turn, then the last D MFMAs (scheduling groups; no effect on the arithmetic).  Left to
+// itself the scheduler reads each fragment just before its MFMA into the same registers, so every MFMA of the chain
+// waits a whole LDS round trip.
+constexpr int PF_AHEAD = 4;
+template <int D, int N>
+__device__ __forceinline__ void pipeline_reads() {
+    __builtin_amdgcn_sched_group_barrier(0x100, D, 0); // DS reads
+#pragma unroll
+    for (int i = 0; i < N - D; i++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, D, 0);
+}
+
+// Workgroup = (128 query rows, layer, kv head, key segment), 8 waves: wave w holds rows 32 (w % 4) .. + 31 and runs the
+// segment's tiles of parity w / 4 on v_mfma_f32_32x32x16_f16: S^T = K Q^T, P taken straight from the S^T accumulators,
+// O^T += V^T P^T.  The two waves of a SIMD hold the same rows on alternate tiles, so one's softmax runs under the
+// other's MFMAs.  A pair of tiles (64 KB) is copied HBM / L2 -> LDS while the pair before it is computed: one barrier per
+// pair.  At the end the two parities' states are merged through LDS, each wave finishing half of its rows' dims.
+// What bounds it: the matrix cores (2,048 cycles per pair of tiles on a SIMD) and the softmax between its two products.
+// The workgroups of one (layer, kv head, segment) have indices equal mod the number of those (8 for one layer): one XCD,
+// whose L2 then serves all but the first of its row blocks.
+constexpr int PA_BUF = 2 * KV16_TILE;                     // one pair of tiles
+constexpr int PA_LDS = 2 * PA_BUF + 8 * 32 * 8;           // two pairs, (m, l) of 8 waves x 32 rows
+constexpr int SQ_LD = HD + 8;                             // query staging rows (halves)
+static_assert(PA_LDS >= PF2_ROWS * SQ_LD * 2, "query staging inside the tile buffers");
+
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_prefill_attn(PrefillArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane & 31, hf = lane >> 5;
-    const bool producer = wv >= 4;
-    const int pw = wv - 4;
-    const StoreLayout & S = a.S;
-    int bi = blockIdx.x;
-    const int rb = bi % a.nrb;
-    bi /= a.nrb;
-    const int g = bi % NKV, k = bi / NKV;
+    const int par = wv >> 2, wr = wv & 3;
+    const int combos = a.nl * a.ng * a.nseg;
+    const int rb = blockIdx.x / combos, cb = blockIdx.x - rb * combos;
+    const int k = cb % a.nseg, u = cb / a.nseg, gi = u % a.ng, l = u / a.ng, g = a.g0 + gi;
     const int r0 = PF2_ROWS * rb, rlast = min(a.R, r0 + PF2_ROWS) - 1;
     const int pmax = a.n0 + rlast / GQA;
     const int c0 = k * a.seg;
     if (c0 > pmax) return;
     const int c1 = min(c0 + a.seg, pmax + 1);
-    const int ntiles = (c1 - c0 + ATP - 1) / ATP;
+    const int ntiles = (c1 - c0 + ATP - 1) / ATP, nsteps = (ntiles + 1) / 2;
     const unsigned lds0 = (unsigned) (size_t) (__attribute__((address_space(3))) uint8_t *) smem;
-    _Float16 * const buf0 = reinterpret_cast<_Float16 *>(smem + PQ_STAGES);
-    // by value: held in registers, not re-read from the kernel arguments for every tile
-    const SideLayout SK = S.side[a.layer][0];
-    const SideLayout SV = S.side[a.layer][1];
-    const size_t ring0 = (size_t) (a.seq * NKV + g) * S.kvrc;
-    const int L = a.L, ws = a.ws;
-    auto is_ring = [&](int i) { return S.kvrc > 0 && c0 + ATP * i >= ws; };
-    // the producer's tiles are issued in order 0, 1, 2, ..: the page and offset of the next one are tracked (a tile
-    // never straddles a page: pages hold a multiple of 32 positions), and a page's physical index is looked up when the
-    // previous tile ends the previous page, one tile before its copies are issued
-    const int * const pt = S.ptab + (size_t) a.seq * S.pt_stride;
-    int nx_lp = c0 / S.page, nx_off = c0 - nx_lp * S.page;
-    int nx_phys = ((const_int_p) pt)[nx_lp];
-    // producer: the copies of quarter pw of tile i into stage i % 2
-    auto issue = [&](int i) {
-        const int p0t = c0 + ATP * i, nv = min(ATP, L - p0t);
-        const int q0 = min(8 * pw, nv - 1), nq = min(8, nv - q0), p0 = p0t + q0;
-        const unsigned lds = (unsigned) __builtin_amdgcn_readfirstlane(lds0 + ((i & 1) * 4 + pw) * PQ_REGION);
-        const bool ring = is_ring(i);
-        const size_t mr = (size_t) (g * S.n_pages + nx_phys) * S.page + nx_off + q0;
-        nx_off += ATP;
-        if (nx_off == S.page) {
-            nx_off = 0;
-            nx_lp++;
-            if (i + 1 < ntiles) nx_phys = ((const_int_p) pt)[nx_lp];
-        }
-        const TileSrc t = tile_src_row<KB, VB>(S.kvrc, SK, SV, !ring || !SK.ring || !SV.ring ? mr : 0, p0, ring0, ring);
-        if (ring) pq_issue<8, 8>(t, nq, lds, lane);
-        else pq_issue<KB, VB>(t, nq, lds, lane);
+    const uint8_t * const src0 = a.kv16 + ((size_t) u * a.kv_tiles + c0 / ATP) * KV16_TILE + (size_t) wv * (PA_BUF / 8);
+    // wave w copies an eighth of the pair of step s (8 KiB) into buffer s % 2; the pair's second tile may lie past the
+    // last one of the segment: in bounds (the scratch holds a spare tile), its bytes are not used
+    auto issue = [&](int s) {
+        const unsigned to = (unsigned) __builtin_amdgcn_readfirstlane(lds0 + (s & 1) * PA_BUF + wv * (PA_BUF / 8));
+        dma16s_pieces<8, false>(uniform_ptr(src0 + (size_t) s * PA_BUF), 16 * lane, to);
     };
-    auto dequant = [&](int i) {
-        const uint8_t * reg = smem + ((i & 1) * 4 + pw) * PQ_REGION;
-        _Float16 * sK = buf0 + (i & 1) * (PQ_BUF / 2);
-        _Float16 * sV = sK + ATP * SK_LD;
-        if (is_ring(i)) pq_dequant<8, 8>(reg, pw, lane, sK, sV);
-        else pq_dequant<KB, VB>(reg, pw, lane, sK, sV);
-    };
-    // ---- query rows: all 8 waves stage 16 rows each (prep, FWHT for rotated K, * 1/16, fp16), consumers take fragments;
+    // ---- query rows: all 8 waves stage 16 rows each (prep, FWHT for rotated K, * 1/16, fp16), then take fragments;
     // loaded 8 rows at a time (independent loads, one wait)
-    _Float16 * const qs = reinterpret_cast<_Float16 *>(smem);
+    const float * const q = a.q + (size_t) l * a.T * NH * a.qs;
+    const float * const qnw = a.qnw ? a.qnw + (size_t) l * HD : nullptr;
+    const bool krot = (a.krot >> (a.layer + l)) & 1u;
+    _Float16 * const sq = reinterpret_cast<_Float16 *>(smem);
     for (int jb = 0; jb < 16; jb += 8) {
         float4 xs[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int r = r0 + 16 * wv + jb + u, t = r / GQA, hh = r - GQA * t;
-            xs[u] = r < a.R ? *reinterpret_cast<const float4 *>(a.q + ((size_t) t * NH + GQA * g + hh) * a.qs + 4 * lane)
+        for (int v = 0; v < 8; v++) {
+            const int r = r0 + 16 * wv + jb + v, t = r / GQA, hh = r - GQA * t;
+            xs[v] = r < a.R ? *reinterpret_cast<const float4 *>(q + ((size_t) t * NH + GQA * g + hh) * a.qs + 4 * lane)
                             : make_float4(0.f, 0.f, 0.f, 0.f);
         }
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-        const int rl = 16 * wv + jb + u, r = r0 + rl;
-        half2v o0 = {(_Float16) 0.f, (_Float16) 0.f}, o1 = o0;
-        if (r < a.R) {
-            const int t = r / GQA;
-            const float4 x = xs[u];
-            float v[4] = {x.x, x.y, x.z, x.w};
-            if (a.qnw) qk_prep(v, a.qnw, a.rope + (size_t) (a.n0 + t) * 32);
-            if (a.krot) fwht256_w64(v);
-            o0[0] = (_Float16) (v[0] * 0.0625f); // (pair order, as the K rows of the fp16 tile)
-            o0[1] = (_Float16) (v[2] * 0.0625f);
-            o1[0] = (_Float16) (v[1] * 0.0625f);
-            o1[1] = (_Float16) (v[3] * 0.0625f);
+        for (int v = 0; v < 8; v++) {
+            const int rl = 16 * wv + jb + v, r = r0 + rl;
+            half2v o0 = {(_Float16) 0.f, (_Float16) 0.f}, o1 = o0;
+            if (r < a.R) {
+                const int t = r / GQA;
+                const float4 x = xs[v];
+                float y[4] = {x.x, x.y, x.z, x.w};
+                if (qnw) qk_prep(y, qnw, a.rope + (size_t) (a.n0 + t) * 32);
+                if (krot) fwht256_w64(y);
+                o0[0] = (_Float16) (y[0] * 0.0625f); // (pair order, as the K fragments)
+                o0[1] = (_Float16) (y[2] * 0.0625f);
+                o1[0] = (_Float16) (y[1] * 0.0625f);
+                o1[1] = (_Float16) (y[3] * 0.0625f);
+            }
+            *reinterpret_cast<uint2 *>(sq + rl * SQ_LD + 4 * lane) = make_uint2(as_u(o0), as_u(o1));
         }
-        *reinterpret_cast<uint2 *>(qs + rl * SK_LD + 4 * lane) = make_uint2(as_u(o0), as_u(o1));
-    }
     }
     __syncthreads();
-    // Both roles pass the same barriers: two after the staging, then one per tile.
-    if (producer) {
-        // the producers set the pace (their dequantization and fp16 tile writes take longer per tile than a consumer's
-        // MFMAs and softmax): on a SIMD shared with a consumer, the arbiter's preference for the older wave (the
-        // consumer) would otherwise give the consumer's issue slots first
-        __builtin_amdgcn_s_setprio(1);
-        __syncthreads(); // the consumers hold their query fragments: the staging area is free
-        issue(0);
-        if (ntiles > 1) issue(1);
-        if (ntiles > 1) vm_wait<5>();
-        else vm_wait<0>();
-        dequant(0);
-        lds_drain();
-        if (ntiles > 2) issue(2);
-        __syncthreads(); // buffer 0 complete
-        for (int i = 0; i < ntiles; i++) {
-            if (i + 1 < ntiles) {
-                if (i + 2 < ntiles) vm_wait<5>(); // tile i + 1 landed (tile i + 2 may be in flight)
-                else vm_wait<0>();
-                dequant(i + 1);
-                lds_drain();
-                if (i + 3 < ntiles) issue(i + 3);
-            }
-            __syncthreads(); // buffer (i + 1) % 2 complete, buffer i % 2 free
-        }
-        return;
-    }
     half8 qf[16];
 #pragma unroll
-    for (int ks = 0; ks < 16; ks++) qf[ks] = *reinterpret_cast<const half8 *>(qs + (32 * wv + c) * SK_LD + 16 * ks + 8 * hf);
-    __syncthreads();
-    __syncthreads();
-    const int row = r0 + 32 * wv + c;
+    for (int ks = 0; ks < 16; ks++) qf[ks] = *reinterpret_cast<const half8 *>(sq + (32 * wr + c) * SQ_LD + 16 * ks + 8 * hf);
+    __syncthreads(); // every wave holds its fragments: the staging area is free
+    issue(0);
+    const int row = r0 + 32 * wr + c;
     const int lim = row < a.R ? a.n0 + row / GQA : -1;
-    const int lim_min = a.n0 + (r0 + 32 * wv) / GQA;
-    float m = -INFINITY, l = 0.f;
+    const int lim_min = a.n0 + (r0 + 32 * wr) / GQA;
+    const bool rows = r0 + 32 * wr < a.R; // the wave has rows at all
+    float m = -INFINITY, ls = 0.f;        // running max (log2 units) and sum
     f32x16 O[8];
 #pragma unroll
     for (int db = 0; db < 8; db++)
 #pragma unroll
         for (int e = 0; e < 16; e++) O[db][e] = 0.f;
     constexpr float RESCALE_LOG2 = 8.f;
-    for (int i = 0; i < ntiles; i++) {
-        const _Float16 * const sK = buf0 + (i & 1) * (PQ_BUF / 2);
-        const _Float16 * const sV = sK + ATP * SK_LD;
-        // V operand of O^T += V^T P^T (lane l: dim 32 db + l % 32, the 8 positions of P's k order for half hf) by two
-        // transposed reads of 4 positions: lane a = q + 4 j of each 16-lane group g addresses position 16 s2 + 4 hf + j
-        // (+ 8 for the second read), dims 32 db + 16 (g & 1) + 4 q .. + 3, and lane i of the group receives dim
-        // 32 db + 16 (g & 1) + i of the 4 positions
-        const unsigned v_lane = (unsigned) (size_t) (const __attribute__((address_space(3))) _Float16 *) sV +
-                                2 * ((4 * hf + ((lane >> 2) & 3)) * SV_LD + 16 * ((lane >> 4) & 1) + 4 * (lane & 3));
+    for (int s = 0; s < nsteps; s++) {
+        vm_wait<0>();
+        __syncthreads(); // the pair of step s is complete, and every wave is done with the buffer of step s - 1
+        if (s + 1 < nsteps) issue(s + 1);
+        const int i = 2 * s + par;
+        if (i >= ntiles || !rows) continue;
+        const uint8_t * const tile = smem + (s & 1) * PA_BUF + par * KV16_TILE + 16 * lane;
         const int p0 = c0 + ATP * i;
         f32x16 sacc;
 #pragma unroll
         for (int e = 0; e < 16; e++) sacc[e] = 0.f;
 #pragma unroll
-        for (int ks = 0; ks < 16; ks++) {
-            const half8 ak = *reinterpret_cast<const half8 *>(sK + c * SK_LD + 16 * ks + 8 * hf);
-            sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ak, qf[ks], sacc, 0, 0, 0);
-        }
-        // the K fragments are read PF_K ahead of their MFMAs: each read's LDS latency then hides behind the MFMAs
-        // already issued instead of standing between two MFMAs of the chain
-        pipeline_reads<PF_K, 16>();
-        // fully visible tiles (wave-uniform) skip the causal mask
+        for (int ks = 0; ks < 16; ks++)
+            sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(tile + 1024 * ks), qf[ks], sacc, 0, 0, 0);
+        pipeline_reads<PF_AHEAD, 16>();
         float mx = -INFINITY;
-        if (p0 + ATP - 1 <= lim_min) {
+        if (p0 + ATP - 1 <= lim_min) { // fully visible tiles (wave-uniform) skip the causal mask
 #pragma unroll
-            for (int e = 0; e < 16; e++) {
-                sacc[e] = sacc[e] * LOG2E;
-                mx = fmaxf(mx, sacc[e]);
-            }
+            for (int e = 0; e < 16; e++) mx = fmaxf(mx, sacc[e]);
         } else {
 #pragma unroll
             for (int e = 0; e < 16; e++) {
                 const int pos = p0 + 8 * (e >> 2) + 4 * hf + (e & 3);
-                sacc[e] = pos <= lim ? sacc[e] * LOG2E : -INFINITY;
+                sacc[e] = pos <= lim ? sacc[e] : -INFINITY;
                 mx = fmaxf(mx, sacc[e]);
             }
         }
-        mx = fmaxf(mx, shfl_xor(mx, 32));
+        mx = fmaxf(mx, shfl_xor(mx, 32)) * LOG2E;
         const float mnew = mx > m + RESCALE_LOG2 ? mx : m;
         float al = 1.f, ps = 0.f;
         if (mnew != -INFINITY) {
             al = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mnew);
 #pragma unroll
             for (int e = 0; e < 16; e++) {
-                sacc[e] = __builtin_amdgcn_exp2f(sacc[e] - mnew);
+                sacc[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[e], LOG2E, -mnew));
                 ps += sacc[e];
             }
         } else {
@@ -591,7 +581,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
         ps += shfl_xor(ps, 32);
         const bool rescale = al != 1.f && m != -INFINITY;
-        l = __builtin_fmaf(l, al, ps);
+        ls = __builtin_fmaf(ls, al, ps);
         m = mnew;
         if (__any(rescale)) {
 #pragma unroll
@@ -605,49 +595,76 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int db = 0; db < 8; db++)
 #pragma unroll
-            for (int s2 = 0; s2 < 2; s2++) {
-                const unsigned vo = v_lane + 2 * ((16 * s2) * SV_LD + 32 * db);
-                const half8 av = __builtin_shufflevector(read_tr16(vo), read_tr16(vo + 2 * 8 * SV_LD), 0, 1, 2, 3, 4, 5, 6, 7);
-                O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, pb[s2], O[db], 0, 0, 0);
-            }
-        pipeline_reads<PF_V, 16, 2>(); // (the score registers are free here: the V fragments have room to run further ahead)
-        __syncthreads(); // buffer i % 2 free for the producers
+            for (int s2 = 0; s2 < 2; s2++)
+                O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(tile + 1024 * (16 + 2 * db + s2)), pb[s2], O[db],
+                                                               0, 0, 0);
+        pipeline_reads<PF_AHEAD, 16>();
     }
+    // ---- the two parities of each row, even tiles first: M = max, O = e0 O0 + e1 O1, l likewise.  Each wave gives the
+    // other parity's wave half of its dims (blocks 4 (1 - par) .. + 3) and finishes the other half
+    float2 * const s_ml = reinterpret_cast<float2 *>(smem + 2 * PA_BUF);
+    float4 * const s_o = reinterpret_cast<float4 *>(smem); // [8 waves][16][64]
+    __syncthreads();
+    if (hf == 0) s_ml[wv * 32 + c] = make_float2(m, ls);
+#pragma unroll
+    for (int d = 0; d < 4; d++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            float4 x;
+            x.x = par ? O[d][4 * j] : O[4 + d][4 * j];
+            x.y = par ? O[d][4 * j + 1] : O[4 + d][4 * j + 1];
+            x.z = par ? O[d][4 * j + 2] : O[4 + d][4 * j + 2];
+            x.w = par ? O[d][4 * j + 3] : O[4 + d][4 * j + 3];
+            s_o[(wv * 16 + 4 * d + j) * 64 + lane] = x;
+        }
+    __syncthreads();
     if (row < a.R) {
-        const size_t u = (size_t) (g * a.nseg + k) * a.R + row;
-        if (hf == 0) a.ml[u] = make_float2(m, l);
-        float * const dst = a.part + u * HD;
+        const float2 ml0 = s_ml[wr * 32 + c], ml1 = s_ml[(4 + wr) * 32 + c];
+        const float M = fmaxf(ml0.x, ml1.x);
+        const float e0 = ml0.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml0.x - M);
+        const float e1 = ml1.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml1.x - M);
+        const size_t at = ((size_t) u * a.nseg + k) * a.R + row;
+        if (hf == 0 && par == 0) a.ml[at] = make_float2(M, __builtin_fmaf(e1, ml1.y, e0 * ml0.y));
+        float * const dst = a.part + at * HD;
+        const float4 * const o = s_o + ((wv ^ 4) * 16) * 64 + lane;
 #pragma unroll
-        for (int db = 0; db < 8; db++)
+        for (int d = 0; d < 4; d++)
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                *reinterpret_cast<float4 *>(dst + 32 * db + 8 * j + 4 * hf) =
-                    make_float4(O[db][4 * j], O[db][4 * j + 2], O[db][4 * j + 1], O[db][4 * j + 3]); // (V's dims are in pair order)
+            for (int j = 0; j < 4; j++) {
+                const float4 z = o[(4 * d + j) * 64];
+                const float zi[4] = {z.x, z.y, z.z, z.w};
+                float y[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float own = par ? O[4 + d][4 * j + i] : O[d][4 * j + i];
+                    y[i] = par ? __builtin_fmaf(e1, own, e0 * zi[i]) : __builtin_fmaf(e1, zi[i], e0 * own);
+                }
+                store_part(dst + 32 * (4 * par + d) + 8 * j + 4 * hf, make_float4(y[0], y[2], y[1], y[3])); // (V's dims are in pair order)
+            }
     }
 }
 
-// One wave per (row, kv head) of a prefill piece: the row's segments 0 .. pos / a.seg folded in segment order
-// (M' = max(M, m_k), O' = O e^(M - M') + O_k e^(m_k - M'), l likewise), y = O / l, then the output epilogue.
+// One wave per (layer, kv head, row) of a prefill piece: the row's segments 0 .. pos / a.seg folded in segment order
+// (M' = max(M, m_k), O' = O e^(M - M') + O_k e^(m_k - M'), l likewise; two at most, pf_seg), y = O / l, then the output
+// epilogue.
 __global__ __launch_bounds__(256) void k_prefill_combine(PrefillArgs a) {
     const int wid = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (wid >= a.R * NKV) return;
-    const int r = wid % a.R, g = wid / a.R;
+    if (wid >= a.R * a.nl * a.ng) return;
+    const int r = wid % a.R, u = wid / a.R, g = a.g0 + u % a.ng, l = u / a.ng;
     const int t = r / GQA, hh = r - GQA * t, pos = a.n0 + t;
     const int nk = pos / a.seg + 1;
     float M = -INFINITY, den = 0.f;
     float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
-    // up to 8 segments' partials loaded in one round, then folded in order (the fold is the same sequence of operations
-    // as one segment at a time)
-    constexpr int RND = 8;
+    constexpr int RND = 2; // one round of loads
     for (int k0 = 0; k0 < nk; k0 += RND) {
         float2 mls[RND];
         float4 os[RND];
 #pragma unroll
         for (int j = 0; j < RND; j++)
             if (k0 + j < nk) {
-                const size_t u = (size_t) (g * a.nseg + k0 + j) * a.R + r;
-                mls[j] = a.ml[u];
-                os[j] = *reinterpret_cast<const float4 *>(a.part + u * HD + 4 * lane);
+                const size_t at = ((size_t) u * a.nseg + k0 + j) * a.R + r;
+                mls[j] = a.ml[at];
+                os[j] = *reinterpret_cast<const float4 *>(a.part + at * HD + 4 * lane);
             }
 #pragma unroll
         for (int j = 0; j < RND; j++)
@@ -667,8 +684,9 @@ __global__ __launch_bounds__(256) void k_prefill_combine(PrefillArgs a) {
     }
     float v[4] = {num.x / den, num.y / den, num.z / den, num.w / den};
     const int h = GQA * g + hh;
-    finish_row(v, a.vrot, a.gate ? a.gate + ((size_t) t * NH + h) * a.gs : nullptr, a.out + ((size_t) t * NH + h) * HD, a.q32a,
-               a.q32b, a.q32m, (size_t) t, h);
+    const size_t trow = (size_t) l * a.T + t;
+    finish_row(v, (a.vrot >> (a.layer + l)) & 1u, a.gate ? a.gate + (trow * NH + h) * a.gs : nullptr, a.out + (trow * NH + h) * HD, a.q32a,
+               a.q32b, a.q32m, trow, h);
 }
 
 // ------------------------------------------------------------------------------------------------ dispatch
@@ -764,14 +782,14 @@ hipError_t launch_attn(const AttnArgs & a, int kb, int vb, int max_blocks, int o
 
 typedef void (*PrefillKernel)(PrefillArgs);
 
-static PrefillKernel pick_prefill(int kb, int vb) {
+static PrefillKernel pick_prefill_kv(int kb, int vb) {
 #define QKV_VB(K)                                                                                                      \
     switch (vb) {                                                                                                      \
-    case 4: return k_prefill3<K, 4>;                                                                                    \
-    case 5: return k_prefill3<K, 5>;                                                                                    \
-    case 6: return k_prefill3<K, 6>;                                                                                    \
-    case 7: return k_prefill3<K, 7>;                                                                                    \
-    case 8: return k_prefill3<K, 8>;                                                                                    \
+    case 4: return k_prefill_kv<K, 4>;                                                                                 \
+    case 5: return k_prefill_kv<K, 5>;                                                                                 \
+    case 6: return k_prefill_kv<K, 6>;                                                                                 \
+    case 7: return k_prefill_kv<K, 7>;                                                                                 \
+    case 8: return k_prefill_kv<K, 8>;                                                                                 \
     default: return nullptr;                                                                                           \
     }
     switch (kb) {
@@ -785,26 +803,25 @@ static PrefillKernel pick_prefill(int kb, int vb) {
 #undef QKV_VB
 }
 
-hipError_t launch_prefill(const PrefillArgs & a, int kb, int vb, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
-    PrefillKernel k = pick_prefill(kb, vb);
-    if (!k) return hipErrorInvalidValue;
-    constexpr int lds = PQ_LDS;
-    static thread_local const void * configured[32];
-    static thread_local int n_configured = 0;
-    bool done = false;
-    for (int i = 0; i < n_configured; i++) done |= configured[i] == (const void *) k;
-    if (!done) {
-        const hipError_t e = hipFuncSetAttribute((const void *) k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+hipError_t launch_prefill(const PrefillArgs & a, int kb, int vb, hipStream_t st) {
+    PrefillKernel kv = pick_prefill_kv(kb, vb);
+    if (!kv) return hipErrorInvalidValue;
+    static thread_local bool configured = false;
+    if (!configured) {
+        const hipError_t e = hipFuncSetAttribute((const void *) k_prefill_attn, hipFuncAttributeMaxDynamicSharedMemorySize, PA_LDS);
         if (e != hipSuccess) return e;
-        if (n_configured < 32) configured[n_configured++] = (const void *) k;
+        configured = true;
     }
-    hipExtLaunchKernelGGL(k, dim3(a.nrb * NKV * a.nseg), dim3(512), lds, st, ev0, nullptr, 0, a);
+    const int units = a.nl * a.ng, tiles = (a.L + ATP - 1) / ATP - a.t0;
+    hipLaunchKernelGGL(kv, dim3(tiles, units), dim3(256), 0, st, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipExtLaunchKernelGGL(k_prefill_combine, dim3((a.R * NKV + 3) / 4), dim3(256), 0, st, nullptr, ev1, 0, a);
+    hipLaunchKernelGGL(k_prefill_attn, dim3(a.nrb * units * a.nseg), dim3(512), PA_LDS, st, a);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_prefill_combine, dim3((a.R * units + 3) / 4), dim3(256), 0, st, a);
     return hipGetLastError();
 }
-
 
 template <int KB, int VB>
 static hipError_t prefetch_kb_vb(const AttnArgs & a, int tiles, hipStream_t st) {

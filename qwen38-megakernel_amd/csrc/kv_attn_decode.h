@@ -216,7 +216,6 @@ __device__ __forceinline__ void dma16(const void * g, unsigned lds) {
     if constexpr (NT) asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" QKV_DMA_CPOL ::"s"(lds), "v"(g) : "memory");
     else asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(g) : "memory");
 }
-__device__ __forceinline__ void dma16_keep(const void * g, unsigned lds) { dma16<false>(g, lds); }
 // the same with a scalar base address and a 32-bit per-lane byte offset (no 64-bit vector address per copy)
 template <bool NT = true>
 __device__ __forceinline__ void dma16s(const void * base, unsigned voff, unsigned lds) {

@@ -122,34 +122,40 @@ inline void fill_head(AttnArgs & a) {
     h.pad[0] = h.pad[1] = h.pad[2] = 0;
 }
 
-// one prefill piece of one layer: query rows r = 6 t + hh (token t = 0 .. Tp-1 at position n0 + t, query head
-// 6 g + hh of kv head g), keys in absolute segments of `seg` positions (pf_seg of the piece's bucket)
+// one prefill piece over a run of layers with the same K / V bits: query rows r = 6 t + hh (token t = 0 .. Tp-1 at
+// position n0 + t, query head 6 g + hh of kv head g), keys in absolute segments of `seg` positions (pf_seg of the
+// piece's bucket).  Unit u = l ng + (g - g0): layer l of the run, kv head g
 struct PrefillArgs {
     StoreLayout S;
-    int layer, seq;
+    int layer, seq;    // first slot of the run
+    int nl, g0, ng;    // layers and kv heads (g0 .. g0 + ng - 1) of the launch
     int n0, Tp, L, ws; // first query position, rows' tokens, L = n0 + Tp (one 640-bucket), window start of the bucket
+    int T;             // tokens of the whole call (a layer's stride in q, out, gate and the units)
     int R, nrb, nseg;  // 6 Tp rows per kv head, ceil(R / PF2_ROWS) row blocks, ceil(L / seg) key segments
     int seg;           // key positions per segment
-    int krot, vrot;
-    const float * q;   // [Tp][NH][qs]
+    int t0, kv_tiles;  // first tile that k_prefill_kv (re)writes; tiles per unit of kv16
+    int skip0, skip1;  // tiles skip0 .. skip1 - 1 are as the previous piece left them
+    unsigned krot, vrot; // per-slot bit masks: K / V stored rotated
+    const float * q;   // [nl][T][NH][qs] from the piece's first token
     int qs;
-    const float * qnw; // optional q-norm weights [HD] (the Q prep, table rope)
+    const float * qnw; // optional q-norm weights [nl][HD] (the Q prep, table rope)
     const float2 * rope;
-    float * out;       // [Tp][NH][HD]
-    const float * gate; // optional [Tp][NH][gs]
+    float * out;       // [nl][T][NH][HD]
+    const float * gate; // optional [nl][T][NH][gs]
     int gs;
-    int8_t * q32a;     // optional o_proj units [Tp][192][16] (a / b), meta [Tp][192][4]
+    int8_t * q32a;     // optional o_proj units [nl][T][192][16] (a / b), meta [nl][T][192][4]
     int8_t * q32b;
     uint16_t * q32m;
-    float * part;      // [NKV][nseg][R][HD] per-segment partial outputs (unnormalised)
-    float2 * ml;       // [NKV][nseg][R] (max in log2 units, sum)
+    uint8_t * kv16;    // [nl ng][kv_tiles][KV16_TILE] fp16 operand tiles (kv_attn.hip)
+    float * part;      // [nl ng][nseg][R][HD] per-segment partial outputs (unnormalised)
+    float2 * ml;       // [nl ng][nseg][R] (max in log2 units, sum)
 };
+constexpr int KV16_TILE = 2 * ATP * HD * 2; // one tile's K and V as fp16
 // key positions per prefill segment: 128 ceil(Lb / 256) with Lb = L rounded up to its 640-bucket: two segments per row
 // at most, the same segments for every row of a bucket (every row's result is a function of its position).  A full
 // 640-position piece then runs 30 row blocks x 4 kv heads x 2 segments = 240 workgroups, one round on 256 CUs at one
-// workgroup per CU; more segments repeat each workgroup's query staging and partial stores (about 4 segments: 9% slower
-// on a 16,384-position prompt, about 8: 23%; odd counts leave a partial round: about 3 segments 21% slower; one
-// segment uses half the CUs: 39% slower)
+// workgroup per CU; more segments repeat each workgroup's query staging and partial stores, and odd counts leave a
+// partial round (3, 4 or 8 segments measured 9-23% slower on a 16,384-position prompt, one segment 39%)
 inline int pf_seg(int L) {
     const int lb = (L + ATT_BUCKET - 1) / ATT_BUCKET * ATT_BUCKET;
     return 128 * ((lb + 255) / 256);
@@ -182,6 +188,7 @@ hipError_t launch_attn(const AttnArgs & a, int kb, int vb, int max_blocks, int o
 // the first `tiles` tiles of every wave slice of the attention launch `a` read into the L2 its workgroups will use
 hipError_t launch_prefetch(const AttnArgs & a, int kb, int vb, int tiles, hipStream_t st);
 hipError_t launch_combine(const AttnArgs & a, hipStream_t st, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
-hipError_t launch_prefill(const PrefillArgs & a, int kb, int vb, hipStream_t st, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
+// the piece's keys as fp16 tiles (tiles t0 ..), the attention and the combine
+hipError_t launch_prefill(const PrefillArgs & a, int kb, int vb, hipStream_t st);
 
 } // namespace qkv
