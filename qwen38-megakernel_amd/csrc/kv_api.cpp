@@ -41,6 +41,7 @@ constexpr size_t PREFILL_KV16_MAX = 640ull << 20;
 // (layer, kv head, segment) on an XCD share its L2 (two layers of 60,621 positions in one launch: 1,910 us for a 433-token
 // chunk, one at a time 1,590; four layers of 1,111 positions: 307 us together, 330 one at a time)
 constexpr size_t PREFILL_L2 = 32ull << 20;
+constexpr size_t PREFILL_PART = 256ull << 20; // segment partials of a launch over several layers or pieces
 constexpr int ATT_BUCKET_ = 640;
 constexpr int ATP_ = 32;
 
@@ -755,62 +756,106 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
         }
         hipStream_t st = static_cast<hipStream_t>(stream);
         const size_t esz = dtype ? 2 : 4, krow = (size_t) n_layers * NKV * HD;
-        // The fp16 tiles of every (layer, kv head): when all of them fit the scratch, they are kept from piece to piece
-        // of this call and a piece rewrites only what changed: its own rows, and the rows that the window has moved past
-        // (read as packed rows from now on).  Otherwise each launch holds one layer's heads (as many as fit) and writes
-        // all their tiles.  (One tile to spare: the attention copies tiles in pairs.)
-        const int kv_tiles = (pos + T + ATP_ - 1) / ATP_ + 1;
-        const size_t unit = (size_t) kv_tiles * KV16_TILE, fit = PREFILL_KV16_MAX / unit;
+        // The fp16 tiles of every (layer, kv head): when all of them fit the scratch, they are kept through the call.  The
+        // pieces then run in groups of up to PF_PIECES: a group's rows are stored, their tiles added (from the main rows and,
+        // with a window, from the q8 rows, which the ring must still hold: a group is no longer than the ring), and its
+        // pieces attend together.  Otherwise a launch holds one piece and one layer's heads, as many as fit, and writes all
+        // their tiles.  (One tile to spare: the attention copies tiles in pairs.)
+        const int end = pos + T, kv_tiles = (end + ATP_ - 1) / ATP_ + 1;
+        const int in_group = s.kvrc > 0 ? std::min(PF_PIECES, s.kvrc / ATT_BUCKET_) : PF_PIECES;
+        // the window's tiles a group can see: its pieces' and, before them, the first one's window
+        const int q_tiles = s.kvrc > 0 ? (s.kvrc / ATT_BUCKET_ + in_group) * (ATT_BUCKET_ / ATP_) + 2 : 0;
+        const size_t unit = (size_t) kv_tiles * KV16_TILE, qunit = (size_t) q_tiles * KV16_TILE, fit = PREFILL_KV16_MAX / (unit + qunit);
         const bool keep = (size_t) n_layers * NKV <= fit;
-        const int ng = fit >= 4 ? 4 : fit >= 2 ? 2 : 1;
-        s.grow(s.kv16, s.kv16_bytes, unit * (size_t) (keep ? n_layers * NKV : ng));
-        int ws0 = -1, L0 = 0; // the previous piece's window start and length
+        const int ng = keep ? NKV : fit >= 4 ? 4 : fit >= 2 ? 2 : 1;
+        const size_t units_all = keep ? (size_t) n_layers * NKV : (size_t) ng;
+        s.grow(s.kv16, s.kv16_bytes, units_all * (unit + qunit));
+        uint8_t * const kv16 = static_cast<uint8_t *>(s.kv16), * const kq16 = kv16 + units_all * unit;
+        PrefillArgs p{};
+        p.S = s.S;
+        p.seq = seq;
+        p.T = T;
+        p.ng = ng;
+        p.kv_tiles = kv_tiles;
+        p.q_tiles = q_tiles;
+        p.qs = qs;
+        p.gs = gs;
+        p.rope = qnw ? s.rope : nullptr;
+        for (int l = 0; l < s.n_layers; l++) {
+            p.krot |= (unsigned) s.spec.kr[l] << l;
+            p.vrot |= (unsigned) s.spec.vr[l] << l;
+        }
+        // consecutive layers with the same K/V bits share their launches, while their tiles fit the L2s and their partials
+        // the workspace (rows: partial rows per layer and kv head of a group)
+        auto run_end = [&](int l, size_t rows) {
+            const SideLayout * a = s.S.side[layer0 + l];
+            int e = l + 1;
+            while (keep && e < n_layers && (size_t) (e + 1 - l) * NKV * unit <= PREFILL_L2 && (size_t) (e + 1 - l) * NKV * rows * HD * 4 <= PREFILL_PART &&
+                   s.S.side[layer0 + e][0].bits == a[0].bits && s.S.side[layer0 + e][1].bits == a[1].bits)
+                e++;
+            return e;
+        };
+        auto set_run = [&](int l, int e) {
+            p.layer = layer0 + l;
+            p.nl = e - l;
+            p.kv16 = kv16 + (keep ? (size_t) l * NKV * unit : 0);
+            p.kq16 = kq16 + (keep ? (size_t) l * NKV * qunit : 0);
+        };
+        auto bits = [&](int l, int w) { return s.S.side[layer0 + l][w].bits; };
+        if (keep && pos > 0 && s.kvrc > 0) { // the window's rows before the call, before its own replace them in the ring
+            p.L = pos;
+            p.q0 = window_start(pos + 1, s.win) / ATP_;
+            p.q1 = (pos + ATP_ - 1) / ATP_;
+            for (int l = 0, e; l < n_layers; l = e) {
+                e = run_end(l, 0);
+                set_run(l, e);
+                HCK(launch_prefill_kv(p, bits(l, 0), bits(l, 1), st));
+            }
+        }
         for (int a0 = 0; a0 < T;) {
-            const int b = std::min(T, ((pos + a0) / ATT_BUCKET_ + 1) * ATT_BUCKET_ - pos);
-            const int n0 = pos + a0, Tp = b - a0;
-            HCK(launch_append(s.S, seq, layer0, n_layers, n0, Tp, static_cast<const char *>(k) + a0 * krow * esz,
+            // the group: tokens a0 .. b - 1, pieces first .. last
+            const int n0 = pos + a0, first = n0 / ATT_BUCKET_;
+            auto piece = [&](int i) {
+                PrefillPiece P{};
+                P.n0 = std::max(n0, i * ATT_BUCKET_);
+                const int L = std::min(end, (i + 1) * ATT_BUCKET_);
+                P.R = GQA * (L - P.n0);
+                P.ws = s.kvrc > 0 ? window_start(L, s.win) : INT32_MAX;
+                P.seg = pf_seg(L);
+                P.nseg = (L + P.seg - 1) / P.seg;
+                P.t0 = P.n0 - n0;
+                return P;
+            };
+            int last = first;
+            size_t part_rows = (size_t) piece(first).R * piece(first).nseg;
+            while (keep && last + 1 - first < in_group && (last + 1) * ATT_BUCKET_ < end) {
+                const PrefillPiece P = piece(last + 1);
+                const size_t more = part_rows + (size_t) P.R * P.nseg;
+                if (more * NKV * HD * 4 > PREFILL_PART) break;
+                part_rows = more;
+                last++;
+            }
+            const int L = std::min(end, (last + 1) * ATT_BUCKET_), b = L - pos;
+            HCK(launch_append(s.S, seq, layer0, n_layers, n0, b - a0, static_cast<const char *>(k) + a0 * krow * esz,
                               static_cast<const char *>(v) + a0 * krow * esz, dtype, st, nullptr, nullptr, knw, knw ? s.rope : nullptr));
-            s.top[seq] = std::max(s.top[seq], n0 + Tp);
-            s.n[seq] = std::max(s.n[seq], n0 + Tp);
-            PrefillArgs p{};
-            p.S = s.S;
-            p.seq = seq;
-            p.n0 = n0;
-            p.Tp = Tp;
-            p.L = n0 + Tp;
-            p.ws = window_start(p.L, s.win);
-            p.T = T;
-            p.R = GQA * Tp;
-            p.nrb = (p.R + PF2_ROWS - 1) / PF2_ROWS;
-            p.seg = pf_seg(p.L);
-            p.nseg = (p.L + p.seg - 1) / p.seg;
-            if (keep && ws0 >= 0) { // (ws is a multiple of the tile; L0's tile may be a partial one)
-                p.t0 = (s.kvrc > 0 ? ws0 : L0) / ATP_;
-                p.skip0 = s.kvrc > 0 ? p.ws / ATP_ : 0;
-                p.skip1 = L0 / ATP_;
-            }
-            p.kv_tiles = kv_tiles;
-            p.qs = qs;
-            p.gs = gs;
-            p.rope = qnw ? s.rope : nullptr;
-            for (int l = 0; l < s.n_layers; l++) {
-                p.krot |= (unsigned) s.spec.kr[l] << l;
-                p.vrot |= (unsigned) s.spec.vr[l] << l;
-            }
-            for (int l = 0; l < n_layers;) { // consecutive layers with the same K/V bits share their launches
-                const int sl = layer0 + l, kb = s.S.side[sl][0].bits, vb = s.S.side[sl][1].bits;
-                int e = l + 1;
-                while (keep && e < n_layers && (size_t) (e + 1 - l) * NKV * unit <= PREFILL_L2 && s.S.side[layer0 + e][0].bits == kb && s.S.side[layer0 + e][1].bits == vb) e++;
-                p.layer = sl;
-                p.nl = e - l;
-                p.ng = keep ? NKV : ng;
+            s.top[seq] = std::max(s.top[seq], L);
+            s.n[seq] = std::max(s.n[seq], L);
+            p.L = L;
+            p.p0 = keep && a0 > 0 ? n0 / ATP_ : 0; // (the rows before the call with the first group's)
+            p.p1 = (L + ATP_ - 1) / ATP_;
+            p.q0 = s.kvrc == 0 ? 0 : keep ? n0 / ATP_ : window_start(L, s.win) / ATP_;
+            p.q1 = s.kvrc == 0 ? 0 : p.p1;
+            p.np = 0;
+            for (int i = last; i >= first; i--) p.pc[p.np++] = piece(i); // the longest contexts first
+            for (int l = 0, e; l < n_layers; l = e) {
+                e = run_end(l, part_rows);
+                set_run(l, e);
                 const size_t units = (size_t) p.nl * p.ng;
-                s.grow(s.part, s.part_bytes, units * p.nseg * p.R * HD * sizeof(float));
-                s.grow(s.ml, s.ml_bytes, units * p.nseg * p.R * sizeof(float2));
+                s.grow(s.part, s.part_bytes, units * part_rows * HD * sizeof(float));
+                s.grow(s.ml, s.ml_bytes, units * part_rows * sizeof(float2));
                 p.part = static_cast<float *>(s.part);
                 p.ml = static_cast<float2 *>(s.ml);
-                p.kv16 = static_cast<uint8_t *>(s.kv16) + (keep ? (size_t) l * NKV * unit : 0);
-                const size_t trow = (size_t) l * T + a0; // first token row of the piece in this run's block
+                const size_t trow = (size_t) l * T + a0; // first token row of the group in this run's block
                 p.q = q + trow * NH * qs;
                 p.qnw = qnw ? qnw + (size_t) l * HD : nullptr;
                 p.out = out + trow * NH * HD;
@@ -818,11 +863,12 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
                 p.q32a = q32a ? q32a + trow * 192 * 16 : nullptr;
                 p.q32b = q32b ? q32b + trow * 192 * 16 : nullptr;
                 p.q32m = q32m ? q32m + trow * 192 * 4 : nullptr;
-                for (p.g0 = 0; p.g0 < NKV; p.g0 += p.ng) HCK(launch_prefill(p, kb, vb, st));
-                l = e;
+                for (p.g0 = 0; p.g0 < NKV; p.g0 += p.ng) {
+                    HCK(launch_prefill_kv(p, bits(l, 0), bits(l, 1), st));
+                    HCK(launch_prefill(p, st));
+                }
+                p.g0 = 0;
             }
-            ws0 = p.ws;
-            L0 = p.L;
             a0 = b;
         }
         return 0;

@@ -294,18 +294,21 @@ hipError_t launch_combine(const AttnArgs & a, hipStream_t st, hipEvent_t ev0, hi
 }
 
 // ------------------------------------------------------------------------------------------------ prefill
-// Causal attention of one prefill piece (pk_attn8's exact form, prefill_attn.cuh:698-702; pieces and window
-// prefill_host.cu:606-615), in three launches over every layer of a run (equal K / V bits):
-//   k_prefill_kv       the piece's keys as fp16 MFMA operands in a scratch buffer (PrefillArgs::kv16), each tile once
+// Causal attention of a group of prefill pieces (pk_attn8's exact form, prefill_attn.cuh:698-702; pieces and window
+// prefill_host.cu:606-615), over every layer of a run (equal K / V bits):
+//   k_prefill_kv       keys as fp16 MFMA operands in scratch buffers (PrefillArgs::kv16, kq16), each tile once
 //   k_prefill_attn     the attention over them: no unpacking in its loop
 //   k_prefill_combine  the segments of each row, the output epilogue
 // A piece has up to 30 row blocks of 128 per kv head, and unpacking the stored rows is as much work as a row block's
 // share of the attention: done inside the attention kernel, it took half of every workgroup's waves (16,384-position
-// prompt: 640 TFLOP/s).  Done once, it is a pass over the keys (4 KB written per position) that a piece pays back from
-// the second row block on; one row block alone still gains, its tiles no longer waiting on the unpacking.
+// prompt: 5.07 ms per layer, 4.19 with the keys unpacked once).  A key is read as its packed row by pieces whose window
+// starts after it and as its q8 window row by the others, so both forms are kept: the window's for as long as a piece
+// of the call can see it.  With both at hand the pieces of a group need not be stored one by one: up to PF_PIECES of them
+// share each launch, the longest contexts first, and a CU that finishes one workgroup goes on to the next (one piece per
+// launch left 67 us of starts, ends and short launches around 95 us of tiles).
 //
-// Keys are cut into absolute segments of a.seg positions (a function of the row's bucket).  Within a segment even and odd
-// tiles are two online softmaxes, merged in that order; the combine folds the row's segments 0 .. pos / a.seg in order:
+// Keys are cut into absolute segments of a piece's seg positions (a function of its bucket).  Within a segment even and
+// odd tiles are two online softmaxes, merged in that order; the combine folds the row's segments 0 .. pos / seg in order:
 // each output is a function of its position and the store only, whatever the chunking of the prefill.
 
 // 32 values of scale block b (dims 32 b .. 32 b + 31) of one staged row of B bits -> 16 fp16 pairs fp16_rn(d q) in
@@ -395,23 +398,25 @@ __device__ __forceinline__ void pq_dequant(const uint8_t * reg, int pw, int lane
     for (int k = 0; k < 4; k++) vd[k] = make_uint4(as_u(o[4 * k]), as_u(o[4 * k + 1]), as_u(o[4 * k + 2]), as_u(o[4 * k + 3]));
 }
 
-// Tiles a.t0 .. of every (layer, kv head) of the launch: one workgroup of 4 waves per tile, each wave copying 8 positions
-// HBM -> LDS and unpacking what it copied.  HBM-bound: 4 workgroups per CU (38 KiB of LDS each) keep copies in flight.
+// Tiles p0 .. p1 - 1 (main rows) and q0 .. q1 - 1 (window rows) of every (layer, kv head) of the launch: one workgroup of
+// 4 waves per tile, each wave copying 8 positions HBM -> LDS and unpacking what it copied.  HBM-bound: 4 workgroups per
+// CU (38 KiB of LDS each) keep copies in flight.
 template <int KB, int VB>
 __global__ __launch_bounds__(256) void k_prefill_kv(PrefillArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t smem[PKV_LDS];
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const StoreLayout & S = a.S;
-    const int t = a.t0 + blockIdx.x, u = blockIdx.y, l = u / a.ng, g = a.g0 + u % a.ng;
+    const int u = blockIdx.y, l = u / a.ng, g = a.g0 + u % a.ng;
+    const int x = blockIdx.x, np = a.p1 - a.p0;
+    const bool ring = x >= np;
+    const int t = ring ? a.q0 + x - np : a.p0 + x;
     const SideLayout SK = S.side[a.layer + l][0], SV = S.side[a.layer + l][1];
-    if (t >= a.skip0 && t < a.skip1) return;
     const int p0t = ATP * t, nv = min(ATP, a.L - p0t);
     const int q0 = min(8 * wv, nv - 1), nq = min(8, nv - q0), p0 = p0t + q0;
-    const bool ring = S.kvrc > 0 && p0t >= a.ws;
     const TileSrc src = tile_src<KB, VB>(S, SK, SV, g, p0, page_of(S, a.seq, p0), (size_t) (a.seq * NKV + g) * S.kvrc, ring);
     const unsigned lds = (unsigned) __builtin_amdgcn_readfirstlane(
         (unsigned) (size_t) (__attribute__((address_space(3))) uint8_t *) smem + wv * PQ_REGION);
-    uint8_t * const tile = a.kv16 + ((size_t) u * a.kv_tiles + t) * KV16_TILE;
+    uint8_t * const tile = ring ? a.kq16 + ((size_t) u * a.q_tiles + t % a.q_tiles) * KV16_TILE : a.kv16 + ((size_t) u * a.kv_tiles + t) * KV16_TILE;
     uint8_t * const reg = smem + wv * PQ_REGION;
     _Float16 * const sV = reinterpret_cast<_Float16 *>(smem + 4 * PQ_REGION);
     if (ring) {
@@ -455,14 +460,24 @@ __device__ __forceinline__ void pipeline_reads() {
     __builtin_amdgcn_sched_group_barrier(0x008, D, 0);
 }
 
+// the order of a tile's O += P V region: the first half's exponentials, then an MFMA, a fragment read and a few of the
+// second half's (later the sum's) VALU instructions in turn
+__device__ __forceinline__ void pipeline_pv() {
+    __builtin_amdgcn_sched_group_barrier(0x002, 24, 0); // VALU
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // MFMA
+        if (i < 16 - PF_AHEAD) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+    }
+}
+
 // Workgroup = (128 query rows, layer, kv head, key segment), 8 waves: wave w holds rows 32 (w % 4) .. + 31 and runs the
 // segment's tiles of parity w / 4 on v_mfma_f32_32x32x16_f16: S^T = K Q^T, P taken straight from the S^T accumulators,
 // O^T += V^T P^T.  The two waves of a SIMD hold the same rows on alternate tiles, so one's softmax runs under the
 // other's MFMAs.  A pair of tiles (64 KB) is copied HBM / L2 -> LDS while the pair before it is computed: one barrier per
 // pair.  At the end the two parities' states are merged through LDS, each wave finishing half of its rows' dims.
 // What bounds it: the matrix cores (2,048 cycles per pair of tiles on a SIMD) and the softmax between its two products.
-// The workgroups of one (layer, kv head, segment) have indices equal mod the number of those (8 for one layer): one XCD,
-// whose L2 then serves all but the first of its row blocks.
 constexpr int PA_BUF = 2 * KV16_TILE;                     // one pair of tiles
 constexpr int PA_LDS = 2 * PA_BUF + 8 * 32 * 8;           // two pairs, (m, l) of 8 waves x 32 rows
 constexpr int SQ_LD = HD + 8;                             // query staging rows (halves)
@@ -472,26 +487,45 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane & 31, hf = lane >> 5;
     const int par = wv >> 2, wr = wv & 3;
-    const int combos = a.nl * a.ng * a.nseg;
-    const int rb = blockIdx.x / combos, cb = blockIdx.x - rb * combos;
-    const int k = cb % a.nseg, u = cb / a.nseg, gi = u % a.ng, l = u / a.ng, g = a.g0 + gi;
-    const int r0 = PF2_ROWS * rb, rlast = min(a.R, r0 + PF2_ROWS) - 1;
-    const int pmax = a.n0 + rlast / GQA;
-    const int c0 = k * a.seg;
+    int pi = 0;
+#pragma unroll
+    for (int i = 1; i < PF_PIECES; i++)
+        if (i < a.np && (int) blockIdx.x >= a.pc[i].blk0) pi = i;
+    const PrefillPiece P = a.pc[pi];
+    const int combos = a.nl * a.ng * P.nseg, blk = blockIdx.x - P.blk0;
+    // a (layer, kv head, segment)'s row blocks on one XCD, side by side (workgroups are dealt to the 8 XCDs round robin):
+    // they read the same tiles at about the same time, and the XCD's L2 serves all but the first
+    int rb, cb;
+    if (combos % 8 == 0) {
+        const int nrb = (P.R + PF2_ROWS - 1) / PF2_ROWS, i = blk >> 3, j = i / nrb;
+        cb = (blk & 7) + 8 * j;
+        rb = i - j * nrb;
+    } else {
+        rb = blk / combos;
+        cb = blk - rb * combos;
+    }
+    const int k = cb % P.nseg, u = cb / P.nseg, gi = u % a.ng, l = u / a.ng, g = a.g0 + gi;
+    const int r0 = PF2_ROWS * rb, rlast = min(P.R, r0 + PF2_ROWS) - 1;
+    const int pmax = P.n0 + rlast / GQA;
+    const int c0 = k * P.seg;
     if (c0 > pmax) return;
-    const int c1 = min(c0 + a.seg, pmax + 1);
+    const int c1 = min(c0 + P.seg, pmax + 1);
     const int ntiles = (c1 - c0 + ATP - 1) / ATP, nsteps = (ntiles + 1) / 2;
     const unsigned lds0 = (unsigned) (size_t) (__attribute__((address_space(3))) uint8_t *) smem;
-    const uint8_t * const src0 = a.kv16 + ((size_t) u * a.kv_tiles + c0 / ATP) * KV16_TILE + (size_t) wv * (PA_BUF / 8);
-    // wave w copies an eighth of the pair of step s (8 KiB) into buffer s % 2; the pair's second tile may lie past the
-    // last one of the segment: in bounds (the scratch holds a spare tile), its bytes are not used
+    const uint8_t * const main0 = a.kv16 + (size_t) u * a.kv_tiles * KV16_TILE + (size_t) wv * (PA_BUF / 8);
+    const uint8_t * const win0 = a.kq16 + (size_t) u * a.q_tiles * KV16_TILE + (size_t) wv * (PA_BUF / 8);
+    // wave w copies an eighth of the pair of step s (8 KiB) into buffer s % 2: main rows below the window, its q8 rows from
+    // there on (the window starts at an even tile and q_tiles is even: a pair never straddles either).  The pair's second
+    // tile may lie past the last one of the segment: in bounds (each unit holds a spare tile), its bytes are not used
     auto issue = [&](int s) {
+        const int t = c0 / ATP + 2 * s;
+        const uint8_t * const src = ATP * t >= P.ws ? win0 + (size_t) (t % max(a.q_tiles, 1)) * KV16_TILE : main0 + (size_t) t * KV16_TILE;
         const unsigned to = (unsigned) __builtin_amdgcn_readfirstlane(lds0 + (s & 1) * PA_BUF + wv * (PA_BUF / 8));
-        dma16s_pieces<8, false>(uniform_ptr(src0 + (size_t) s * PA_BUF), 16 * lane, to);
+        dma16s_pieces<8, false>(uniform_ptr(src), 16 * lane, to);
     };
     // ---- query rows: all 8 waves stage 16 rows each (prep, FWHT for rotated K, * 1/16, fp16), then take fragments;
     // loaded 8 rows at a time (independent loads, one wait)
-    const float * const q = a.q + (size_t) l * a.T * NH * a.qs;
+    const float * const q = a.q + ((size_t) l * a.T + P.t0) * NH * a.qs;
     const float * const qnw = a.qnw ? a.qnw + (size_t) l * HD : nullptr;
     const bool krot = (a.krot >> (a.layer + l)) & 1u;
     _Float16 * const sq = reinterpret_cast<_Float16 *>(smem);
@@ -500,18 +534,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int v = 0; v < 8; v++) {
             const int r = r0 + 16 * wv + jb + v, t = r / GQA, hh = r - GQA * t;
-            xs[v] = r < a.R ? *reinterpret_cast<const float4 *>(q + ((size_t) t * NH + GQA * g + hh) * a.qs + 4 * lane)
+            xs[v] = r < P.R ? *reinterpret_cast<const float4 *>(q + ((size_t) t * NH + GQA * g + hh) * a.qs + 4 * lane)
                             : make_float4(0.f, 0.f, 0.f, 0.f);
         }
 #pragma unroll
         for (int v = 0; v < 8; v++) {
             const int rl = 16 * wv + jb + v, r = r0 + rl;
             half2v o0 = {(_Float16) 0.f, (_Float16) 0.f}, o1 = o0;
-            if (r < a.R) {
+            if (r < P.R) {
                 const int t = r / GQA;
                 const float4 x = xs[v];
                 float y[4] = {x.x, x.y, x.z, x.w};
-                if (qnw) qk_prep(y, qnw, a.rope + (size_t) (a.n0 + t) * 32);
+                if (qnw) qk_prep(y, qnw, a.rope + (size_t) (P.n0 + t) * 32);
                 if (krot) fwht256_w64(y);
                 o0[0] = (_Float16) (y[0] * 0.0625f); // (pair order, as the K fragments)
                 o0[1] = (_Float16) (y[2] * 0.0625f);
@@ -528,9 +562,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __syncthreads(); // every wave holds its fragments: the staging area is free
     issue(0);
     const int row = r0 + 32 * wr + c;
-    const int lim = row < a.R ? a.n0 + row / GQA : -1;
-    const int lim_min = a.n0 + (r0 + 32 * wr) / GQA;
-    const bool rows = r0 + 32 * wr < a.R; // the wave has rows at all
+    const int lim = row < P.R ? P.n0 + row / GQA : -1;
+    const int lim_min = P.n0 + (r0 + 32 * wr) / GQA;
+    const bool rows = r0 + 32 * wr < P.R; // the wave has rows at all
     float m = -INFINITY, ls = 0.f;        // running max (log2 units) and sum
     f32x16 O[8];
 #pragma unroll
@@ -553,52 +587,54 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int ks = 0; ks < 16; ks++)
             sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(tile + 1024 * ks), qf[ks], sacc, 0, 0, 0);
         pipeline_reads<PF_AHEAD, 16>();
-        float mx = -INFINITY;
-        if (p0 + ATP - 1 <= lim_min) { // fully visible tiles (wave-uniform) skip the causal mask
+        // the first V fragments, in flight during the softmax
+        half8 va[PF_AHEAD];
 #pragma unroll
-            for (int e = 0; e < 16; e++) mx = fmaxf(mx, sacc[e]);
-        } else {
+        for (int j = 0; j < PF_AHEAD; j++) va[j] = *reinterpret_cast<const half8 *>(tile + 1024 * (16 + 2 * j));
+        if (p0 + ATP - 1 > lim_min) { // fully visible tiles (wave-uniform) skip the causal mask
 #pragma unroll
             for (int e = 0; e < 16; e++) {
                 const int pos = p0 + 8 * (e >> 2) + 4 * hf + (e & 3);
                 sacc[e] = pos <= lim ? sacc[e] : -INFINITY;
-                mx = fmaxf(mx, sacc[e]);
             }
         }
+        // maxima and sums as four independent chains: a wave's own dependent instructions are what a step waits for
+        float mx4[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) mx4[e] = fmaxf(fmaxf(sacc[e], sacc[4 + e]), fmaxf(sacc[8 + e], sacc[12 + e]));
+        float mx = fmaxf(fmaxf(mx4[0], mx4[1]), fmaxf(mx4[2], mx4[3]));
         mx = fmaxf(mx, shfl_xor(mx, 32)) * LOG2E;
         const float mnew = mx > m + RESCALE_LOG2 ? mx : m;
-        float al = 1.f, ps = 0.f;
-        if (mnew != -INFINITY) {
-            al = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mnew);
-#pragma unroll
-            for (int e = 0; e < 16; e++) {
-                sacc[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[e], LOG2E, -mnew));
-                ps += sacc[e];
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 16; e++) sacc[e] = 0.f;
-        }
-        ps += shfl_xor(ps, 32);
-        const bool rescale = al != 1.f && m != -INFINITY;
-        ls = __builtin_fmaf(ls, al, ps);
-        m = mnew;
-        if (__any(rescale)) {
+        const float al = m == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mnew); // (O and l are zero before the first key)
+        if (__any(al != 1.f)) {
 #pragma unroll
             for (int db = 0; db < 8; db++) O[db] *= al;
         }
+        const float sh = mnew == -INFINITY ? 0.f : -mnew; // (no visible key yet: every P is exp2(-inf) = 0)
+        m = mnew;
+        // P of positions 16 s2 .. (half of the tile) and its share of O += P V: the second half's exponentials run under
+        // the first half's MFMAs
         half8 pb[2];
 #pragma unroll
-        for (int s2 = 0; s2 < 2; s2++)
+        for (int s2 = 0; s2 < 2; s2++) {
 #pragma unroll
-            for (int e = 0; e < 8; e++) pb[s2][e] = (_Float16) sacc[8 * s2 + e];
+            for (int e = 8 * s2; e < 8 * s2 + 8; e++) {
+                sacc[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[e], LOG2E, sh));
+                pb[s2][e - 8 * s2] = (_Float16) sacc[e];
+            }
 #pragma unroll
-        for (int db = 0; db < 8; db++)
+            for (int db = 0; db < 8; db++) {
+                const half8 v = s2 == 0 && db < PF_AHEAD ? va[db] : *reinterpret_cast<const half8 *>(tile + 1024 * (16 + 2 * db + s2));
+                O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, pb[s2], O[db], 0, 0, 0);
+            }
+        }
+        float ps4[4];
 #pragma unroll
-            for (int s2 = 0; s2 < 2; s2++)
-                O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(tile + 1024 * (16 + 2 * db + s2)), pb[s2], O[db],
-                                                               0, 0, 0);
-        pipeline_reads<PF_AHEAD, 16>();
+        for (int e = 0; e < 4; e++) ps4[e] = (sacc[e] + sacc[4 + e]) + (sacc[8 + e] + sacc[12 + e]);
+        float ps = (ps4[0] + ps4[1]) + (ps4[2] + ps4[3]);
+        ps += shfl_xor(ps, 32);
+        ls = __builtin_fmaf(ls, al, ps);
+        pipeline_pv();
     }
     // ---- the two parities of each row, even tiles first: M = max, O = e0 O0 + e1 O1, l likewise.  Each wave gives the
     // other parity's wave half of its dims (blocks 4 (1 - par) .. + 3) and finishes the other half
@@ -618,12 +654,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             s_o[(wv * 16 + 4 * d + j) * 64 + lane] = x;
         }
     __syncthreads();
-    if (row < a.R) {
+    if (row < P.R) {
         const float2 ml0 = s_ml[wr * 32 + c], ml1 = s_ml[(4 + wr) * 32 + c];
         const float M = fmaxf(ml0.x, ml1.x);
         const float e0 = ml0.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml0.x - M);
         const float e1 = ml1.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml1.x - M);
-        const size_t at = ((size_t) u * a.nseg + k) * a.R + row;
+        const size_t at = (size_t) P.part0 + ((size_t) u * P.nseg + k) * P.R + row;
         if (hf == 0 && par == 0) a.ml[at] = make_float2(M, __builtin_fmaf(e1, ml1.y, e0 * ml0.y));
         float * const dst = a.part + at * HD;
         const float4 * const o = s_o + ((wv ^ 4) * 16) * 64 + lane;
@@ -644,25 +680,31 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
-// One wave per (layer, kv head, row) of a prefill piece: the row's segments 0 .. pos / a.seg folded in segment order
-// (M' = max(M, m_k), O' = O e^(M - M') + O_k e^(m_k - M'), l likewise; two at most, pf_seg), y = O / l, then the output
+// One wave per (layer, kv head, row) of the group: the row's segments 0 .. pos / seg folded in segment order
+// (M' = max(M, m_k), O' = O e^(M - M') + O_k e^(m_k - M'), l likewise; eight at most, pf_seg), y = O / l, then the output
 // epilogue.
 __global__ __launch_bounds__(256) void k_prefill_combine(PrefillArgs a) {
-    const int wid = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (wid >= a.R * a.nl * a.ng) return;
-    const int r = wid % a.R, u = wid / a.R, g = a.g0 + u % a.ng, l = u / a.ng;
-    const int t = r / GQA, hh = r - GQA * t, pos = a.n0 + t;
-    const int nk = pos / a.seg + 1;
+    const int wid = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    int pi = 0;
+#pragma unroll
+    for (int i = 1; i < PF_PIECES; i++)
+        if (i < a.np && wid >= a.pc[i].row0) pi = i;
+    const PrefillPiece P = a.pc[pi];
+    const int w = wid - P.row0;
+    if (w >= P.R * a.nl * a.ng) return;
+    const int r = w % P.R, u = w / P.R, g = a.g0 + u % a.ng, l = u / a.ng;
+    const int t = r / GQA, hh = r - GQA * t, pos = P.n0 + t;
+    const int nk = pos / P.seg + 1;
     float M = -INFINITY, den = 0.f;
     float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
-    constexpr int RND = 2; // one round of loads
+    constexpr int RND = 4; // loaded together
     for (int k0 = 0; k0 < nk; k0 += RND) {
         float2 mls[RND];
         float4 os[RND];
 #pragma unroll
         for (int j = 0; j < RND; j++)
             if (k0 + j < nk) {
-                const size_t at = ((size_t) u * a.nseg + k0 + j) * a.R + r;
+                const size_t at = (size_t) P.part0 + ((size_t) u * P.nseg + k0 + j) * P.R + r;
                 mls[j] = a.ml[at];
                 os[j] = *reinterpret_cast<const float4 *>(a.part + at * HD + 4 * lane);
             }
@@ -684,7 +726,7 @@ __global__ __launch_bounds__(256) void k_prefill_combine(PrefillArgs a) {
     }
     float v[4] = {num.x / den, num.y / den, num.z / den, num.w / den};
     const int h = GQA * g + hh;
-    const size_t trow = (size_t) l * a.T + t;
+    const size_t trow = (size_t) l * a.T + P.t0 + t;
     finish_row(v, (a.vrot >> (a.layer + l)) & 1u, a.gate ? a.gate + (trow * NH + h) * a.gs : nullptr, a.out + (trow * NH + h) * HD, a.q32a,
                a.q32b, a.q32m, trow, h);
 }
@@ -803,23 +845,36 @@ static PrefillKernel pick_prefill_kv(int kb, int vb) {
 #undef QKV_VB
 }
 
-hipError_t launch_prefill(const PrefillArgs & a, int kb, int vb, hipStream_t st) {
+hipError_t launch_prefill_kv(const PrefillArgs & a, int kb, int vb, hipStream_t st) {
     PrefillKernel kv = pick_prefill_kv(kb, vb);
     if (!kv) return hipErrorInvalidValue;
+    const int tiles = a.p1 - a.p0 + a.q1 - a.q0;
+    if (tiles > 0) hipLaunchKernelGGL(kv, dim3(tiles, a.nl * a.ng), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_prefill(PrefillArgs & a, hipStream_t st) {
     static thread_local bool configured = false;
     if (!configured) {
         const hipError_t e = hipFuncSetAttribute((const void *) k_prefill_attn, hipFuncAttributeMaxDynamicSharedMemorySize, PA_LDS);
         if (e != hipSuccess) return e;
         configured = true;
     }
-    const int units = a.nl * a.ng, tiles = (a.L + ATP - 1) / ATP - a.t0;
-    hipLaunchKernelGGL(kv, dim3(tiles, units), dim3(256), 0, st, a);
-    hipError_t e = hipGetLastError();
+    const int units = a.nl * a.ng;
+    int blocks = 0, rows = 0, part = 0;
+    for (int i = 0; i < a.np; i++) {
+        PrefillPiece & P = a.pc[i];
+        P.blk0 = blocks;
+        P.row0 = rows;
+        P.part0 = part;
+        blocks += (P.R + PF2_ROWS - 1) / PF2_ROWS * units * P.nseg;
+        rows += P.R * units;
+        part += P.R * units * P.nseg;
+    }
+    hipLaunchKernelGGL(k_prefill_attn, dim3(blocks), dim3(512), PA_LDS, st, a);
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_prefill_attn, dim3(a.nrb * units * a.nseg), dim3(512), PA_LDS, st, a);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_prefill_combine, dim3((a.R * units + 3) / 4), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_prefill_combine, dim3((rows + 3) / 4), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 

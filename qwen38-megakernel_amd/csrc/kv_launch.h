@@ -122,21 +122,29 @@ inline void fill_head(AttnArgs & a) {
     h.pad[0] = h.pad[1] = h.pad[2] = 0;
 }
 
-// one prefill piece over a run of layers with the same K / V bits: query rows r = 6 t + hh (token t = 0 .. Tp-1 at
-// position n0 + t, query head 6 g + hh of kv head g), keys in absolute segments of `seg` positions (pf_seg of the
-// piece's bucket).  Unit u = l ng + (g - g0): layer l of the run, kv head g
+// one prefill piece: the rows of a call that share a 640-position bucket (one window start, one segment length)
+struct PrefillPiece {
+    int n0, R, ws;  // first query position, 6 rows per token, window start: keys from ws on are the window's q8 rows
+    int seg, nseg;  // key positions per segment (pf_seg), ceil(L / seg) segments of the piece's context L
+    int t0;         // the piece's first token within the group
+    int blk0, row0; // first workgroup of the attention, first row of the combine
+    int part0;      // first row of part / ml, in rows
+};
+constexpr int PF_PIECES = 4; // pieces per launch at most
+// a group of consecutive prefill pieces over a run of layers with the same K / V bits: query rows r = 6 t + hh (token t of a
+// piece, query head 6 g + hh of kv head g).  Unit u = l ng + (g - g0): layer l of the run, kv head g
 struct PrefillArgs {
     StoreLayout S;
     int layer, seq;    // first slot of the run
     int nl, g0, ng;    // layers and kv heads (g0 .. g0 + ng - 1) of the launch
-    int n0, Tp, L, ws; // first query position, rows' tokens, L = n0 + Tp (one 640-bucket), window start of the bucket
+    int np;            // pieces, the longest context first in blk0 order
+    PrefillPiece pc[PF_PIECES];
     int T;             // tokens of the whole call (a layer's stride in q, out, gate and the units)
-    int R, nrb, nseg;  // 6 Tp rows per kv head, ceil(R / PF2_ROWS) row blocks, ceil(L / seg) key segments
-    int seg;           // key positions per segment
-    int t0, kv_tiles;  // first tile that k_prefill_kv (re)writes; tiles per unit of kv16
-    int skip0, skip1;  // tiles skip0 .. skip1 - 1 are as the previous piece left them
+    int L;             // stored positions after the group
+    int p0, p1, q0, q1; // tiles that k_prefill_kv writes: p0 .. p1 - 1 from the main rows, q0 .. q1 - 1 from the window's
+    int kv_tiles, q_tiles; // tiles per unit of kv16 (main rows) and kq16 (window rows, tile t at t % q_tiles)
     unsigned krot, vrot; // per-slot bit masks: K / V stored rotated
-    const float * q;   // [nl][T][NH][qs] from the piece's first token
+    const float * q;   // [nl][T][NH][qs] from the group's first token
     int qs;
     const float * qnw; // optional q-norm weights [nl][HD] (the Q prep, table rope)
     const float2 * rope;
@@ -146,19 +154,23 @@ struct PrefillArgs {
     int8_t * q32a;     // optional o_proj units [nl][T][192][16] (a / b), meta [nl][T][192][4]
     int8_t * q32b;
     uint16_t * q32m;
-    uint8_t * kv16;    // [nl ng][kv_tiles][KV16_TILE] fp16 operand tiles (kv_attn.hip)
-    float * part;      // [nl ng][nseg][R][HD] per-segment partial outputs (unnormalised)
-    float2 * ml;       // [nl ng][nseg][R] (max in log2 units, sum)
+    uint8_t * kv16;    // [nl ng][kv_tiles][KV16_TILE] fp16 operand tiles (kv_attn.hip) of the main rows
+    uint8_t * kq16;    // [nl ng][q_tiles][KV16_TILE] of the window rows
+    float * part;      // per piece [nl ng][nseg][R][HD] per-segment partial outputs (unnormalised)
+    float2 * ml;       // per piece [nl ng][nseg][R] (max in log2 units, sum)
 };
 constexpr int KV16_TILE = 2 * ATP * HD * 2; // one tile's K and V as fp16
-// key positions per prefill segment: 128 ceil(Lb / 256) with Lb = L rounded up to its 640-bucket: two segments per row
-// at most, the same segments for every row of a bucket (every row's result is a function of its position).  A full
-// 640-position piece then runs 30 row blocks x 4 kv heads x 2 segments = 240 workgroups, one round on 256 CUs at one
-// workgroup per CU; more segments repeat each workgroup's query staging and partial stores, and odd counts leave a
-// partial round (3, 4 or 8 segments measured 9-23% slower on a 16,384-position prompt, one segment 39%)
+// key positions per prefill segment: 2, 4 or 8 segments over the row's 640-bucket end, in multiples of 128 -- the same for
+// every row of a bucket (every row's result is a function of its position).  A workgroup is (128 query rows, kv head,
+// segment): a full 640-position piece has 240 of them with two segments, one round on 256 CUs, and more segments repeat
+// each workgroup's query staging and partial stores.  Short chunks far into a context have few row blocks, so more
+// segments pay there (60,000 positions, 2 / 4 / 8 segments: 16 tokens 731 / 412 / 252 us, 256 tokens 706 / 474 / 506, 512
+// tokens 830 / 862 / 811, 640 tokens 946 / 962 / 1,003), and up to 20,480 positions whole prompts decide (16,384 with
+// four segments: 9% slower).
 inline int pf_seg(int L) {
     const int lb = (L + ATT_BUCKET - 1) / ATT_BUCKET * ATT_BUCKET;
-    return 128 * ((lb + 255) / 256);
+    const int n = lb > 64 * ATT_BUCKET ? 8 : lb > 32 * ATT_BUCKET ? 4 : 2;
+    return 128 * ((lb + 128 * n - 1) / (128 * n));
 }
 constexpr int PF2_ROWS = 128; // query rows per prefill workgroup (32 per wave)
 
@@ -188,7 +200,9 @@ hipError_t launch_attn(const AttnArgs & a, int kb, int vb, int max_blocks, int o
 // the first `tiles` tiles of every wave slice of the attention launch `a` read into the L2 its workgroups will use
 hipError_t launch_prefetch(const AttnArgs & a, int kb, int vb, int tiles, hipStream_t st);
 hipError_t launch_combine(const AttnArgs & a, hipStream_t st, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
-// the piece's keys as fp16 tiles (tiles t0 ..), the attention and the combine
-hipError_t launch_prefill(const PrefillArgs & a, int kb, int vb, hipStream_t st);
+// the tiles p0 .. and q0 .. as fp16 operands
+hipError_t launch_prefill_kv(const PrefillArgs & a, int kb, int vb, hipStream_t st);
+// the group's attention and combine (fills blk0 and row0)
+hipError_t launch_prefill(PrefillArgs & a, hipStream_t st);
 
 } // namespace qkv

@@ -13,7 +13,7 @@ store's last T positions):
         equal; at T = 8 tokens 0 and 5 bitwise equal to one-token calls at their own lengths.
 (T = 1, 2, 3, 4, 5, 8: the reference's own T set for this matrix.)
 One case at 200,031 positions (bucket 200,320, 13 tiles per wave) runs D at T = 1 and 8.  The prefill kernel of each
-format (k_prefill3, one instantiation per (K bits, V bits) pair as well) runs a 2,600-position prompt.
+format (k_prefill_kv, one instantiation per (K bits, V bits) pair as well) runs a 2,600-position prompt.
 """
 from concurrent.futures import ThreadPoolExecutor
 

@@ -207,3 +207,69 @@ def test_prefill_after_appends(qkv, oracle, torch_gpu, spec, win, win_all):
                                  ring_k, ring_v)
         assert rel_err(out[0, a - P0:b - P0], ref) <= 2e-3, (a, b)
     st.close()
+
+
+def fill(torch, st, P, nl, seed, chunk=4096):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    for p in range(0, P, chunk):
+        c = min(chunk, P - p)
+        k, v = (torch.randn(c, nl, NKV, HD, device="cuda", dtype=torch.float16, generator=g) for _ in range(2))
+        st.append(0, 0, nl, p, c, k.data_ptr(), v.data_ptr(), 1)
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("L0,T,spec,win", [(20700, 400, "K*=5r,V*=6", 2048), (41000, 300, "K*=6r,V*=4r", 1024), (170000, 70, "", 0)])
+def test_prefill_far_into_a_context(qkv, torch_gpu, L0, T, spec, win):
+    """Chunks far into a context: four key segments per row past 20,480 positions, eight past 40,960 (both across the
+    boundary of the rule and of a 640-position bucket), and a context whose fp16 tiles exceed the scratch for all four kv
+    heads at once.  Bitwise the same in one chunk and in three, and each row within the two forms' tolerances (2e-3 each
+    of the exact attention) of the decode attention at its length."""
+    torch = torch_gpu
+    g = torch.Generator(device="cuda")
+    g.manual_seed(L0)
+    k, v = (torch.randn(T, 1, NKV, HD, device="cuda", generator=g) for _ in range(2))
+    q = torch.randn(1, T, NH, HD, device="cuda", generator=g)
+    outs = []
+    for chunks in ([T], [T // 3, 1, T - T // 3 - 1]):
+        st = qkv.KVStore(spec, win=win, n_layers=1, ctx=L0 + T)
+        fill(torch, st, L0, 1, L0 + 1)
+        o, p = torch.full_like(q, float("nan")), 0
+        for c in chunks:
+            oc = torch.empty(1, c, NH, HD, device="cuda")
+            st.prefill(0, 0, 1, L0 + p, c, k[p:].data_ptr(), v[p:].data_ptr(), 0, q[0, p:].data_ptr(), oc.data_ptr())
+            torch.cuda.synchronize()
+            o[:, p:p + c] = oc
+            p += c
+        outs.append(o)
+        if len(outs) == 1:
+            st.close()
+    assert torch.equal(outs[0], outs[1])
+    d = torch.empty(1, 1, 1, NH, HD, device="cuda")
+    for t in (T - 1, T - 30, T - 59):  # (rows of the last bucket: the ring still holds their windows)
+        st.attend(0, 1, [0], [L0 + t + 1], 1, q[0, t].data_ptr(), d.data_ptr())
+        torch.cuda.synchronize()
+        assert rel_err(outs[0][0, t].cpu().numpy(), d[0, 0, 0].cpu().numpy()) <= 2 * 2e-3, t
+    st.close()
+
+
+def test_prefill_more_layers_than_the_scratch_holds(qkv, torch_gpu):
+    """17 layers at 9,740 positions: their fp16 tiles exceed the scratch, so each launch holds one layer and one piece and
+    writes all its tiles (window tiles included).  Bitwise the layers' own calls, which keep theirs."""
+    torch = torch_gpu
+    nl, L0, T = 17, 9610, 130  # (one bucket: the ring still holds its window when a layer is stored again)
+    st = qkv.KVStore("K*=5r,V*=6", win=2048, n_layers=nl, ctx=L0 + T)
+    fill(torch, st, L0, nl, 7)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(8)
+    k, v = (torch.randn(T, nl, NKV, HD, device="cuda", generator=g) for _ in range(2))
+    q = torch.randn(nl, T, NH, HD, device="cuda", generator=g)
+    o = torch.full_like(q, float("nan"))
+    st.prefill(0, 0, nl, L0, T, k.data_ptr(), v.data_ptr(), 0, q.data_ptr(), o.data_ptr())
+    torch.cuda.synchronize()
+    for l in (0, 9, 16):
+        kl, vl, ol = k[:, l].contiguous(), v[:, l].contiguous(), torch.empty_like(q[l])
+        st.prefill(0, l, 1, L0, T, kl.data_ptr(), vl.data_ptr(), 0, q[l].contiguous().data_ptr(), ol.data_ptr())
+        torch.cuda.synchronize()
+        assert torch.equal(ol, o[l]), l
+    st.close()
