@@ -44,6 +44,9 @@ __global__ __launch_bounds__(256) void k_prefetch(AttnArgs a, int tiles) {
 }
 
 // ------------------------------------------------------------------------------------------------ output epilogue
+// the sigmoid output gate (qwen38_mk.cu:4686)
+__device__ __forceinline__ float gated(float v, float g) { return v / (1.0f + expf(-g)); }
+
 // One output row y (head h of token row trow, lane l holding dims 4l .. 4l+3) after the merge: the V un-rotation when
 // V is stored rotated, the sigmoid output gate (qwen38_mk.cu:4686) when grow is given, the fp32 store, and when q32a
 // is given the o_proj activation units of q32_store (qwen38_mk.cu:283-307): block k = lane / 8 of the head's 8 blocks of
@@ -55,10 +58,10 @@ __device__ __forceinline__ void finish_row(float (&v)[4], bool vrot, const float
     if (vrot) fwht256_w64(v);
     if (grow) {
         const float4 gt = *reinterpret_cast<const float4 *>(grow + 4 * lane);
-        v[0] = v[0] / (1.0f + expf(-gt.x));
-        v[1] = v[1] / (1.0f + expf(-gt.y));
-        v[2] = v[2] / (1.0f + expf(-gt.z));
-        v[3] = v[3] / (1.0f + expf(-gt.w));
+        v[0] = gated(v[0], gt.x);
+        v[1] = gated(v[1], gt.y);
+        v[2] = gated(v[2], gt.z);
+        v[3] = gated(v[3], gt.w);
     }
     *reinterpret_cast<float4 *>(orow + 4 * lane) = make_float4(v[0], v[1], v[2], v[3]);
     if (q32a) {
@@ -86,17 +89,18 @@ __device__ __forceinline__ void finish_row(float (&v)[4], bool vrot, const float
 
 // ------------------------------------------------------------------------------------------------ combine
 // The merge of a head's segment partials (attn_combine, qwen38_mk.cu:4617-4700: y = sum_c e_c O_c / sum_c e_c l_c with
-// e_c = exp(m_c - M)), in two forms with fixed orders (no bit depends on scheduling):
-//   row form   (combine_row)  one workgroup per output row (layer, sequence, kv head, row r).  Wave w loads the
-//              segments c = w, w+4, .. at once, weights them by exp2(m_c - M_w) against its own maximum M_w and sums
-//              them in segment order; the four wave sums are rescaled to M = max M_w and added in wave order; y = O / l,
-//              then the V un-rotation, gate and o_proj units (finish_row).
-//   split form (combine_split) one workgroup per (output row, 64-dim quarter), for launches without rotated V, gate or
-//              units.  Lane group s = 4 w + l / 16 takes the segments c = s, s + 16, .. and sums them the same way;
-//              the 4 groups of a wave are merged by permlane swaps, the 4 waves in wave order.
+// e_c = exp(m_c - M)).  16 slots: slot s takes the segments c = s, s + 16, .., weighted by exp2(m_c - M_s) against its own
+// maximum M_s and summed in segment order; slots 4 w .. 4 w + 3 are merged pairwise, ((0, 1), (2, 3)), then the four
+// groups in order (fixed orders: no bit depends on scheduling).  In two forms, the same bits before the epilogue:
+//   split form  one workgroup per (output row, 64-dim quarter), for launches without rotated V or o_proj units.  A slot is a
+//               16-lane group: 4 waves hold the 16 slots.  The gate, elementwise, is applied here.
+//   row form    one workgroup of 16 waves per output row, a slot per wave, then the V un-rotation, gate and o_proj units
+//               of the whole row (finish_row).
+// A combine waits on one round of loads from beyond the writers' L2s, so both forms have 8 loads per lane at most in
+// flight at once (the row form with 4 waves of 32 loads: 7.4 against 5.9 us on 96 rows of 105 segments).
 // Both run as a kernel of their own after the attention launch (an in-launch merge by extra workgroups that wait for
 // a head's segments measured slower: partials then have to be written through to the coherence point shared by the
-// XCDs before the waiting workgroup may read them).  scratch: LDS of 4 KiB + 32 B.
+// XCDs before the waiting workgroup may read them).
 // the output row of combine workgroup b of a launch: (layer, sequence, kv head, row r) with r fastest
 struct CombineRow {
     int l, si, g, r;
@@ -112,66 +116,141 @@ __device__ __forceinline__ CombineRow combine_row_of(const AttnArgs & a, int b) 
     return c;
 }
 
-__device__ __forceinline__ void combine_row(const AttnArgs & a, const CombineRow & cr, uint8_t * scratch) {
-    float4 (*s_num)[64] = reinterpret_cast<float4 (*)[64]>(scratch);         // [AWAVES][64]
-    float2 * s_md = reinterpret_cast<float2 *>(scratch + AWAVES * 64 * 16); // [AWAVES] (max, denominator)
-    const int R = a.R, T = a.T, r = cr.r, g = cr.g, si = cr.si, l = cr.l;
-    const SeqDesc & sd = a.sd[si];
-    const int nseg = sd.nseg;
-    const size_t head0 = (size_t) sd.item0 + (size_t) (l * NKV + g) * nseg;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    // one round of loads: wave w's segments c = w, w + 4, .. (all issued before any is used)
-    constexpr int PER = MAX_SEG / AWAVES;
-    float2 ml[PER];
-    float4 o[PER];
+constexpr int CSLOTS = 16, CPER = MAX_SEG / CSLOTS; // slots, segments per slot at most
+
+// one slot's share of a row: segments slot, slot + 16, .. of the head whose segment 0 is item head0, dims dim .. dim + 3
+struct CombineAcc {
+    float4 num;
+    float den, M;
+};
+__device__ __forceinline__ CombineAcc combine_slot(const float * __restrict__ part, const float2 * __restrict__ ml_, size_t head0, int nseg, int R,
+                                                   int r, int slot, int dim) {
+    float2 ml[CPER];
+    float4 o[CPER];
 #pragma unroll
-    for (int k = 0; k < PER; k++) {
-        const int c = wv + AWAVES * k;
+    for (int k = 0; k < CPER; k++) {
+        const int c = slot + CSLOTS * k;
         if (c < nseg) {
-            ml[k] = a.ml[(head0 + c) * R + r];
-            o[k] = *reinterpret_cast<const float4 *>(a.part + ((head0 + c) * R + r) * HD + 4 * lane);
+            ml[k] = ml_[(head0 + c) * R + r];
+            o[k] = *reinterpret_cast<const float4 *>(part + ((head0 + c) * R + r) * HD + dim);
         }
     }
-    float Mw = -INFINITY;
+    CombineAcc x{make_float4(0.f, 0.f, 0.f, 0.f), 0.f, -INFINITY};
 #pragma unroll
-    for (int k = 0; k < PER; k++)
-        if (wv + AWAVES * k < nseg) Mw = fmaxf(Mw, ml[k].x);
-    float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
-    float den = 0.f;
+    for (int k = 0; k < CPER; k++)
+        if (slot + CSLOTS * k < nseg) x.M = fmaxf(x.M, ml[k].x);
 #pragma unroll
-    for (int k = 0; k < PER; k++) {
-        const int c = wv + AWAVES * k;
-        if (c < nseg) {
-            const float e = ml[k].x == -INFINITY ? 0.f : exp2f(ml[k].x - Mw);
-            num.x = __builtin_fmaf(e, o[k].x, num.x);
-            num.y = __builtin_fmaf(e, o[k].y, num.y);
-            num.z = __builtin_fmaf(e, o[k].z, num.z);
-            num.w = __builtin_fmaf(e, o[k].w, num.w);
-            den = __builtin_fmaf(e, ml[k].y, den);
+    for (int k = 0; k < CPER; k++) {
+        if (slot + CSLOTS * k < nseg) {
+            const float e = ml[k].x == -INFINITY ? 0.f : exp2f(ml[k].x - x.M);
+            x.num.x = __builtin_fmaf(e, o[k].x, x.num.x);
+            x.num.y = __builtin_fmaf(e, o[k].y, x.num.y);
+            x.num.z = __builtin_fmaf(e, o[k].z, x.num.z);
+            x.num.w = __builtin_fmaf(e, o[k].w, x.num.w);
+            x.den = __builtin_fmaf(e, ml[k].y, x.den);
         }
     }
-    s_num[wv][lane] = num;
-    if (lane == 0) s_md[wv] = make_float2(Mw, den);
+    return x;
+}
+// x weighted by e
+__device__ __forceinline__ void combine_scale(CombineAcc & x, float e) {
+    x.num.x *= e;
+    x.num.y *= e;
+    x.num.z *= e;
+    x.num.w *= e;
+    x.den *= e;
+}
+// the four groups of slots (sums against maximum md.x, denominators md.y) in order, y = O / l; s_num: group k's float4 at
+// s_num[stride k]
+__device__ __forceinline__ float4 combine_groups(const float4 * s_num, int stride, const float2 (&md)[AWAVES]) {
+    float M = md[0].x;
+#pragma unroll
+    for (int k = 1; k < AWAVES; k++) M = fmaxf(M, md[k].x);
+    float4 y = make_float4(0.f, 0.f, 0.f, 0.f);
+    float dd = 0.f;
+#pragma unroll
+    for (int k = 0; k < AWAVES; k++) {
+        const float e = md[k].x == -INFINITY ? 0.f : exp2f(md[k].x - M);
+        const float4 z = s_num[stride * k];
+        y.x = __builtin_fmaf(e, z.x, y.x);
+        y.y = __builtin_fmaf(e, z.y, y.y);
+        y.z = __builtin_fmaf(e, z.z, y.z);
+        y.w = __builtin_fmaf(e, z.w, y.w);
+        dd = __builtin_fmaf(e, md[k].y, dd);
+    }
+    return make_float4(y.x / dd, y.y / dd, y.z / dd, y.w / dd);
+}
+// one (row, 64-dim quarter dq) of the output from the row's segment partials; part / ml / out / gate as in AttnArgs, nseg
+// and item0 those of the row's sequence si
+__device__ __forceinline__ void combine_split_core(const float * __restrict__ part, const float2 * __restrict__ ml_, float * out, const float * gate,
+                                                   int gs, int R, int T, int nseq, int nseg, int item0, const CombineRow & cr, int dq) {
+    __shared__ float4 s_num[AWAVES][16];
+    __shared__ float2 s_md[AWAVES];
+    const int r = cr.r, g = cr.g, si = cr.si, l = cr.l;
+    const size_t head0 = (size_t) item0 + (size_t) (l * NKV + g) * nseg;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, sub = lane >> 4, dl = lane & 15;
+    const int dim = 64 * dq + 4 * dl;
+    const int h = GQA * g + r / T, t = r % T;
+    const size_t orow = ((size_t) (l * nseq + si) * T + t) * NH + h;
+    float4 gt = make_float4(0.f, 0.f, 0.f, 0.f); // (loaded with the partials)
+    if (gate && wv == 0 && sub == 0) gt = *reinterpret_cast<const float4 *>(gate + orow * gs + dim);
+    CombineAcc x = combine_slot(part, ml_, head0, nseg, R, r, 4 * wv + sub, dim);
+    // the wave's 4 lane groups (same dims, slots 4 w .. 4 w + 3)
+    const float Mw = quad_max(x.M);
+    combine_scale(x, x.M == -INFINITY ? 0.f : exp2f(x.M - Mw));
+    x.num.x = quad_sum(x.num.x);
+    x.num.y = quad_sum(x.num.y);
+    x.num.z = quad_sum(x.num.z);
+    x.num.w = quad_sum(x.num.w);
+    x.den = quad_sum(x.den);
+    if (sub == 0) s_num[wv][dl] = x.num;
+    if (lane == 0) s_md[wv] = make_float2(Mw, x.den);
+    __syncthreads();
+    if (wv == 0 && sub == 0) {
+        const float2 md[AWAVES] = {s_md[0], s_md[1], s_md[2], s_md[3]};
+        float4 y = combine_groups(&s_num[0][dl], 16, md);
+        if (gate) y = make_float4(gated(y.x, gt.x), gated(y.y, gt.y), gated(y.z, gt.z), gated(y.w, gt.w));
+        *reinterpret_cast<float4 *>(out + orow * HD + dim) = y;
+    }
+}
+
+__global__ __launch_bounds__(64 * CSLOTS) void k_combine(AttnArgs a) {
+    __shared__ float4 s_num[CSLOTS][64];
+    __shared__ float2 s_md[CSLOTS];
+    const CombineRow cr = combine_row_of(a, blockIdx.x);
+    const int r = cr.r, g = cr.g, si = cr.si, l = cr.l, T = a.T;
+    const int nseg = a.sd[si].nseg;
+    const size_t head0 = (size_t) a.sd[si].item0 + (size_t) (l * NKV + g) * nseg;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const CombineAcc x = combine_slot(a.part, a.ml, head0, nseg, a.R, r, wv, 4 * lane);
+    s_num[wv][lane] = x.num;
+    if (lane == 0) s_md[wv] = make_float2(x.M, x.den);
+    __syncthreads();
+    if (wv >= AWAVES) return;
+    // wave w merges slots 4 w .. 4 w + 3 pairwise
+    {
+        float2 md[4];
+        float M = -INFINITY;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            md[k] = s_md[4 * wv + k];
+            M = fmaxf(M, md[k].x);
+        }
+        CombineAcc y[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            y[k] = CombineAcc{s_num[4 * wv + k][lane], md[k].y, md[k].x};
+            combine_scale(y[k], md[k].x == -INFINITY ? 0.f : exp2f(md[k].x - M));
+        }
+        s_num[4 * wv][lane] = make_float4((y[0].num.x + y[1].num.x) + (y[2].num.x + y[3].num.x), (y[0].num.y + y[1].num.y) + (y[2].num.y + y[3].num.y),
+                                          (y[0].num.z + y[1].num.z) + (y[2].num.z + y[3].num.z), (y[0].num.w + y[1].num.w) + (y[2].num.w + y[3].num.w));
+        if (lane == 0) s_md[4 * wv] = make_float2(M, (y[0].den + y[1].den) + (y[2].den + y[3].den));
+    }
     __syncthreads();
     if (wv == 0) {
-        // the 4 wave sums in wave order, each rescaled to the overall max
-        float M = s_md[0].x;
-#pragma unroll
-        for (int k = 1; k < AWAVES; k++) M = fmaxf(M, s_md[k].x);
-        float4 y = make_float4(0.f, 0.f, 0.f, 0.f);
-        float dd = 0.f;
-#pragma unroll
-        for (int k = 0; k < AWAVES; k++) {
-            const float2 md = s_md[k];
-            const float e = md.x == -INFINITY ? 0.f : exp2f(md.x - M);
-            const float4 z = s_num[k][lane];
-            y.x = __builtin_fmaf(e, z.x, y.x);
-            y.y = __builtin_fmaf(e, z.y, y.y);
-            y.z = __builtin_fmaf(e, z.z, y.z);
-            y.w = __builtin_fmaf(e, z.w, y.w);
-            dd = __builtin_fmaf(e, md.y, dd);
-        }
-        float v[4] = {y.x / dd, y.y / dd, y.z / dd, y.w / dd};
+        const float2 md[AWAVES] = {s_md[0], s_md[4], s_md[8], s_md[12]};
+        const float4 y = combine_groups(&s_num[0][lane], 4 * 64, md);
+        float v[4] = {y.x, y.y, y.z, y.w};
         const int h = GQA * g + r / T, t = r % T;
         const size_t trow = (size_t) (l * a.nseq + si) * T + t; // the token's row of 24 x 256 outputs
         finish_row(v, (a.vrot >> (a.layer0 + l)) & 1u, a.gate ? a.gate + (trow * NH + h) * a.gs : nullptr, a.out + (trow * NH + h) * HD,
@@ -179,94 +258,16 @@ __device__ __forceinline__ void combine_row(const AttnArgs & a, const CombineRow
     }
 }
 
-// one (row, 64-dim quarter dq) of the output from the row's segment partials; part / ml / out as in AttnArgs, nseg and
-// item0 those of the row's sequence si
-__device__ __forceinline__ void combine_split_core(const float * __restrict__ part, const float2 * __restrict__ ml_, float * out, int R, int T,
-                                                   int nseq, int nseg, int item0, const CombineRow & cr, int dq, uint8_t * scratch) {
-    float4 (*s_num)[16] = reinterpret_cast<float4 (*)[16]>(scratch);        // [AWAVES][16]
-    float2 * s_md = reinterpret_cast<float2 *>(scratch + AWAVES * 16 * 16); // [AWAVES]
-    const int r = cr.r, g = cr.g, si = cr.si, l = cr.l;
-    const size_t head0 = (size_t) item0 + (size_t) (l * NKV + g) * nseg;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, sub = lane >> 4, dl = lane & 15;
-    const int slot = 4 * wv + sub, dim = 64 * dq + 4 * dl;
-    constexpr int PER = MAX_SEG / 16;
-    float2 ml[PER];
-    float4 o[PER];
-#pragma unroll
-    for (int k = 0; k < PER; k++) {
-        const int c = slot + 16 * k;
-        if (c < nseg) {
-            ml[k] = ml_[(head0 + c) * R + r];
-            o[k] = *reinterpret_cast<const float4 *>(part + ((head0 + c) * R + r) * HD + dim);
-        }
-    }
-    float Ms = -INFINITY;
-#pragma unroll
-    for (int k = 0; k < PER; k++)
-        if (slot + 16 * k < nseg) Ms = fmaxf(Ms, ml[k].x);
-    float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
-    float den = 0.f;
-#pragma unroll
-    for (int k = 0; k < PER; k++) {
-        if (slot + 16 * k < nseg) {
-            const float e = ml[k].x == -INFINITY ? 0.f : exp2f(ml[k].x - Ms);
-            num.x = __builtin_fmaf(e, o[k].x, num.x);
-            num.y = __builtin_fmaf(e, o[k].y, num.y);
-            num.z = __builtin_fmaf(e, o[k].z, num.z);
-            num.w = __builtin_fmaf(e, o[k].w, num.w);
-            den = __builtin_fmaf(e, ml[k].y, den);
-        }
-    }
-    // the wave's 4 lane groups (same dims, slots 4 w .. 4 w + 3)
-    const float Mw = quad_max(Ms);
-    const float ew = Ms == -INFINITY ? 0.f : exp2f(Ms - Mw);
-    num.x = quad_sum(ew * num.x);
-    num.y = quad_sum(ew * num.y);
-    num.z = quad_sum(ew * num.z);
-    num.w = quad_sum(ew * num.w);
-    den = quad_sum(ew * den);
-    if (sub == 0) s_num[wv][dl] = num;
-    if (lane == 0) s_md[wv] = make_float2(Mw, den);
-    __syncthreads();
-    if (wv == 0 && sub == 0) {
-        float M = s_md[0].x;
-#pragma unroll
-        for (int k = 1; k < AWAVES; k++) M = fmaxf(M, s_md[k].x);
-        float4 y = make_float4(0.f, 0.f, 0.f, 0.f);
-        float dd = 0.f;
-#pragma unroll
-        for (int k = 0; k < AWAVES; k++) {
-            const float2 md = s_md[k];
-            const float e = md.x == -INFINITY ? 0.f : exp2f(md.x - M);
-            const float4 z = s_num[k][dl];
-            y.x = __builtin_fmaf(e, z.x, y.x);
-            y.y = __builtin_fmaf(e, z.y, y.y);
-            y.z = __builtin_fmaf(e, z.z, y.z);
-            y.w = __builtin_fmaf(e, z.w, y.w);
-            dd = __builtin_fmaf(e, md.y, dd);
-        }
-        const int h = GQA * g + r / T, t = r % T;
-        *reinterpret_cast<float4 *>(out + (((size_t) (l * nseq + si) * T + t) * NH + h) * HD + dim) =
-            make_float4(y.x / dd, y.y / dd, y.z / dd, y.w / dd);
-    }
-}
-
-__global__ __launch_bounds__(256) void k_combine(AttnArgs a) {
-    __shared__ __attribute__((aligned(16))) uint8_t scratch[AWAVES * 64 * 16 + AWAVES * 8];
-    combine_row(a, combine_row_of(a, blockIdx.x), scratch);
-}
-
 __global__ __launch_bounds__(256) void k_combine_split(AttnArgs a) {
-    __shared__ __attribute__((aligned(16))) uint8_t scratch[AWAVES * 16 * 16 + AWAVES * 8];
     const CombineRow cr = combine_row_of(a, blockIdx.x >> 2);
     const SeqDesc & sd = a.sd[cr.si];
-    combine_split_core(a.part, a.ml, a.out, a.R, a.T, a.nseq, sd.nseg, sd.item0, cr, blockIdx.x & 3, scratch);
+    combine_split_core(a.part, a.ml, a.out, a.gate, a.gs, a.R, a.T, a.nseq, sd.nseg, sd.item0, cr, blockIdx.x & 3);
 }
 
 // the same for one sequence, with every argument a scalar: they arrive preloaded in SGPRs (kernel-argument preloading,
 // build flags of this file), so the partials' loads issue without a round trip to the argument segment first
-__global__ __launch_bounds__(256) void k_combine_split1(const float * part, const float2 * ml, float * out, int R, int T, int nseg, int item0) {
-    __shared__ __attribute__((aligned(16))) uint8_t scratch[AWAVES * 16 * 16 + AWAVES * 8];
+__global__ __launch_bounds__(256) void k_combine_split1(const float * part, const float2 * ml, float * out, int R, int T, int nseg, int item0,
+                                                        const float * gate, int gs) {
     int b = blockIdx.x >> 2;
     CombineRow cr;
     cr.r = b % R;
@@ -274,21 +275,21 @@ __global__ __launch_bounds__(256) void k_combine_split1(const float * part, cons
     cr.g = b % NKV;
     cr.si = 0;
     cr.l = b / NKV;
-    combine_split_core(part, ml, out, R, T, 1, nseg, item0, cr, blockIdx.x & 3, scratch);
+    combine_split_core(part, ml, out, gate, gs, R, T, 1, nseg, item0, cr, blockIdx.x & 3);
 }
 
-// launches whose rows need the whole row in one workgroup (V stored rotated, gate, o_proj units) use the row form
+// launches whose rows need the whole row in one workgroup (V stored rotated, o_proj units) use the row form
 static bool host_combine_needs_rows(const AttnArgs & a) {
     const unsigned vrot = (a.vrot >> a.layer0) & ((a.nl >= 32 ? 0u : 1u << a.nl) - 1u);
-    return vrot || a.gate || a.q32a;
+    return vrot || a.q32a;
 }
 
 hipError_t launch_combine(const AttnArgs & a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
     const unsigned rows = (unsigned) (a.nl * a.nseq * NKV * a.R);
-    if (host_combine_needs_rows(a)) hipExtLaunchKernelGGL(k_combine, dim3(rows), dim3(256), 0, st, ev0, ev1, 0, a);
+    if (host_combine_needs_rows(a)) hipExtLaunchKernelGGL(k_combine, dim3(rows), dim3(64 * CSLOTS), 0, st, ev0, ev1, 0, a);
     else if (a.nseq == 1)
         hipExtLaunchKernelGGL(k_combine_split1, dim3(4 * rows), dim3(256), 0, st, ev0, ev1, 0, (const float *) a.part, (const float2 *) a.ml, a.out,
-                              a.R, a.T, a.sd[0].nseg, a.sd[0].item0);
+                              a.R, a.T, a.sd[0].nseg, a.sd[0].item0, a.gate, a.gs);
     else hipExtLaunchKernelGGL(k_combine_split, dim3(4 * rows), dim3(256), 0, st, ev0, ev1, 0, a);
     return hipGetLastError();
 }

@@ -56,3 +56,35 @@ def test_gated_errors(qkv, torch_gpu):
     with pytest.raises(qkv.KVError):
         st.attend_gated(0, 1, [0], [8], 1, q.data_ptr(), q.data_ptr(), o.data_ptr(), xa.data_ptr())  # a without b / meta
     st.close()
+
+
+@pytest.mark.parametrize("spec,win,lens,T", [
+    ("", 0, [90], 1),                          # one segment
+    ("K*=5r,V*=6", 512, [2100], 3),            # 17 segments: the second round of a slot's loads begins
+    ("K*=5r,V*=5", 2048, [16384, 130], 2),     # 128 segments (the most) beside 2, two sequences
+])
+def test_gate_in_both_merge_forms(qkv, torch_gpu, spec, win, lens, T):
+    # without units the gate is applied by the merge of row quarters, with units by the merge of whole rows: the slots, the
+    # order of their sums and the gate are the same, so the bits are
+    torch = torch_gpu
+    rng = np.random.default_rng(len(lens) + T)
+    nl, nseq = 2, len(lens)
+    st = qkv.KVStore(spec, win=win, n_layers=nl, n_seq=nseq, ctx=max(lens))
+    for s, L in enumerate(lens):
+        K, V = synth_kv(rng, L, nl, outliers=True)
+        append_all(torch, st, s, K, V, chunks=[4096] * 5)
+    q, gate = (torch.from_numpy(rng.standard_normal((nl, nseq, T, NH, HD)).astype(np.float32)).cuda() for _ in range(2))
+    split, rows, plain = (torch.full_like(q, float("nan")) for _ in range(3))
+    xa = torch.zeros((nl, nseq, T, 192, 16), dtype=torch.int8, device="cuda")
+    xb = torch.zeros_like(xa)
+    meta = torch.zeros((nl, nseq, T, 192, 4), dtype=torch.int16, device="cuda")
+    seqs = list(range(nseq))
+    st.attend_gated(0, nl, seqs, lens, T, q.data_ptr(), gate.data_ptr(), split.data_ptr())
+    st.attend_gated(0, nl, seqs, lens, T, q.data_ptr(), gate.data_ptr(), rows.data_ptr(), xa.data_ptr(), xb.data_ptr(), meta.data_ptr())
+    st.attend(0, nl, seqs, lens, T, q.data_ptr(), plain.data_ptr())
+    torch.cuda.synchronize()
+    assert torch.isfinite(split).all() and torch.equal(split, rows)
+    # and the gate is 1 / (1 + exp(-g)) of the ungated row: a few ulp between two libraries' expf and the two quotients
+    exact = plain.double() / (1.0 + torch.exp(-gate.double()))
+    assert ((split.double() - exact).abs() <= 8 * 2.0 ** -24 * exact.abs() + 1e-37).all()
+    st.close()
