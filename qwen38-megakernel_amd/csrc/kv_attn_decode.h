@@ -763,27 +763,39 @@ __device__ __forceinline__ void compute_tile_v(RowState<NP> & st, const half8 * 
     tile_pv<NP, VB, mask_sc<KB, VB>()>(st.acc, raw.v, pb);
 }
 
-// The fused append's rows of one wave (mk_kv_append_attend): positions L - T .. L - 1 of segment [c0, c1) whose tile
-// falls in slice sl, sides w0 .. w1 (0 = K, 1 = V), each stored by store_row exactly as k_append stores it.  Plain
-// values (a called function: inlined, its code made the fused kernels' tile loop slower); called only from the
-// fused-append kernels (APPEND), so the plain kernels carry neither the store code nor a call.
-static __device__ __noinline__ void append_rows(const void * kin, const void * vin, int f16, int kin_nl, const int * ptab, int pt_stride, int page,
-                                         int n_pages, int kvrc, uint8_t * kvals, uint16_t * kscs, int8_t * kring, uint16_t * krsc,
-                                         int kbits, int krot, uint8_t * vvals, uint16_t * vscs, int8_t * vring, uint16_t * vrsc,
-                                         int vbits, int vrot, int seq, int g, int l, int si, int L, int T, int c0, int c1, int sl, int w0,
-                                         int w1) {
-    const RowGeo G{ptab, pt_stride, page, n_pages, kvrc};
-    const SideLayout K{kvals, kscs, kring, krsc, kbits, krot}, V{vvals, vscs, vring, vrsc, vbits, vrot};
-    const int pa = max(L - T, c0), pb = min(L, c1);
-    for (int p = pa; p < pb; p++) {
-        if (((p - c0) >> 5) % AWAVES != sl) continue;
-        const size_t row = ((((size_t) si * T + (p - (L - T))) * kin_nl + l) * NKV + g) * HD;
-        for (int w = w0; w <= w1; w++) {
-            float v[4];
-            load_row4(w ? vin : kin, row, f16, v);
-            store_row(G, w ? V : K, seq, g, p, true, v);
-        }
+// The fused append's rows of one workgroup (mk_kv_append_attend): positions pa .. pb - 1 of its segment, both sides,
+// stored by store_row_at exactly as k_append stores them, row i (side i & 1 of position pa + i / 2) by wave i % nw.  A row is
+// one dependent chain of loads, cross-lane steps and a quotient; spread over the waves, a step's two rows take one chain's
+// time before the tiles are read, not two behind one another in the wave that reads their tile (16 layers at 9,001 positions:
+// 283 -> 265 us).  gbase: the main-store row of position 0 of a sequence with contiguous pages, -1 for others (page
+// table).  in0: the element offset of position pa's input row.  Plain values (a called function: inlined, its code made the
+// fused kernels' tile loop slower) arrive in vector registers: they are made scalar first, so that the chain holds no
+// divergent branch.  Called only from the fused-append kernels (APPEND): the plain kernels carry neither the store code nor
+// a call.  The caller waits for every wave's rows (append_done).
+static __device__ __noinline__ void append_rows(const void * kin, const void * vin, int f16, size_t in0, int in_stride, const int * ptab,
+                                                int pt_stride, int page, int n_pages, int kvrc, uint8_t * kvals, uint16_t * kscs, int8_t * kring,
+                                                uint16_t * krsc, int kbits, int krot, uint8_t * vvals, uint16_t * vscs, int8_t * vring,
+                                                uint16_t * vrsc, int vbits, int vrot, long long gbase, int seq, int g, int pa, int pb, int wv,
+                                                int nw) {
+    auto u = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+    const int n = 2 * (u(pb) - u(pa)), w = u(wv) & 1;
+    const SideLayout sd = w ? SideLayout{uniform_ptr(vvals), uniform_ptr(vscs), uniform_ptr(vring), uniform_ptr(vrsc), u(vbits), u(vrot)}
+                            : SideLayout{uniform_ptr(kvals), uniform_ptr(kscs), uniform_ptr(kring), uniform_ptr(krsc), u(kbits), u(krot)};
+    const RowGeo G{uniform_ptr(ptab), u(pt_stride), u(page), u(n_pages), u(kvrc)};
+    const bool paged = u((int) (gbase >> 32)) < 0;
+    const void * const in = uniform_ptr(w ? vin : kin);
+    for (int i = u(wv); i < n; i += u(nw)) { // (nw is even: a wave stays on its side)
+        const int p = u(pa) + (i >> 1);
+        float v[4];
+        load_row4(in, in0 + (size_t) (i >> 1) * in_stride, u(f16), v);
+        store_row_at(sd, paged ? main_row(G, u(seq), u(g), p) : (size_t) gbase + p, G.kvrc > 0 ? ring_row(G, u(seq), u(g), p) : 0, true, v);
     }
+}
+// the workgroup's stored rows are in L2 before any of its copies read them (a workgroup's waves share one CU's L1, which
+// writes through)
+__device__ __forceinline__ void append_done() {
+    vm_wait<0>();
+    __syncthreads();
 }
 
 // wave issue priority 0..3 from the tiles a wave has left: the instruction arbiter otherwise favours the older
@@ -965,23 +977,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SMALL ? 3 :
         // the main-store row of position p is then gbase + p)
         auto tile_page = [&](int i) { return sd.pbase >= 0 ? 0 : page_of(paged_geo(), seq, c0 + ATP * (sl + AWAVES * i)); };
         int phys_cur = my > 0 ? tile_page(0) : 0; // page of the tile in the stage (tile i while step i runs)
-        // fused append (APPEND kernels only): a wave whose tiles hold new positions (L - T .. L - 1) stores those rows
-        // before its first copy (a called function waits for every load at entry, so it runs before any copy is issued)
-        bool has_new = false;
-        if (APPEND && a.kin) {
-            const int pa = max(L - T, c0), pb = min(L, c1);
-            for (int p = pa; p < pb; p++) has_new |= ((p - c0) >> 5) % AWAVES == sl;
+        // fused append (APPEND kernels only): a workgroup whose segment holds new positions (pa .. c1 - 1) stores those rows
+        // before its first copies (a called function waits for every load at entry, so it runs before any copy is issued)
+        if constexpr (APPEND) {
+            const int pa = max(L - T, c0);
+            if (a.kin && pa < c1) {
+                append_rows(a.kin, a.vin, a.kin_f16, ((((size_t) si * T + (pa - (L - T))) * a.kin_nl + l) * NKV + g) * HD, a.kin_nl * NKV * HD,
+                            geo.ptab, geo.pt_stride, geo.page, geo.n_pages, geo.kvrc, SK.vals, SK.scs, SK.ring, SK.rsc, SK.bits, SK.rot, SV.vals,
+                            SV.scs, SV.ring, SV.rsc, SV.bits, SV.rot, sd.pbase >= 0 ? (long long) gbase : -1, seq, g, pa, c1, wv, AWAVES);
+                append_done();
+            }
         }
         // ---- queries: FWHT when K is stored rotated, * 1/16, fp16 (qwen38_mk.cu:2873-2880), rows r = hh T + t.  The
         // wave's rows are loaded before its first tile copy and waited for alone (loads return in order: vmcnt at most
         // the copy count), so they are converted while tile 0 streams.  Only the copy issue runs between the loads and
         // the wait (the loaded registers must not be read or moved before it).
-        if constexpr (APPEND)
-            if (has_new) {
-                append_rows(a.kin, a.vin, a.kin_f16, a.kin_nl, geo.ptab, geo.pt_stride, geo.page, geo.n_pages, geo.kvrc, SK.vals, SK.scs, SK.ring,
-                            SK.rsc, SK.bits, SK.rot, SV.vals, SV.scs, SV.ring, SV.rsc, SV.bits, SV.rot, seq, g, l, si, L, T, c0, c1, sl, 0, 1);
-                vm_wait<0>(); // the stored rows are in L2 before this wave's copies read them
-            }
         constexpr int QPW = RP / AWAVES; // rows per wave
         f32x4 qx[QPW];
 #pragma unroll
@@ -1299,14 +1309,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 qx[j] = wv + NW * j < R ? *reinterpret_cast<const f32x4 *>(q_addr(G, j)) : f32x4{0.f, 0.f, 0.f, 0.f};
         } else {
             if constexpr (APPEND) {
-                bool has_new = false;
-                if (a.kin)
-                    for (int p = max(G.L - T, G.c0); p < min(G.L, G.c1); p++) has_new |= ((p - G.c0) >> 5) % AWAVES == sl;
-                if (has_new) {
-                    append_rows(a.kin, a.vin, a.kin_f16, a.kin_nl, S.ptab, S.pt_stride, S.page, S.n_pages, S.kvrc, G.SK.vals, G.SK.scs,
-                                G.SK.ring, G.SK.rsc, G.SK.bits, G.SK.rot, G.SV.vals, G.SV.scs, G.SV.ring, G.SV.rsc, G.SV.bits, G.SV.rot,
-                                G.seq, G.g, G.l, G.si, G.L, T, G.c0, G.c1, sl, hf, hf);
-                    vm_wait<0>(); // the stored rows are in L2 before this wave's copies read them
+                const int pa = max(G.L - T, G.c0);
+                if (a.kin && pa < G.c1) {
+                    append_rows(a.kin, a.vin, a.kin_f16, ((((size_t) G.si * T + (pa - (G.L - T))) * a.kin_nl + G.l) * NKV + G.g) * HD,
+                                a.kin_nl * NKV * HD, S.ptab, S.pt_stride, S.page, S.n_pages, S.kvrc, SK.vals, SK.scs, SK.ring, SK.rsc, SK.bits, SK.rot,
+                                SV.vals, SV.scs, SV.ring, SV.rsc, SV.bits, SV.rot,
+                                G.pbase >= 0 ? (long long) (G.g * S.n_pages + G.pbase) * S.page : -1, G.seq, G.g, pa, G.c1, wv, NW);
+                    append_done();
                 }
             }
             // loaded before the first copy and waited for alone (loads return in order), as in k_attn

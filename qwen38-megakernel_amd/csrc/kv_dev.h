@@ -291,13 +291,6 @@ __device__ __forceinline__ void store_row_at(const SideLayout & sd, size_t row, 
         if ((lane & 7) == 0) st_row(sd.rsc + rr * 8 + (lane >> 3), rs);
     }
 }
-__device__ __forceinline__ void store_row(const RowGeo & S, const SideLayout & sd, int seq, int g, int p, bool ring, float (&v)[4]) {
-    store_row_at(sd, main_row(S, seq, g, p), S.kvrc > 0 ? ring_row(S, seq, g, p) : 0, ring, v);
-}
-
-__device__ __forceinline__ void store_row(const StoreLayout & S, const SideLayout & sd, int seq, int g, int p, bool ring, float (&v)[4]) {
-    store_row(geo_of(S), sd, seq, g, p, ring, v);
-}
 
 // ------------------------------------------------------------------------------------------------ dequantization
 // fp16 operands are built from magic pairs (kv_codes.h): a half such as 0x6400 | n is 1024 + n exactly (n < 1024), so

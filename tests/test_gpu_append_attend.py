@@ -97,3 +97,39 @@ def test_append_attend_errors(qkv, torch_gpu):
     st.append_attend(0, 1, [0], [1001], 1, k.data_ptr(), k.data_ptr(), 0, q.data_ptr(), out.data_ptr())
     torch.cuda.synchronize()
     assert st.digest(0)[1] == 1001
+
+
+@pytest.mark.parametrize("T,wide", [(1, 2), (8, 2), (8, 1)])
+def test_fused_rows_across_pages_and_segments(qkv, torch_gpu, T, wide):
+    # the step's rows spread over a workgroup's waves: a page and a segment boundary inside the T rows of both sequences, a ring
+    # that has wrapped, and another format per side; the pages of sequence 0 contiguous, those of sequence 1 not
+    torch = torch_gpu
+    rng = np.random.default_rng(5 + T)
+    lens, page, ctx, nl = [1155, 2435], 64, 2624, 2  # rows 1147 .. 1154 around 1152 = 18 pages = 9 segments, 2427 .. 2434 around 2432
+    kw = dict(win=640, n_layers=nl, n_seq=2, ctx=ctx, page=page, n_pages=0)
+    a, b = (qkv.KVStore("K0=6r,V0=7,K1=5r,V1=4r", **kw) for _ in range(2))
+    b.config("wide", wide)
+    npg = ctx // page
+    for st in (a, b):
+        st.set_pages(0, np.arange(npg))
+        st.set_pages(1, npg + np.arange(npg)[::-1])
+    keep = []
+    for s, L in enumerate(lens):
+        K0, V0 = synth_kv(rng, L - T, nl, outliers=True)
+        append_all(torch, a, s, K0, V0, chunks=[4096])
+        append_all(torch, b, s, K0, V0, chunks=[4096])
+    K, V = step_inputs(rng, 2, T, nl)
+    q = torch.from_numpy(rng.standard_normal((nl, 2, T, NH, HD)).astype(np.float32)).cuda()
+    out_a, out_b = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
+    for s, L in enumerate(lens):
+        kd, vd = to_dev(torch, K[s], False), to_dev(torch, V[s], False)
+        keep += [kd, vd]
+        a.append(s, 0, nl, L - T, T, kd.data_ptr(), vd.data_ptr(), 0)
+    a.attend(0, nl, [0, 1], lens, T, q.data_ptr(), out_a.data_ptr())
+    kd, vd = to_dev(torch, K, False), to_dev(torch, V, False)
+    b.append_attend(0, nl, [0, 1], lens, T, kd.data_ptr(), vd.data_ptr(), 0, q.data_ptr(), out_b.data_ptr())
+    torch.cuda.synchronize()
+    assert torch.isfinite(out_a).all() and torch.equal(out_a, out_b)
+    assert all(a.digest(s) == b.digest(s) for s in (0, 1))
+    a.close()
+    b.close()
