@@ -195,15 +195,26 @@ struct Store {
     // A buffer that has to grow takes at least 1.5 times its old size, so a context that grows step by step
     // reallocates a logarithmic number of times and the retired buffers together stay below twice the live one.
     std::vector<void *> retired;
-    void grow(void *& p, size_t & have, size_t need) {
-        if (need <= have) return;
-        if (have) need = std::max(need, have + have / 2);
+    hipError_t try_grow(void *& p, size_t & have, size_t need) {
+        if (need <= have) return hipSuccess;
+        size_t want = have ? std::max(need, have + have / 2) : need;
         void * q = nullptr;
-        HCK(hipMalloc(&q, need));
+        hipError_t e = hipMalloc(&q, want);
+        if (e != hipSuccess && want > need) {
+            (void) hipGetLastError();
+            want = need;
+            e = hipMalloc(&q, want);
+        }
+        if (e != hipSuccess) {
+            (void) hipGetLastError(); // (reported here, not by a later call)
+            return e;
+        }
         if (p) retired.push_back(p);
         p = q;
-        have = need;
+        have = want;
+        return hipSuccess;
     }
+    void grow(void *& p, size_t & have, size_t need) { HCK(try_grow(p, have, need)); }
     size_t main_row(int seq, int g, int p) const {
         const int lp = p / page;
         return (size_t) (g * n_pages + ptab[(size_t) seq * pt_stride + lp]) * page + (p - lp * page);
@@ -766,10 +777,15 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
         // the window's tiles a group can see: its pieces' and, before them, the first one's window
         const int q_tiles = s.kvrc > 0 ? (s.kvrc / ATT_BUCKET_ + in_group) * (ATT_BUCKET_ / ATP_) + 2 : 0;
         const size_t unit = (size_t) kv_tiles * KV16_TILE, qunit = (size_t) q_tiles * KV16_TILE, fit = PREFILL_KV16_MAX / (unit + qunit);
-        const bool keep = (size_t) n_layers * NKV <= fit;
-        const int ng = keep ? NKV : fit >= 4 ? 4 : fit >= 2 ? 2 : 1;
-        const size_t units_all = keep ? (size_t) n_layers * NKV : (size_t) ng;
-        s.grow(s.kv16, s.kv16_bytes, units_all * (unit + qunit));
+        bool keep = (size_t) n_layers * NKV <= fit;
+        int ng = keep || fit >= 4 ? NKV : fit >= 2 ? 2 : 1;
+        auto units = [&]() { return keep ? (size_t) n_layers * NKV : (size_t) ng; };
+        while (s.try_grow(s.kv16, s.kv16_bytes, units() * (unit + qunit)) != hipSuccess) { // (a nearly full device: less at a time)
+            if (keep) keep = false;
+            else if (ng > 1) ng /= 2;
+            else throw std::runtime_error("no device memory for the prefill's " + std::to_string(unit + qunit) + " bytes of key tiles");
+        }
+        const size_t units_all = units();
         uint8_t * const kv16 = static_cast<uint8_t *>(s.kv16), * const kq16 = kv16 + units_all * unit;
         PrefillArgs p{};
         p.S = s.S;
@@ -850,9 +866,9 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
             for (int l = 0, e; l < n_layers; l = e) {
                 e = run_end(l, part_rows);
                 set_run(l, e);
-                const size_t units = (size_t) p.nl * p.ng;
-                s.grow(s.part, s.part_bytes, units * part_rows * HD * sizeof(float));
-                s.grow(s.ml, s.ml_bytes, units * part_rows * sizeof(float2));
+                const size_t run_rows = (size_t) p.nl * p.ng * part_rows;
+                s.grow(s.part, s.part_bytes, run_rows * HD * sizeof(float));
+                s.grow(s.ml, s.ml_bytes, run_rows * sizeof(float2));
                 p.part = static_cast<float *>(s.part);
                 p.ml = static_cast<float2 *>(s.ml);
                 const size_t trow = (size_t) l * T + a0; // first token row of the group in this run's block
