@@ -744,9 +744,9 @@ int mk_kv_attend_prep(void * h, int layer0, int n_layers, int n_seq, const int *
                        static_cast<int8_t *>(q32b), q32meta, stream);
 }
 
-// prefill: the chunk pos .. pos+T-1 in pieces ending at 640-bucket boundaries; each piece's K/V rows are stored, then
-// every layer's queries of the piece attend (prefill_host.cu:606-615).  k, v: [T][n_layers][4][256]; q: [n_layers][T][24][qs];
-// out: [n_layers][T][24][256]; gate [n_layers][T][24][gs]; q32 [n_layers][T][192][16 | 4].
+// prefill: the chunk pos .. pos+T-1 in pieces ending at 640-bucket boundaries, each reading the window of its bucket
+// (prefill_host.cu:606-615); the pieces of a group are stored together, then every layer's queries of the group attend.
+// k, v: [T][n_layers][4][256]; q: [n_layers][T][24][qs]; out: [n_layers][T][24][256]; gate [n_layers][T][24][gs]; q32 [n_layers][T][192][16 | 4].
 static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, int T, const void * k, const void * v, int dtype,
                         const float * knw, const float * q, int qs, const float * qnw, const float * gate, int gs, float * out,
                         int8_t * q32a, int8_t * q32b, uint16_t * q32m, void * stream) {
@@ -843,10 +843,10 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
                 return P;
             };
             int last = first;
-            size_t part_rows = (size_t) piece(first).R * piece(first).nseg;
+            auto partials = [](const PrefillPiece & P) { return P.nseg == 1 ? (size_t) 0 : (size_t) P.R * P.nseg; };
+            size_t part_rows = partials(piece(first));
             while (keep && last + 1 - first < in_group && (last + 1) * ATT_BUCKET_ < end) {
-                const PrefillPiece P = piece(last + 1);
-                const size_t more = part_rows + (size_t) P.R * P.nseg;
+                const size_t more = part_rows + partials(piece(last + 1));
                 if (more * NKV * HD * 4 > PREFILL_PART) break;
                 part_rows = more;
                 last++;
@@ -862,14 +862,23 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
             p.q0 = s.kvrc == 0 ? 0 : keep ? n0 / ATP_ : window_start(L, s.win) / ATP_;
             p.q1 = s.kvrc == 0 ? 0 : p.p1;
             p.np = 0;
-            for (int i = last; i >= first; i--) p.pc[p.np++] = piece(i); // the longest contexts first
+            int q_blocks = 0;
+            for (int i = last; i >= first; i--) { // the longest contexts first
+                PrefillPiece & P = p.pc[p.np++];
+                P = piece(i);
+                P.qb0 = q_blocks;
+                q_blocks += (P.R + 31) / 32;
+            }
             for (int l = 0, e; l < n_layers; l = e) {
                 e = run_end(l, part_rows);
                 set_run(l, e);
-                const size_t run_rows = (size_t) p.nl * p.ng * part_rows;
-                s.grow(s.part, s.part_bytes, run_rows * HD * sizeof(float));
+                const unsigned slots = ((1u << p.nl) - 1u) << p.layer;
+                p.q_blocks = p.pc[0].nseg > 1 && (qnw || (p.krot & slots)) ? q_blocks : 0;
+                const size_t run_rows = (size_t) p.nl * p.ng * part_rows, part_need = run_rows * HD * sizeof(float);
+                s.grow(s.part, s.part_bytes, part_need + (size_t) p.nl * p.ng * p.q_blocks * Q16_BLOCK); // (the queries after the partials)
                 s.grow(s.ml, s.ml_bytes, run_rows * sizeof(float2));
                 p.part = static_cast<float *>(s.part);
+                p.q16 = static_cast<uint8_t *>(s.part) + part_need;
                 p.ml = static_cast<float2 *>(s.ml);
                 const size_t trow = (size_t) l * T + a0; // first token row of the group in this run's block
                 p.q = q + trow * NH * qs;

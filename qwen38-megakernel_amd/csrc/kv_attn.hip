@@ -297,7 +297,7 @@ hipError_t launch_combine(const AttnArgs & a, hipStream_t st, hipEvent_t ev0, hi
 // ------------------------------------------------------------------------------------------------ prefill
 // Causal attention of a group of prefill pieces (pk_attn8's exact form, prefill_attn.cuh:698-702; pieces and window
 // prefill_host.cu:606-615), over every layer of a run (equal K / V bits):
-//   k_prefill_kv       keys as fp16 MFMA operands in scratch buffers (PrefillArgs::kv16, kq16), each tile once
+//   k_prefill_kv       keys and queries as fp16 MFMA operands in scratch buffers (PrefillArgs::kv16, kq16, q16), each once
 //   k_prefill_attn     the attention over them: no unpacking in its loop
 //   k_prefill_combine  the segments of each row, the output epilogue
 // A piece has up to 30 row blocks of 128 per kv head, and unpacking the stored rows is as much work as a row block's
@@ -360,6 +360,8 @@ constexpr int PQ_REGION = 5120;   // per wave: K rows 2 KB, V rows 2 KB, scales 
 constexpr int SV_LD = HD + 24;    // V rows of the transposing buffer 560 bytes apart: the 4 rows that one 16-lane group of
                                   // a transposed read addresses start 32 bytes apart in the banks
 constexpr int PKV_LDS = 4 * PQ_REGION + ATP * SV_LD * 2;
+constexpr int SQ_LD = HD + 8;     // query staging rows (halves)
+static_assert(PKV_LDS >= 32 * SQ_LD * 2, "query staging");
 
 // the 8 positions of quarter pw of a tile: one wave's copies (5 instructions) into its region
 template <int KB, int VB>
@@ -399,16 +401,68 @@ __device__ __forceinline__ void pq_dequant(const uint8_t * reg, int pw, int lane
     for (int k = 0; k < 4; k++) vd[k] = make_uint4(as_u(o[4 * k]), as_u(o[4 * k + 1]), as_u(o[4 * k + 2]), as_u(o[4 * k + 3]));
 }
 
-// Tiles p0 .. p1 - 1 (main rows) and q0 .. q1 - 1 (window rows) of every (layer, kv head) of the launch: one workgroup of
-// 4 waves per tile, each wave copying 8 positions HBM -> LDS and unpacking what it copied.  HBM-bound: 4 workgroups per
-// CU (38 KiB of LDS each) keep copies in flight.
+// 32 query rows (block qb of unit u) as fp16 operands: prep, FWHT for rotated K, * 1/16, each wave 8 rows (independent
+// loads, one wait), then into fragments: B of S^T = K Q^T, K step ks, lane l: row l % 32, dims 16 ks + 8 (l / 32) .. + 7
+// (pair order) at q16 + Q16_BLOCK (u q_blocks + qb) + 1024 ks + 16 l.  Once per row, not once per key segment, and in
+// workgroups of their own beside the tiles': in the attention kernel the rows of a workgroup took 13 us before its first
+// tile (24 with the prep), as much as 9 pairs of tiles.  Which rows come here: PrefillArgs::q16.
+__device__ __forceinline__ void prefill_queries(const PrefillArgs & a, int u, int l, int g, int qb, int wv, int lane, _Float16 * sq) {
+    int pi = 0;
+#pragma unroll
+    for (int i = 1; i < PF_PIECES; i++)
+        if (i < a.np && qb >= a.pc[i].qb0) pi = i;
+    const PrefillPiece P = a.pc[pi];
+    const float * const q = a.q + ((size_t) l * a.T + P.t0) * NH * a.qs;
+    const float * const qnw = a.qnw ? a.qnw + (size_t) l * HD : nullptr;
+    const bool krot = (a.krot >> (a.layer + l)) & 1u;
+    const int r0 = 32 * (qb - P.qb0);
+    float4 xs[8];
+#pragma unroll
+    for (int v = 0; v < 8; v++) {
+        const int r = r0 + 8 * wv + v, t = r / GQA, hh = r - GQA * t;
+        xs[v] = r < P.R ? *reinterpret_cast<const float4 *>(q + ((size_t) t * NH + GQA * g + hh) * a.qs + 4 * lane)
+                        : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int v = 0; v < 8; v++) {
+        const int rl = 8 * wv + v, r = r0 + rl;
+        half2v o0 = {(_Float16) 0.f, (_Float16) 0.f}, o1 = o0;
+        if (r < P.R) {
+            const int t = r / GQA;
+            float y[4] = {xs[v].x, xs[v].y, xs[v].z, xs[v].w};
+            if (qnw) qk_prep(y, qnw, a.rope + (size_t) (P.n0 + t) * 32);
+            if (krot) fwht256_w64(y);
+            o0[0] = (_Float16) (y[0] * 0.0625f); // (pair order, as the K fragments)
+            o0[1] = (_Float16) (y[2] * 0.0625f);
+            o1[0] = (_Float16) (y[1] * 0.0625f);
+            o1[1] = (_Float16) (y[3] * 0.0625f);
+        }
+        *reinterpret_cast<uint2 *>(sq + rl * SQ_LD + 4 * lane) = make_uint2(as_u(o0), as_u(o1));
+    }
+    __syncthreads();
+    uint8_t * const dst = a.q16 + ((size_t) u * a.q_blocks + qb) * Q16_BLOCK;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int ks = 4 * wv + k;
+        *reinterpret_cast<uint4 *>(dst + 1024 * ks + 16 * lane) =
+            *reinterpret_cast<const uint4 *>(sq + (lane & 31) * SQ_LD + 16 * ks + 8 * (lane >> 5));
+    }
+}
+
+// Blocks 0 .. q_blocks - 1 of a unit (layer, kv head): its query rows (prefill_queries).  The others: tiles p0 .. p1 - 1
+// (main rows) and q0 .. q1 - 1 (window rows), one workgroup of 4 waves per tile, each wave copying 8 positions HBM -> LDS
+// and unpacking what it copied.  HBM-bound: 4 workgroups per CU (38 KiB of LDS each) keep copies in flight.
 template <int KB, int VB>
 __global__ __launch_bounds__(256) void k_prefill_kv(PrefillArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t smem[PKV_LDS];
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const StoreLayout & S = a.S;
     const int u = blockIdx.y, l = u / a.ng, g = a.g0 + u % a.ng;
-    const int x = blockIdx.x, np = a.p1 - a.p0;
+    if ((int) blockIdx.x < a.q_blocks) {
+        prefill_queries(a, u, l, g, blockIdx.x, wv, lane, reinterpret_cast<_Float16 *>(smem));
+        return;
+    }
+    const int x = blockIdx.x - a.q_blocks, np = a.p1 - a.p0;
     const bool ring = x >= np;
     const int t = ring ? a.q0 + x - np : a.p0 + x;
     const SideLayout SK = S.side[a.layer + l][0], SV = S.side[a.layer + l][1];
@@ -480,10 +534,15 @@ __device__ __forceinline__ void pipeline_pv() {
 // pair.  At the end the two parities' states are merged through LDS, each wave finishing half of its rows' dims.
 // What bounds it: the matrix cores (2,048 cycles per pair of tiles on a SIMD) and the softmax between its two products.
 constexpr int PA_BUF = 2 * KV16_TILE;                     // one pair of tiles
-constexpr int PA_LDS = 2 * PA_BUF + 8 * 32 * 8;           // two pairs, (m, l) of 8 waves x 32 rows
-constexpr int SQ_LD = HD + 8;                             // query staging rows (halves)
+constexpr int SY_LD = HD + 4;                             // output rows (floats) of a single-segment piece
+constexpr int PA_ML = PF2_ROWS * SY_LD * 4;               // (m, l) of 8 waves x 32 rows, after the pairs and the output rows
+constexpr int PA_LDS = PA_ML + 8 * 32 * 8;
+static_assert(PA_ML >= 2 * PA_BUF, "two pairs");
 static_assert(PA_LDS >= PF2_ROWS * SQ_LD * 2, "query staging inside the tile buffers");
 
+// QPRE: the query operands come from q16 (prefill_queries); otherwise the workgroup prepares its own rows (PrefillArgs::q16).
+// A piece of one segment writes its output rows itself (finish_row) instead of partials for the combine.
+template <bool QPRE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_prefill_attn(PrefillArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane & 31, hf = lane >> 5;
@@ -505,7 +564,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         rb = blk / combos;
         cb = blk - rb * combos;
     }
-    const int k = cb % P.nseg, u = cb / P.nseg, gi = u % a.ng, l = u / a.ng, g = a.g0 + gi;
+    const int k = cb % P.nseg, u = cb / P.nseg, l = u / a.ng, g = a.g0 + u % a.ng;
     const int r0 = PF2_ROWS * rb, rlast = min(P.R, r0 + PF2_ROWS) - 1;
     const int pmax = P.n0 + rlast / GQA;
     const int c0 = k * P.seg;
@@ -524,49 +583,60 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const unsigned to = (unsigned) __builtin_amdgcn_readfirstlane(lds0 + (s & 1) * PA_BUF + wv * (PA_BUF / 8));
         dma16s_pieces<8, false>(uniform_ptr(src), 16 * lane, to);
     };
-    // ---- query rows: all 8 waves stage 16 rows each (prep, FWHT for rotated K, * 1/16, fp16), then take fragments;
-    // loaded 8 rows at a time (independent loads, one wait)
-    const float * const q = a.q + ((size_t) l * a.T + P.t0) * NH * a.qs;
-    const float * const qnw = a.qnw ? a.qnw + (size_t) l * HD : nullptr;
-    const bool krot = (a.krot >> (a.layer + l)) & 1u;
-    _Float16 * const sq = reinterpret_cast<_Float16 *>(smem);
-    for (int jb = 0; jb < 16; jb += 8) {
-        float4 xs[8];
-#pragma unroll
-        for (int v = 0; v < 8; v++) {
-            const int r = r0 + 16 * wv + jb + v, t = r / GQA, hh = r - GQA * t;
-            xs[v] = r < P.R ? *reinterpret_cast<const float4 *>(q + ((size_t) t * NH + GQA * g + hh) * a.qs + 4 * lane)
-                            : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-#pragma unroll
-        for (int v = 0; v < 8; v++) {
-            const int rl = 16 * wv + jb + v, r = r0 + rl;
-            half2v o0 = {(_Float16) 0.f, (_Float16) 0.f}, o1 = o0;
-            if (r < P.R) {
-                const int t = r / GQA;
-                const float4 x = xs[v];
-                float y[4] = {x.x, x.y, x.z, x.w};
-                if (qnw) qk_prep(y, qnw, a.rope + (size_t) (P.n0 + t) * 32);
-                if (krot) fwht256_w64(y);
-                o0[0] = (_Float16) (y[0] * 0.0625f); // (pair order, as the K fragments)
-                o0[1] = (_Float16) (y[2] * 0.0625f);
-                o1[0] = (_Float16) (y[1] * 0.0625f);
-                o1[1] = (_Float16) (y[3] * 0.0625f);
-            }
-            *reinterpret_cast<uint2 *>(sq + rl * SQ_LD + 4 * lane) = make_uint2(as_u(o0), as_u(o1));
-        }
-    }
-    __syncthreads();
+    const bool rows = r0 + 32 * wr < P.R; // the wave has rows at all
     half8 qf[16];
+    if constexpr (QPRE) {
+        issue(0);
+        const uint8_t * const qsrc = a.q16 + ((size_t) u * a.q_blocks + P.qb0 + (rows ? r0 / 32 + wr : 0)) * Q16_BLOCK + 16 * lane;
 #pragma unroll
-    for (int ks = 0; ks < 16; ks++) qf[ks] = *reinterpret_cast<const half8 *>(sq + (32 * wr + c) * SQ_LD + 16 * ks + 8 * hf);
-    __syncthreads(); // every wave holds its fragments: the staging area is free
-    issue(0);
+        for (int ks = 0; ks < 16; ks++) qf[ks] = *reinterpret_cast<const half8 *>(qsrc + 1024 * ks);
+        // used here, so that the compiler waits for them here and not in the loop, where its wait would also drain the
+        // copies of the next pair of tiles
+#pragma unroll
+        for (int ks = 0; ks < 16; ks++) asm volatile("" : "+v"(qf[ks]));
+    } else {
+        // all 8 waves stage 16 rows each (prep, FWHT for rotated K, * 1/16, fp16), then take fragments; loaded 8 rows at a
+        // time (independent loads, one wait; all 16 at once: 2-7% slower)
+        const float * const q = a.q + ((size_t) l * a.T + P.t0) * NH * a.qs;
+        const float * const qnw = a.qnw ? a.qnw + (size_t) l * HD : nullptr;
+        const bool krot = (a.krot >> (a.layer + l)) & 1u;
+        _Float16 * const sq = reinterpret_cast<_Float16 *>(smem);
+        for (int jb = 0; jb < 16; jb += 8) {
+            float4 xs[8];
+#pragma unroll
+            for (int v = 0; v < 8; v++) {
+                const int r = r0 + 16 * wv + jb + v, t = r / GQA, hh = r - GQA * t;
+                xs[v] = r < P.R ? *reinterpret_cast<const float4 *>(q + ((size_t) t * NH + GQA * g + hh) * a.qs + 4 * lane)
+                                : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+#pragma unroll
+            for (int v = 0; v < 8; v++) {
+                const int rl = 16 * wv + jb + v, r = r0 + rl;
+                half2v o0 = {(_Float16) 0.f, (_Float16) 0.f}, o1 = o0;
+                if (r < P.R) {
+                    const int t = r / GQA;
+                    const float4 x = xs[v];
+                    float y[4] = {x.x, x.y, x.z, x.w};
+                    if (qnw) qk_prep(y, qnw, a.rope + (size_t) (P.n0 + t) * 32);
+                    if (krot) fwht256_w64(y);
+                    o0[0] = (_Float16) (y[0] * 0.0625f); // (pair order, as the K fragments)
+                    o0[1] = (_Float16) (y[2] * 0.0625f);
+                    o1[0] = (_Float16) (y[1] * 0.0625f);
+                    o1[1] = (_Float16) (y[3] * 0.0625f);
+                }
+                *reinterpret_cast<uint2 *>(sq + rl * SQ_LD + 4 * lane) = make_uint2(as_u(o0), as_u(o1));
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int ks = 0; ks < 16; ks++) qf[ks] = *reinterpret_cast<const half8 *>(sq + (32 * wr + c) * SQ_LD + 16 * ks + 8 * hf);
+        __syncthreads(); // every wave holds its fragments: the staging area is free
+        issue(0);
+    }
     const int row = r0 + 32 * wr + c;
     const int lim = row < P.R ? P.n0 + row / GQA : -1;
     const int lim_min = P.n0 + (r0 + 32 * wr) / GQA;
-    const bool rows = r0 + 32 * wr < P.R; // the wave has rows at all
-    float m = -INFINITY, ls = 0.f;        // running max (log2 units) and sum
+    float m = -INFINITY, ls = 0.f; // running max (log2 units) and sum
     f32x16 O[8];
 #pragma unroll
     for (int db = 0; db < 8; db++)
@@ -639,10 +709,56 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     // ---- the two parities of each row, even tiles first: M = max, O = e0 O0 + e1 O1, l likewise.  Each wave gives the
     // other parity's wave half of its dims (blocks 4 (1 - par) .. + 3) and finishes the other half
-    float2 * const s_ml = reinterpret_cast<float2 *>(smem + 2 * PA_BUF);
-    float4 * const s_o = reinterpret_cast<float4 *>(smem); // [8 waves][16][64]
+    float2 * const s_ml = reinterpret_cast<float2 *>(smem + PA_ML);
     __syncthreads();
     if (hf == 0) s_ml[wv * 32 + c] = make_float2(m, ls);
+    // values 4 j .. + 3 of dim block db: dims 32 db + 8 j + 4 hf .. + 3 (V's dims are in pair order)
+    auto weights = [&](float & M, float & e0, float & e1) {
+        const float2 ml0 = s_ml[wr * 32 + c], ml1 = s_ml[(4 + wr) * 32 + c];
+        M = fmaxf(ml0.x, ml1.x);
+        e0 = ml0.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml0.x - M);
+        e1 = ml1.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml1.x - M);
+        return __builtin_fmaf(e1, ml1.y, e0 * ml0.y);
+    };
+    if (P.nseg == 1) { // the output rows: the odd tiles' sums through LDS, merged there, then whole rows per wave
+        float * const sy = reinterpret_cast<float *>(smem);
+        float * const mine = sy + (32 * wr + c) * SY_LD + 4 * hf;
+        if (par == 1) {
+#pragma unroll
+            for (int db = 0; db < 8; db++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    *reinterpret_cast<float4 *>(mine + 32 * db + 8 * j) =
+                        make_float4(O[db][4 * j], O[db][4 * j + 2], O[db][4 * j + 1], O[db][4 * j + 3]);
+        }
+        __syncthreads();
+        if (par == 0) {
+            float M, e0, e1;
+            const float den = weights(M, e0, e1);
+#pragma unroll
+            for (int db = 0; db < 8; db++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    float4 * const at = reinterpret_cast<float4 *>(mine + 32 * db + 8 * j);
+                    const float4 z = *at;
+                    *at = make_float4(__builtin_fmaf(e1, z.x, e0 * O[db][4 * j]), __builtin_fmaf(e1, z.y, e0 * O[db][4 * j + 2]),
+                                      __builtin_fmaf(e1, z.z, e0 * O[db][4 * j + 1]), __builtin_fmaf(e1, z.w, e0 * O[db][4 * j + 3]));
+                }
+            if (hf == 0) s_ml[wv * 32 + c].y = den; // (only this lane pair reads its row's entries above)
+        }
+        __syncthreads();
+        for (int rl = wv; rl < min(PF2_ROWS, P.R - r0); rl += 8) {
+            const float4 x = *reinterpret_cast<const float4 *>(sy + rl * SY_LD + 4 * lane);
+            const float den = s_ml[rl].y;
+            float v[4] = {x.x / den, x.y / den, x.z / den, x.w / den};
+            const int r = r0 + rl, t = r / GQA, h = GQA * g + r - GQA * t;
+            const size_t trow = (size_t) l * a.T + P.t0 + t;
+            finish_row(v, (a.vrot >> (a.layer + l)) & 1u, a.gate ? a.gate + (trow * NH + h) * a.gs : nullptr, a.out + (trow * NH + h) * HD, a.q32a,
+                       a.q32b, a.q32m, trow, h);
+        }
+        return;
+    }
+    float4 * const s_o = reinterpret_cast<float4 *>(smem); // [8 waves][16][64]
 #pragma unroll
     for (int d = 0; d < 4; d++)
 #pragma unroll
@@ -656,12 +772,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
     __syncthreads();
     if (row < P.R) {
-        const float2 ml0 = s_ml[wr * 32 + c], ml1 = s_ml[(4 + wr) * 32 + c];
-        const float M = fmaxf(ml0.x, ml1.x);
-        const float e0 = ml0.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml0.x - M);
-        const float e1 = ml1.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml1.x - M);
+        float M, e0, e1;
+        const float den = weights(M, e0, e1);
         const size_t at = (size_t) P.part0 + ((size_t) u * P.nseg + k) * P.R + row;
-        if (hf == 0 && par == 0) a.ml[at] = make_float2(M, __builtin_fmaf(e1, ml1.y, e0 * ml0.y));
+        if (hf == 0 && par == 0) a.ml[at] = make_float2(M, den);
         float * const dst = a.part + at * HD;
         const float4 * const o = s_o + ((wv ^ 4) * 16) * 64 + lane;
 #pragma unroll
@@ -676,12 +790,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                     const float own = par ? O[4 + d][4 * j + i] : O[d][4 * j + i];
                     y[i] = par ? __builtin_fmaf(e1, own, e0 * zi[i]) : __builtin_fmaf(e1, zi[i], e0 * own);
                 }
-                store_part(dst + 32 * (4 * par + d) + 8 * j + 4 * hf, make_float4(y[0], y[2], y[1], y[3])); // (V's dims are in pair order)
+                store_part(dst + 32 * (4 * par + d) + 8 * j + 4 * hf, make_float4(y[0], y[2], y[1], y[3]));
             }
     }
 }
 
-// One wave per (layer, kv head, row) of the group: the row's segments 0 .. pos / seg folded in segment order
+// One wave per (layer, kv head, row) of the group's pieces of several segments: the row's segments 0 .. pos / seg folded in segment order
 // (M' = max(M, m_k), O' = O e^(M - M') + O_k e^(m_k - M'), l likewise; eight at most, pf_seg), y = O / l, then the output
 // epilogue.
 __global__ __launch_bounds__(256) void k_prefill_combine(PrefillArgs a) {
@@ -692,7 +806,7 @@ __global__ __launch_bounds__(256) void k_prefill_combine(PrefillArgs a) {
         if (i < a.np && wid >= a.pc[i].row0) pi = i;
     const PrefillPiece P = a.pc[pi];
     const int w = wid - P.row0;
-    if (w >= P.R * a.nl * a.ng) return;
+    if (P.nseg == 1 || w >= P.R * a.nl * a.ng) return;
     const int r = w % P.R, u = w / P.R, g = a.g0 + u % a.ng, l = u / a.ng;
     const int t = r / GQA, hh = r - GQA * t, pos = P.n0 + t;
     const int nk = pos / P.seg + 1;
@@ -849,16 +963,18 @@ static PrefillKernel pick_prefill_kv(int kb, int vb) {
 hipError_t launch_prefill_kv(const PrefillArgs & a, int kb, int vb, hipStream_t st) {
     PrefillKernel kv = pick_prefill_kv(kb, vb);
     if (!kv) return hipErrorInvalidValue;
-    const int tiles = a.p1 - a.p0 + a.q1 - a.q0;
-    if (tiles > 0) hipLaunchKernelGGL(kv, dim3(tiles, a.nl * a.ng), dim3(256), 0, st, a);
+    const int blocks = a.q_blocks + a.p1 - a.p0 + a.q1 - a.q0;
+    if (blocks > 0) hipLaunchKernelGGL(kv, dim3(blocks, a.nl * a.ng), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
 hipError_t launch_prefill(PrefillArgs & a, hipStream_t st) {
     static thread_local bool configured = false;
     if (!configured) {
-        const hipError_t e = hipFuncSetAttribute((const void *) k_prefill_attn, hipFuncAttributeMaxDynamicSharedMemorySize, PA_LDS);
-        if (e != hipSuccess) return e;
+        for (PrefillKernel f : {k_prefill_attn<false>, k_prefill_attn<true>}) {
+            const hipError_t e = hipFuncSetAttribute((const void *) f, hipFuncAttributeMaxDynamicSharedMemorySize, PA_LDS);
+            if (e != hipSuccess) return e;
+        }
         configured = true;
     }
     const int units = a.nl * a.ng;
@@ -869,12 +985,13 @@ hipError_t launch_prefill(PrefillArgs & a, hipStream_t st) {
         P.row0 = rows;
         P.part0 = part;
         blocks += (P.R + PF2_ROWS - 1) / PF2_ROWS * units * P.nseg;
+        if (P.nseg == 1) continue; // (the attention writes its output)
         rows += P.R * units;
         part += P.R * units * P.nseg;
     }
-    hipLaunchKernelGGL(k_prefill_attn, dim3(blocks), dim3(512), PA_LDS, st, a);
+    hipLaunchKernelGGL(a.q_blocks ? k_prefill_attn<true> : k_prefill_attn<false>, dim3(blocks), dim3(512), PA_LDS, st, a);
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess || rows == 0) return e;
     hipLaunchKernelGGL(k_prefill_combine, dim3((rows + 3) / 4), dim3(256), 0, st, a);
     return hipGetLastError();
 }

@@ -129,6 +129,7 @@ struct PrefillPiece {
     int t0;         // the piece's first token within the group
     int blk0, row0; // first workgroup of the attention, first row of the combine
     int part0;      // first row of part / ml, in rows
+    int qb0;        // first 32-row block of q16
 };
 constexpr int PF_PIECES = 4; // pieces per launch at most
 // a group of consecutive prefill pieces over a run of layers with the same K / V bits: query rows r = 6 t + hh (token t of a
@@ -144,6 +145,13 @@ struct PrefillArgs {
     int p0, p1, q0, q1; // tiles that k_prefill_kv writes: p0 .. p1 - 1 from the main rows, q0 .. q1 - 1 from the window's
     int kv_tiles, q_tiles; // tiles per unit of kv16 (main rows) and kq16 (window rows, tile t at t % q_tiles)
     unsigned krot, vrot; // per-slot bit masks: K / V stored rotated
+    // 32-row blocks of the group's pieces per unit, and [nl ng][q_blocks][Q16_BLOCK] fp16 operands (kv_attn.hip) of the query
+    // rows, for groups with several segments per row whose queries get the prep or the FWHT: done once per row beside the
+    // tiles' conversion, not by every segment's workgroup (16,384 positions, rotated K: 3,838 -> 3,780 us; a prepped
+    // 433-token chunk at 60,188 over two layers 1,524 -> 1,455).  0 otherwise: the extra pass over the queries then costs
+    // more than it saves (a 1,111-token prompt without either over four layers 285 -> 300)
+    int q_blocks;
+    uint8_t * q16;
     const float * q;   // [nl][T][NH][qs] from the group's first token
     int qs;
     const float * qnw; // optional q-norm weights [nl][HD] (the Q prep, table rope)
@@ -160,16 +168,19 @@ struct PrefillArgs {
     float2 * ml;       // per piece [nl ng][nseg][R] (max in log2 units, sum)
 };
 constexpr int KV16_TILE = 2 * ATP * HD * 2; // one tile's K and V as fp16
-// key positions per prefill segment: 2, 4 or 8 segments over the row's 640-bucket end, in multiples of 128 -- the same for
+constexpr int Q16_BLOCK = 32 * HD * 2;      // 32 query rows as fp16
+// key positions per prefill segment: 1, 2, 4 or 8 segments over the row's 640-bucket end, in multiples of 128 -- the same for
 // every row of a bucket (every row's result is a function of its position).  A workgroup is (128 query rows, kv head,
 // segment): a full 640-position piece has 240 of them with two segments, one round on 256 CUs, and more segments repeat
-// each workgroup's query staging and partial stores.  Short chunks far into a context have few row blocks, so more
+// each workgroup's partial stores.  Short chunks far into a context have few row blocks, so more
 // segments pay there (60,000 positions, 2 / 4 / 8 segments: 16 tokens 731 / 412 / 252 us, 256 tokens 706 / 474 / 506, 512
 // tokens 830 / 862 / 811, 640 tokens 946 / 962 / 1,003), and up to 20,480 positions whole prompts decide (16,384 with
-// four segments: 9% slower).
+// four segments: 9% slower).  Rows of one segment need neither partials nor the combine, which were over half of a short
+// prompt's time: up to 1,280 positions one segment (two / one: 1,111 tokens over four layers 296 / 128 us, over one 80 / 53,
+// 640 tokens 44 / 38, 640 after 640 60 / 54; 128 after 1,072 38 / 47, whose one workgroup per row block walks all keys).
 inline int pf_seg(int L) {
     const int lb = (L + ATT_BUCKET - 1) / ATT_BUCKET * ATT_BUCKET;
-    const int n = lb > 64 * ATT_BUCKET ? 8 : lb > 32 * ATT_BUCKET ? 4 : 2;
+    const int n = lb > 64 * ATT_BUCKET ? 8 : lb > 32 * ATT_BUCKET ? 4 : lb > 2 * ATT_BUCKET ? 2 : 1;
     return 128 * ((lb + 128 * n - 1) / (128 * n));
 }
 constexpr int PF2_ROWS = 128; // query rows per prefill workgroup (32 per wave)
@@ -200,7 +211,7 @@ hipError_t launch_attn(const AttnArgs & a, int kb, int vb, int max_blocks, int o
 // the first `tiles` tiles of every wave slice of the attention launch `a` read into the L2 its workgroups will use
 hipError_t launch_prefetch(const AttnArgs & a, int kb, int vb, int tiles, hipStream_t st);
 hipError_t launch_combine(const AttnArgs & a, hipStream_t st, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
-// the tiles p0 .. and q0 .. as fp16 operands
+// the tiles p0 .. and q0 .., and the pieces' query rows, as fp16 operands
 hipError_t launch_prefill_kv(const PrefillArgs & a, int kb, int vb, hipStream_t st);
 // the group's attention and combine (fills blk0 and row0)
 hipError_t launch_prefill(PrefillArgs & a, hipStream_t st);

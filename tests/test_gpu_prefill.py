@@ -273,3 +273,52 @@ def test_prefill_more_layers_than_the_scratch_holds(qkv, torch_gpu):
         torch.cuda.synchronize()
         assert torch.equal(ol, o[l]), l
     st.close()
+
+
+@pytest.mark.parametrize("P,cut", [(1280, 1279), (1281, 5), (650, 640), (1, 0)])
+def test_prefill_rows_written_without_the_merge(qkv, oracle, torch_gpu, P, cut):
+    # pieces of one key segment (up to 1,280 positions) write their output rows in the attention kernel, later ones through
+    # partials: the bucket's last row and the next one's first, one row alone, rotated and plain V, gate and units.  Every
+    # chunking the same bits; the last row against the decode step's, each side within 1e-3 of the exact attention
+    torch = torch_gpu
+    rng = np.random.default_rng(P)
+    nl, spec = 2, "K0=5r,V0=6r,K1=6,V1=5"
+    K, V = synth_kv(rng, P, nl, outliers=False)
+    k, v = torch.from_numpy(K).cuda(), torch.from_numpy(V).cuda()
+    qg = torch.from_numpy(rng.standard_normal((nl, P, NH, 2 * HD)).astype(np.float32)).cuda()
+    kn, qn = (torch.from_numpy((1 + 0.1 * rng.standard_normal((nl, HD))).astype(np.float32)).cuda() for _ in range(2))
+
+    def run(chunks):
+        st = qkv.KVStore(spec, win=640, n_layers=nl, ctx=1400)
+        outs, xas, p = [], [], 0
+        for c in chunks:
+            if not c:
+                continue
+            kc, vc, qc = k[p:p + c].contiguous(), v[p:p + c].contiguous(), qg[:, p:p + c].contiguous()
+            o = torch.full((nl, c, NH, HD), float("nan"), device="cuda")
+            xa = torch.zeros((nl, c, 192, 16), dtype=torch.int8, device="cuda")
+            xb, meta = torch.zeros_like(xa), torch.zeros((nl, c, 192, 4), dtype=torch.int16, device="cuda")
+            st.prefill_prep(0, 0, nl, p, c, kc.data_ptr(), vc.data_ptr(), kn.data_ptr(), qc.data_ptr(), qn.data_ptr(), o.data_ptr(),
+                            xa.data_ptr(), xb.data_ptr(), meta.data_ptr())
+            torch.cuda.synchronize()
+            outs.append(o)
+            xas.append(torch.cat([xa.flatten(2).int(), xb.flatten(2).int(), meta.flatten(2).int()], dim=2))
+            p += c
+        return st, torch.cat(outs, 1), torch.cat(xas, 1)
+
+    st, one, units = run([P])
+    st2, two, units2 = run([cut, P - cut])
+    assert torch.isfinite(one).all() and torch.equal(one, two) and torch.equal(units, units2)
+    for l in range(nl):
+        for t in (0, P // 2, P - 1):
+            ea, eb, em = oracle.q32_row(one[l, t].cpu().numpy())
+            got = units[l, t].cpu().numpy()
+            assert np.array_equal(got[:3072], ea.reshape(-1)) and np.array_equal(got[3072:6144], eb.reshape(-1))
+            assert np.array_equal(got[6144:].astype(np.int16).view(np.uint16), em.reshape(-1))
+    dec = torch.empty((nl, 1, 1, NH, HD), device="cuda")
+    last = qg[:, P - 1:].contiguous()
+    st.attend_prep(0, nl, [0], [P], 1, last.data_ptr(), qn.data_ptr(), dec.data_ptr())
+    torch.cuda.synchronize()
+    assert rel_err(one[:, P - 1].cpu().numpy(), dec[:, 0, 0].cpu().numpy()) <= 2e-3
+    st.close()
+    st2.close()
