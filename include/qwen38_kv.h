@@ -12,7 +12,9 @@
  * workspace grows on demand (by at least 1.5 times); a buffer it outgrows is kept, not freed, until mk_free, so a HIP
  * graph captured over an earlier call stays valid after a larger call (its replays keep using the old, smaller
  * buffer; a graph replay and an eager call of one handle must still not overlap).  The kept buffers together stay
- * below twice the live workspace.
+ * below twice the live workspace.  The prefill calls also keep their keys as fp16 tiles in it: 1,024 bytes per position,
+ * kv head and layer (plus the window's), at most 640 MiB asked for at a time; a call that needs more runs its layers, and
+ * past that its kv heads, one after another.
  *
  * Shapes: NKV = 4 kv heads, NH = 24 query heads (GQA 6), head dim 256, up to 17 attention slots (layers), up to 8
  * query tokens per attend call, up to 8 sequences per attend call.
@@ -151,8 +153,9 @@ int mk_kv_attend_prep(void * h, int layer0, int n_layers, int n_seq, const int *
  * Prefill of positions pos .. pos+T-1 of sequence seq (pos = the stored length, no gap) for slots layer0 ..
  * layer0+n_layers-1: stores the K/V rows (k, v [T][n_layers][4][256], dtype as mk_kv_append) and computes the causal
  * attention of the chunk's queries (q [n_layers][T][24][256], after RMSNorm/RoPE) over the store, out of the same
- * shape.  The chunk runs in pieces ending at 640-position bucket boundaries, each piece stored and then attended, so
- * its rows read the window of their bucket from the ring (MK_EXACT prefill, prefill_host.cu:606-615).  Each output
+ * shape.  The chunk runs in pieces ending at 640-position bucket boundaries, whose rows read the window of their bucket as
+ * the ring holds it when the piece is stored (MK_EXACT prefill, prefill_host.cu:606-615); up to four pieces, no more than
+ * the ring holds, are stored and attended together.  Each output
  * is a function of its position and the stored rows only: the result does not depend on how a prompt is split into
  * chunks (pk_attn8's exact form, prefill_attn.cuh:698-702).  Replaces pk_attn_prep's kv_store + attn (pk_attn8 /
  * pk_attn9 + combine) of mk_prefill.  Asynchronous on `stream`.
