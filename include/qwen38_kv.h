@@ -13,8 +13,10 @@
  * graph captured over an earlier call stays valid after a larger call (its replays keep using the old, smaller
  * buffer; a graph replay and an eager call of one handle must still not overlap).  The kept buffers together stay
  * below twice the live workspace.  The prefill calls also keep their keys as fp16 tiles in it: 1,024 bytes per position,
- * kv head and layer (plus the window's), at most 640 MiB asked for at a time; a call that needs more runs its layers, and
- * past that its kv heads, one after another.
+ * kv head and layer (plus the window's), at most 640 MiB asked for at a time; a call that needs more, or more than the
+ * device has, runs its layers, and past that its kv heads, one after another.  It holds its whole workspace before it
+ * stores anything: one that cannot have the least of it (one kv head's tiles, and the partials of 640 tokens of one kv
+ * head: 30 MiB past 40,960 positions) is refused and changes nothing.
  *
  * Shapes: NKV = 4 kv heads, NH = 24 query heads (GQA 6), head dim 256, up to 17 attention slots (layers), up to 8
  * query tokens per attend call, up to 8 sequences per attend call.
@@ -213,8 +215,9 @@ int mk_kv_ring_restore(void * h, int seq, int pos, const void * src, long long b
  * workgroups per CU for one-token calls on packed formats of at most 11 bits per K + V value: 0 (default) = three
  * when a launch has more work items than two per CU hold, else two; 2 or 3 = always that; "wide" (T >= 5): 1 = one
  * pass over K/V with 8-wave workgroups holding all 48 rows, 0 = two passes of 24 rows (the second pass's tiles found in
- * the same XCD's L2), 2 (default) = the faster of the two as measured, the two passes, on every format.  Results never
- * depend on any of them. */
+ * the same XCD's L2), 2 (default) = the faster of the two as measured, the two passes, on every format;
+ * "prefill_scratch" bounds the workspace bytes that a prefill call asks for (0, the default: by what the device has).
+ * Results never depend on any of them. */
 int mk_kv_config(void * h, const char * key, long long value);
 
 /* Kernel timing with HIP events on the launch stream (the reference's MK_PROFILE per-phase means, engine.cu:382-506).

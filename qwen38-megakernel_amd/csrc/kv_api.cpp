@@ -149,6 +149,7 @@ struct Store {
     // prefill: the keys of one or more (layer, kv head) units as fp16 tiles (grown on demand, PREFILL_KV16_MAX)
     void * kv16 = nullptr;
     size_t kv16_bytes = 0;
+    size_t prefill_scratch = 0; // most bytes of workspace that a prefill may ask for (0: what the device has)
     int max_blocks = 0;
     int occupancy = 0; // decode workgroups per CU: 0 = by launch size, 2 or 3 (launch_attn)
     // 25..48 query rows per kv head: one pass of 8-wave workgroups (1), two batches of 24 rows (0), or by format (2):
@@ -195,26 +196,42 @@ struct Store {
     // A buffer that has to grow takes at least 1.5 times its old size, so a context that grows step by step
     // reallocates a logarithmic number of times and the retired buffers together stay below twice the live one.
     std::vector<void *> retired;
-    hipError_t try_grow(void *& p, size_t & have, size_t need) {
-        if (need <= have) return hipSuccess;
-        size_t want = have ? std::max(need, have + have / 2) : need;
-        void * q = nullptr;
-        hipError_t e = hipMalloc(&q, want);
-        if (e != hipSuccess && want > need) {
-            (void) hipGetLastError();
-            want = need;
-            e = hipMalloc(&q, want);
-        }
-        if (e != hipSuccess) {
+    struct Want {
+        void ** p;
+        size_t * have;
+        size_t need;
+    };
+    // every buffer of w at least as large as needed, or none of them touched: a buffer allocated before another one's
+    // allocation failed is given back (no work knows it yet)
+    template <size_t N> hipError_t try_hold(const Want (&w)[N]) {
+        retired.reserve(retired.size() + N);
+        hipError_t e = hipSuccess;
+        for (const bool ahead : {true, false}) { // (a nearly full device: no more than needed)
+            void * q[N] = {};
+            size_t got[N] = {};
+            e = hipSuccess;
+            for (size_t i = 0; i < N && e == hipSuccess; i++) {
+                if (w[i].need <= *w[i].have) continue;
+                got[i] = ahead ? std::max(w[i].need, *w[i].have + *w[i].have / 2) : w[i].need;
+                e = hipMalloc(&q[i], got[i]);
+            }
+            if (e == hipSuccess) {
+                for (size_t i = 0; i < N; i++) {
+                    if (!q[i]) continue;
+                    if (*w[i].p) retired.push_back(*w[i].p);
+                    *w[i].p = q[i];
+                    *w[i].have = got[i];
+                }
+                return e;
+            }
             (void) hipGetLastError(); // (reported here, not by a later call)
-            return e;
+            for (void * x : q)
+                if (x) (void) hipFree(x);
+            if (e != hipErrorOutOfMemory) break;
         }
-        if (p) retired.push_back(p);
-        p = q;
-        have = want;
-        return hipSuccess;
+        return e;
     }
-    void grow(void *& p, size_t & have, size_t need) { HCK(try_grow(p, have, need)); }
+    void grow(void *& p, size_t & have, size_t need) { HCK(try_hold<1>({{&p, &have, need}})); }
     size_t main_row(int seq, int g, int p) const {
         const int lp = p / page;
         return (size_t) (g * n_pages + ptab[(size_t) seq * pt_stride + lp]) * page + (p - lp * page);
@@ -744,6 +761,15 @@ int mk_kv_attend_prep(void * h, int layer0, int n_layers, int n_seq, const int *
                        static_cast<int8_t *>(q32b), q32meta, stream);
 }
 
+// how a prefill call is cut into launches
+struct PrefillShape {
+    bool keep;       // the tiles of every (layer, kv head) kept through the call; else one piece of ng kv heads of a layer at a time
+    int ng;          // kv heads per launch
+    int group;       // pieces per launch at most
+    size_t part_max; // bytes of partials of a launch over several layers or pieces at most
+    bool q_once;     // query operands prepared once per row where that pays (PrefillArgs::q16)
+};
+
 // prefill: the chunk pos .. pos+T-1 in pieces ending at 640-bucket boundaries, each reading the window of its bucket
 // (prefill_host.cu:606-615); the pieces of a group are stored together, then every layer's queries of the group attend.
 // k, v: [T][n_layers][4][256]; q: [n_layers][T][24][qs]; out: [n_layers][T][24][256]; gate [n_layers][T][24][gs]; q32 [n_layers][T][192][16 | 4].
@@ -777,21 +803,10 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
         // the window's tiles a group can see: its pieces' and, before them, the first one's window
         const int q_tiles = s.kvrc > 0 ? (s.kvrc / ATT_BUCKET_ + in_group) * (ATT_BUCKET_ / ATP_) + 2 : 0;
         const size_t unit = (size_t) kv_tiles * KV16_TILE, qunit = (size_t) q_tiles * KV16_TILE, fit = PREFILL_KV16_MAX / (unit + qunit);
-        bool keep = (size_t) n_layers * NKV <= fit;
-        int ng = keep || fit >= 4 ? NKV : fit >= 2 ? 2 : 1;
-        auto units = [&]() { return keep ? (size_t) n_layers * NKV : (size_t) ng; };
-        while (s.try_grow(s.kv16, s.kv16_bytes, units() * (unit + qunit)) != hipSuccess) { // (a nearly full device: less at a time)
-            if (keep) keep = false;
-            else if (ng > 1) ng /= 2;
-            else throw std::runtime_error("no device memory for the prefill's " + std::to_string(unit + qunit) + " bytes of key tiles");
-        }
-        const size_t units_all = units();
-        uint8_t * const kv16 = static_cast<uint8_t *>(s.kv16), * const kq16 = kv16 + units_all * unit;
         PrefillArgs p{};
         p.S = s.S;
         p.seq = seq;
         p.T = T;
-        p.ng = ng;
         p.kv_tiles = kv_tiles;
         p.q_tiles = q_tiles;
         p.qs = qs;
@@ -801,85 +816,131 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
             p.krot |= (unsigned) s.spec.kr[l] << l;
             p.vrot |= (unsigned) s.spec.vr[l] << l;
         }
+        PrefillShape sh{};
         // consecutive layers with the same K/V bits share their launches, while their tiles fit the L2s and their partials
         // the workspace (rows: partial rows per layer and kv head of a group)
         auto run_end = [&](int l, size_t rows) {
             const SideLayout * a = s.S.side[layer0 + l];
             int e = l + 1;
-            while (keep && e < n_layers && (size_t) (e + 1 - l) * NKV * unit <= PREFILL_L2 && (size_t) (e + 1 - l) * NKV * rows * HD * 4 <= PREFILL_PART &&
-                   s.S.side[layer0 + e][0].bits == a[0].bits && s.S.side[layer0 + e][1].bits == a[1].bits)
+            while (sh.keep && e < n_layers && (size_t) (e + 1 - l) * NKV * unit <= PREFILL_L2 &&
+                   (size_t) (e + 1 - l) * NKV * rows * HD * 4 <= sh.part_max && s.S.side[layer0 + e][0].bits == a[0].bits &&
+                   s.S.side[layer0 + e][1].bits == a[1].bits)
                 e++;
             return e;
         };
-        auto set_run = [&](int l, int e) {
-            p.layer = layer0 + l;
-            p.nl = e - l;
-            p.kv16 = kv16 + (keep ? (size_t) l * NKV * unit : 0);
-            p.kq16 = kq16 + (keep ? (size_t) l * NKV * qunit : 0);
+        // the call in the shape sh: group(a0, b) for the tokens a0 .. b - 1 of each group of pieces, then run(l, e, a0, n) for
+        // the layers l .. e - 1 of each of its launches, with p's pieces and query blocks set and n partial rows in all
+        auto walk = [&](auto && group, auto && run) {
+            for (int a0 = 0; a0 < T;) {
+                const int n0 = pos + a0, first = n0 / ATT_BUCKET_;
+                auto piece = [&](int i) {
+                    PrefillPiece P{};
+                    P.n0 = std::max(n0, i * ATT_BUCKET_);
+                    const int L = std::min(end, (i + 1) * ATT_BUCKET_);
+                    P.R = GQA * (L - P.n0);
+                    P.ws = s.kvrc > 0 ? window_start(L, s.win) : INT32_MAX;
+                    P.seg = pf_seg(L);
+                    P.nseg = (L + P.seg - 1) / P.seg;
+                    P.t0 = P.n0 - n0;
+                    return P;
+                };
+                int last = first;
+                auto partials = [](const PrefillPiece & P) { return P.nseg == 1 ? (size_t) 0 : (size_t) P.R * P.nseg; };
+                size_t part_rows = partials(piece(first));
+                while (last + 1 - first < sh.group && (last + 1) * ATT_BUCKET_ < end) {
+                    const size_t more = part_rows + partials(piece(last + 1));
+                    if (more * NKV * HD * 4 > sh.part_max) break;
+                    part_rows = more;
+                    last++;
+                }
+                const int L = std::min(end, (last + 1) * ATT_BUCKET_), b = L - pos;
+                p.np = 0;
+                int q_blocks = 0;
+                for (int i = last; i >= first; i--) { // the longest contexts first
+                    PrefillPiece & P = p.pc[p.np++];
+                    P = piece(i);
+                    P.qb0 = q_blocks;
+                    q_blocks += (P.R + 31) / 32;
+                }
+                group(a0, b);
+                for (int l = 0, e; l < n_layers; l = e) {
+                    e = run_end(l, part_rows);
+                    p.layer = layer0 + l;
+                    p.nl = e - l;
+                    const unsigned slots = ((1u << p.nl) - 1u) << p.layer;
+                    p.q_blocks = sh.q_once && p.pc[0].nseg > 1 && (qnw || (p.krot & slots)) ? q_blocks : 0;
+                    run(l, e, a0, (size_t) p.nl * sh.ng * part_rows);
+                }
+                a0 = b;
+            }
+        };
+        // The whole workspace is held before anything is stored: a call that cannot have it changes nothing.  What does not
+        // fit the device (or the scratch knob) is tried in the next smaller shape: one piece and one layer per launch, then
+        // one layer's tiles at a time, then fewer kv heads' -- the same bits in all.
+        size_t part_need = 0, ml_need = 0;
+        auto units = [&]() { return sh.keep ? (size_t) n_layers * NKV : (size_t) sh.ng; };
+        bool held = false;
+        for (int step = 0; !held; step++) {
+            const bool all = (size_t) n_layers * NKV <= fit;
+            const int ng = fit >= 4 ? NKV : fit >= 2 ? 2 : 1; // (kv heads whose tiles stay within PREFILL_KV16_MAX)
+            if (step == 0) sh = all ? PrefillShape{true, NKV, in_group, PREFILL_PART, true} : PrefillShape{false, ng, 1, 0, true};
+            else if (step == 1) sh = PrefillShape{all, all ? NKV : ng, 1, 0, false};
+            else if (sh.keep) sh.keep = false;
+            else if (sh.ng > 1) sh.ng /= 2;
+            else
+                throw std::runtime_error("no device memory for the prefill's workspace of " + std::to_string(units() * (unit + qunit) + part_need + ml_need) +
+                                         " bytes");
+            part_need = ml_need = 0;
+            walk([](int, int) {},
+                 [&](int, int, int, size_t n) {
+                     part_need = std::max(part_need, n * HD * sizeof(float) + (size_t) p.nl * sh.ng * p.q_blocks * Q16_BLOCK);
+                     ml_need = std::max(ml_need, n * sizeof(float2));
+                 });
+            const size_t kv16_need = units() * (unit + qunit);
+            if (s.prefill_scratch && kv16_need + part_need + ml_need > s.prefill_scratch) continue;
+            const hipError_t e = s.try_hold<3>(
+                {{&s.kv16, &s.kv16_bytes, kv16_need}, {&s.part, &s.part_bytes, part_need}, {&s.ml, &s.ml_bytes, ml_need}});
+            held = e == hipSuccess;
+            if (!held && e != hipErrorOutOfMemory) throw HipError(std::string("prefill workspace: ") + hipGetErrorString(e));
+        }
+        uint8_t * const kv16 = static_cast<uint8_t *>(s.kv16), * const kq16 = kv16 + units() * unit;
+        p.ng = sh.ng;
+        p.part = static_cast<float *>(s.part);
+        p.ml = static_cast<float2 *>(s.ml);
+        auto set_tiles = [&](int l) {
+            p.kv16 = kv16 + (sh.keep ? (size_t) l * NKV * unit : 0);
+            p.kq16 = kq16 + (sh.keep ? (size_t) l * NKV * qunit : 0);
         };
         auto bits = [&](int l, int w) { return s.S.side[layer0 + l][w].bits; };
-        if (keep && pos > 0 && s.kvrc > 0) { // the window's rows before the call, before its own replace them in the ring
+        if (sh.keep && pos > 0 && s.kvrc > 0) { // the window's rows before the call, before its own replace them in the ring
             p.L = pos;
             p.q0 = window_start(pos + 1, s.win) / ATP_;
             p.q1 = (pos + ATP_ - 1) / ATP_;
+            p.q_blocks = 0;
             for (int l = 0, e; l < n_layers; l = e) {
                 e = run_end(l, 0);
-                set_run(l, e);
+                p.layer = layer0 + l;
+                p.nl = e - l;
+                set_tiles(l);
                 HCK(launch_prefill_kv(p, bits(l, 0), bits(l, 1), st));
             }
         }
-        for (int a0 = 0; a0 < T;) {
-            // the group: tokens a0 .. b - 1, pieces first .. last
-            const int n0 = pos + a0, first = n0 / ATT_BUCKET_;
-            auto piece = [&](int i) {
-                PrefillPiece P{};
-                P.n0 = std::max(n0, i * ATT_BUCKET_);
-                const int L = std::min(end, (i + 1) * ATT_BUCKET_);
-                P.R = GQA * (L - P.n0);
-                P.ws = s.kvrc > 0 ? window_start(L, s.win) : INT32_MAX;
-                P.seg = pf_seg(L);
-                P.nseg = (L + P.seg - 1) / P.seg;
-                P.t0 = P.n0 - n0;
-                return P;
-            };
-            int last = first;
-            auto partials = [](const PrefillPiece & P) { return P.nseg == 1 ? (size_t) 0 : (size_t) P.R * P.nseg; };
-            size_t part_rows = partials(piece(first));
-            while (keep && last + 1 - first < in_group && (last + 1) * ATT_BUCKET_ < end) {
-                const size_t more = part_rows + partials(piece(last + 1));
-                if (more * NKV * HD * 4 > PREFILL_PART) break;
-                part_rows = more;
-                last++;
-            }
-            const int L = std::min(end, (last + 1) * ATT_BUCKET_), b = L - pos;
-            HCK(launch_append(s.S, seq, layer0, n_layers, n0, b - a0, static_cast<const char *>(k) + a0 * krow * esz,
-                              static_cast<const char *>(v) + a0 * krow * esz, dtype, st, nullptr, nullptr, knw, knw ? s.rope : nullptr));
-            s.top[seq] = std::max(s.top[seq], L);
-            s.n[seq] = std::max(s.n[seq], L);
-            p.L = L;
-            p.p0 = keep && a0 > 0 ? n0 / ATP_ : 0; // (the rows before the call with the first group's)
-            p.p1 = (L + ATP_ - 1) / ATP_;
-            p.q0 = s.kvrc == 0 ? 0 : keep ? n0 / ATP_ : window_start(L, s.win) / ATP_;
-            p.q1 = s.kvrc == 0 ? 0 : p.p1;
-            p.np = 0;
-            int q_blocks = 0;
-            for (int i = last; i >= first; i--) { // the longest contexts first
-                PrefillPiece & P = p.pc[p.np++];
-                P = piece(i);
-                P.qb0 = q_blocks;
-                q_blocks += (P.R + 31) / 32;
-            }
-            for (int l = 0, e; l < n_layers; l = e) {
-                e = run_end(l, part_rows);
-                set_run(l, e);
-                const unsigned slots = ((1u << p.nl) - 1u) << p.layer;
-                p.q_blocks = p.pc[0].nseg > 1 && (qnw || (p.krot & slots)) ? q_blocks : 0;
-                const size_t run_rows = (size_t) p.nl * p.ng * part_rows, part_need = run_rows * HD * sizeof(float);
-                s.grow(s.part, s.part_bytes, part_need + (size_t) p.nl * p.ng * p.q_blocks * Q16_BLOCK); // (the queries after the partials)
-                s.grow(s.ml, s.ml_bytes, run_rows * sizeof(float2));
-                p.part = static_cast<float *>(s.part);
-                p.q16 = static_cast<uint8_t *>(s.part) + part_need;
-                p.ml = static_cast<float2 *>(s.ml);
+        walk(
+            [&](int a0, int b) {
+                const int n0 = pos + a0, L = pos + b;
+                HCK(launch_append(s.S, seq, layer0, n_layers, n0, b - a0, static_cast<const char *>(k) + a0 * krow * esz,
+                                  static_cast<const char *>(v) + a0 * krow * esz, dtype, st, nullptr, nullptr, knw, knw ? s.rope : nullptr));
+                s.top[seq] = std::max(s.top[seq], L);
+                s.n[seq] = std::max(s.n[seq], L);
+                p.L = L;
+                p.p0 = sh.keep && a0 > 0 ? n0 / ATP_ : 0; // (the rows before the call with the first group's)
+                p.p1 = (L + ATP_ - 1) / ATP_;
+                p.q0 = s.kvrc == 0 ? 0 : sh.keep ? n0 / ATP_ : window_start(L, s.win) / ATP_;
+                p.q1 = s.kvrc == 0 ? 0 : p.p1;
+            },
+            [&](int l, int, int a0, size_t n) {
+                set_tiles(l);
+                p.q16 = static_cast<uint8_t *>(s.part) + n * HD * sizeof(float); // (the queries after the partials)
                 const size_t trow = (size_t) l * T + a0; // first token row of the group in this run's block
                 p.q = q + trow * NH * qs;
                 p.qnw = qnw ? qnw + (size_t) l * HD : nullptr;
@@ -893,9 +954,7 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
                     HCK(launch_prefill(p, st));
                 }
                 p.g0 = 0;
-            }
-            a0 = b;
-        }
+            });
         return 0;
     });
 }
@@ -1127,6 +1186,11 @@ int mk_kv_config(void * h, const char * key, long long value) {
         if (!strcmp(key, "occupancy")) {
             if (value != 0 && value != 2 && value != 3) throw std::runtime_error("occupancy must be 0 (by launch size), 2 or 3");
             s.occupancy = (int) value;
+            return 0;
+        }
+        if (!strcmp(key, "prefill_scratch")) {
+            if (value < 0) throw std::runtime_error("prefill_scratch must be >= 0 bytes");
+            s.prefill_scratch = (size_t) value;
             return 0;
         }
         throw std::runtime_error(std::string("unknown knob ") + key);

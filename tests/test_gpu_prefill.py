@@ -322,3 +322,36 @@ def test_prefill_rows_written_without_the_merge(qkv, oracle, torch_gpu, P, cut):
     assert rel_err(one[:, P - 1].cpu().numpy(), dec[:, 0, 0].cpu().numpy()) <= 2e-3
     st.close()
     st2.close()
+
+
+@pytest.mark.parametrize("spec,win,pos", [("K0=5r,V0=6,K1=6,V1=5r", 2048, 2500), ("", 0, 700)])
+def test_prefill_in_less_workspace(qkv, torch_gpu, spec, win, pos):
+    """The shapes that a bound on the workspace leaves, on the way down: four pieces per launch, one piece and one layer, one
+    layer's tiles at a time, two kv heads', one's (test_host_prefill.py follows their launches).  The same bits in all:
+    several groups of a call that starts past a window, and window tiles past the end of their ring (182 tiles, 5,824
+    positions).  Less than that is refused, and nothing is stored."""
+    torch = torch_gpu
+    nl, T = 2, 4000
+    g = torch.Generator(device="cuda")
+    g.manual_seed(pos)
+    k, v = (torch.randn(T, nl, NKV, HD, device="cuda", generator=g) for _ in range(2))
+    qg = torch.randn(nl, T, NH, 2 * HD, device="cuda", generator=g)
+    kn, qn = (1 + 0.1 * torch.randn(nl, HD, device="cuda", generator=g) for _ in range(2))
+    outs = []
+    for room in (0, 140, 90, 45, 24, 10):
+        st = qkv.KVStore(spec, win=win, n_layers=nl, ctx=pos + T)
+        fill(torch, st, pos, nl, 3)
+        st.set_rope()
+        st.config("prefill_scratch", room << 20)
+        o = torch.full((nl, T, NH, HD), float("nan"), device="cuda")
+        args = (0, 0, nl, pos, T, k.data_ptr(), v.data_ptr(), kn.data_ptr(), qg.data_ptr(), qn.data_ptr(), o.data_ptr())
+        if room == 10:
+            with pytest.raises(qkv.KVError, match="no device memory"):
+                st.prefill_prep(*args)
+            assert st.digest(0)[1] == pos
+        else:
+            st.prefill_prep(*args)
+            torch.cuda.synchronize()
+            outs.append(o)
+            assert torch.isfinite(o).all() and torch.equal(o, outs[0]), room
+        st.close()
