@@ -16,7 +16,8 @@
  * kv head and layer (plus the window's), at most 640 MiB asked for at a time; a call that needs more, or more than the
  * device has, runs its layers, and past that its kv heads, one after another.  It holds its whole workspace before it
  * stores anything: one that cannot have the least of it (one kv head's tiles, and the partials of 640 tokens of one kv
- * head: 30 MiB past 40,960 positions) is refused and changes nothing.
+ * head: 30 MiB past 40,960 positions) is refused and changes nothing.  A prefill call may grow it inside a stream capture
+ * (the attend calls may not: warm them up first).
  *
  * Shapes: NKV = 4 kv heads, NH = 24 query heads (GQA 6), head dim 256, up to 17 attention slots (layers), up to 8
  * query tokens per attend call, up to 8 sequences per attend call.

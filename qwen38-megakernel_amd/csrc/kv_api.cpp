@@ -131,6 +131,18 @@ uint64_t dg_hash(const void * p, size_t nb, uint64_t h = 0xcbf29ce484222325ULL) 
     return h;
 }
 
+// while it lives, this thread may call what a stream capture otherwise forbids (hipMalloc, hipFree)
+struct CaptureMode {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool on;
+    explicit CaptureMode(bool relaxed) : on(relaxed) {
+        if (on) (void) hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    ~CaptureMode() {
+        if (on) (void) hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
 struct Store {
     int dev = 0; // the HIP device the store's memory lives on
     int n_layers = 0, n_seq = 0, ctx = 0, page = 0, n_pages = 0, pt_stride = 0, win = 0, kvrc = 0, win_all = 0;
@@ -202,9 +214,11 @@ struct Store {
         size_t need;
     };
     // every buffer of w at least as large as needed, or none of them touched: a buffer allocated before another one's
-    // allocation failed is given back (no work knows it yet)
-    template <size_t N> hipError_t try_hold(const Want (&w)[N]) {
+    // allocation failed is given back (no work knows it yet).  in_capture: also while a stream of the program is being
+    // captured (the buffers outlive the graph as any other's do, to mk_free)
+    template <size_t N> hipError_t try_hold(const Want (&w)[N], bool in_capture = false) {
         retired.reserve(retired.size() + N);
+        const CaptureMode mode(in_capture);
         hipError_t e = hipSuccess;
         for (const bool ahead : {true, false}) { // (a nearly full device: no more than needed)
             void * q[N] = {};
@@ -898,8 +912,10 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
                  });
             const size_t kv16_need = units() * (unit + qunit);
             if (s.prefill_scratch && kv16_need + part_need + ml_need > s.prefill_scratch) continue;
+            // (in_capture: the tiles grow with the context, so a program that captures its chunks one after another, warmed up on
+            // the first, allocates inside every capture that goes further than any call before it)
             const hipError_t e = s.try_hold<3>(
-                {{&s.kv16, &s.kv16_bytes, kv16_need}, {&s.part, &s.part_bytes, part_need}, {&s.ml, &s.ml_bytes, ml_need}});
+                {{&s.kv16, &s.kv16_bytes, kv16_need}, {&s.part, &s.part_bytes, part_need}, {&s.ml, &s.ml_bytes, ml_need}}, true);
             held = e == hipSuccess;
             if (!held && e != hipErrorOutOfMemory) throw HipError(std::string("prefill workspace: ") + hipGetErrorString(e));
         }

@@ -15,6 +15,8 @@
 namespace {
 size_t limit_ = 0, used_ = 0, next_ = 1 << 20; // bytes of the device, allocated, next address
 int error_ = 0;                                // hipMalloc returns this, if set
+bool capturing_ = false;                       // a stream is being captured: hipMalloc only in the relaxed mode
+hipStreamCaptureMode mode_ = hipStreamCaptureModeGlobal;
 std::map<size_t, size_t> live_;                // address -> bytes
 std::string bad_;
 int appends_ = 0, launches_ = 0, most_pieces_ = 0, most_layers_ = 0, least_heads_ = 4;
@@ -116,6 +118,7 @@ hipError_t launch_prefetch(const AttnArgs &, int, int, int, hipStream_t) { retur
 extern "C" {
 hipError_t hipMalloc(void ** p, size_t n) {
     if (error_) return (hipError_t) error_;
+    if (capturing_ && mode_ != hipStreamCaptureModeRelaxed) return hipErrorStreamCaptureUnsupported;
     if (limit_ && used_ + n > limit_) return hipErrorOutOfMemory;
     used_ += n;
     live_[next_] = n;
@@ -128,6 +131,7 @@ hipError_t hipFree(void * p) {
     live_.erase((size_t) p);
     return hipSuccess;
 }
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode * m) { return std::swap(mode_, *m), hipSuccess; }
 hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t *, unsigned) { return hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
@@ -144,6 +148,11 @@ hipError_t hipMemset(void *, int, size_t) { return hipSuccess; }
 void model_room(size_t room, int error) {
     limit_ = room ? used_ + room : 0;
     error_ = error;
+}
+// -> 1 if the thread's capture mode is the program's again
+int model_capture(int on) {
+    capturing_ = on;
+    return mode_ == hipStreamCaptureModeGlobal;
 }
 size_t model_used(void) { return used_; }
 void model_begin(const float * out) {

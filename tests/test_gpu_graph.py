@@ -76,3 +76,35 @@ def test_graph_survives_workspace_growth(qkv, torch_gpu):
         graph.replay()
         torch.cuda.synchronize()
         np.testing.assert_array_equal(out.cpu().numpy(), ref, err_msg=f"replay {rep}")
+
+
+def test_prefill_captured_past_the_warmed_up_context(qkv, torch_gpu):
+    """A prefill chunk captured far past the chunk the workspace was warmed up on: its key tiles need more room, allocated
+    inside the capture.  Every replay, with an eager chunk between, gives the eager bits."""
+    torch = torch_gpu
+    rng = np.random.default_rng(97)
+    L, T = 12000, 150  # (one bucket: the ring still holds the window when the chunk is stored again)
+    st = qkv.KVStore("K*=5r,V*=6", win=2048, n_layers=1, ctx=L + T)
+    K, V = synth_kv(rng, L + T, 1, outliers=True)
+    k, v = torch.from_numpy(K).cuda(), torch.from_numpy(V).cuda()
+    q = torch.from_numpy(rng.standard_normal((1, T, NH, HD)).astype(np.float32)).cuda()
+    warm, out = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
+    st.prefill(0, 0, 1, 0, T, k.data_ptr(), v.data_ptr(), 0, q.data_ptr(), warm.data_ptr())  # the warm-up
+    append_all(torch, st, 0, K[:L], V[:L], chunks=[4096] * 3)
+    chunk = (0, 0, 1, L, T, k[L:].data_ptr(), v[L:].data_ptr(), 0, q.data_ptr())
+    side = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(graph, stream=side):
+            st.prefill(*chunk, out.data_ptr(), side.cuda_stream)
+    eager = torch.full_like(q, float("nan"))
+    st.prefill(*chunk, eager.data_ptr())
+    torch.cuda.synchronize()
+    assert torch.isfinite(eager).all()
+    for rep in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), rep
+        st.prefill(*chunk, warm.data_ptr())
+        torch.cuda.synchronize()

@@ -121,3 +121,15 @@ def test_other_errors_are_reported_as_they_are(lib):
     r = st.prefill(0, 2000)
     assert "illegal state" in r and "no device memory" not in r and st.stored() == 0
     st.close()
+
+
+def test_a_longer_context_inside_a_capture(lib):
+    # warmed up on the first chunk; the captured one reads 40 times as many keys
+    st = Store(lib, F, 2048, 1, 50000)
+    st.prefill(0, 640)
+    st.append(40000)
+    lib.model_capture(1)
+    r = st.prefill(40000, 640)
+    assert lib.model_capture(0) == 1  # (the thread's capture mode as it was)
+    assert r[4] == 4 and st.stored() == 40640, r
+    st.close()
