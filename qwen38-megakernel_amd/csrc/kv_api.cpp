@@ -814,8 +814,10 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
         // their tiles.  (One tile to spare: the attention copies tiles in pairs.)
         const int end = pos + T, kv_tiles = (end + ATP_ - 1) / ATP_ + 1;
         const int in_group = s.kvrc > 0 ? std::min(PF_PIECES, s.kvrc / ATT_BUCKET_) : PF_PIECES;
-        // the window's tiles a group can see: its pieces' and, before them, the first one's window
-        const int q_tiles = s.kvrc > 0 ? (s.kvrc / ATT_BUCKET_ + in_group) * (ATT_BUCKET_ / ATP_) + 2 : 0;
+        // the window's tiles a group can see: its pieces' and, before them, the first one's window, but no more than there are
+        // (even: a pair of tiles does not wrap)
+        const int q_tiles =
+            s.kvrc > 0 ? std::min((s.kvrc / ATT_BUCKET_ + in_group) * (ATT_BUCKET_ / ATP_) + 2, (kv_tiles + 1) / 2 * 2) : 0;
         const size_t unit = (size_t) kv_tiles * KV16_TILE, qunit = (size_t) q_tiles * KV16_TILE, fit = PREFILL_KV16_MAX / (unit + qunit);
         PrefillArgs p{};
         p.S = s.S;

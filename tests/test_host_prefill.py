@@ -133,3 +133,13 @@ def test_a_longer_context_inside_a_capture(lib):
     assert lib.model_capture(0) == 1  # (the thread's capture mode as it was)
     assert r[4] == 4 and st.stored() == 40640, r
     st.close()
+
+
+def test_a_short_prompt_with_a_large_window(lib):
+    # 16 tokens over 16 layers: two tiles of each kind per layer and head, not the 362 that the window can have
+    st = Store(lib, F, 8192, 16, 20000)
+    used = lib.model_used()
+    r = st.prefill(0, 16)
+    assert r[1:4] == (2, 1, 16), r  # all layers' tiles in one launch, all layers in one attention
+    assert lib.model_used() - used == 16 * 4 * (2 + 2) * 32768
+    st.close()
