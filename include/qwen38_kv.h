@@ -13,7 +13,7 @@
  * graph captured over an earlier call stays valid after a larger call (its replays keep using the old, smaller
  * buffer; a graph replay and an eager call of one handle must still not overlap).  The kept buffers together stay
  * below twice the live workspace.  The prefill calls also keep their keys as fp16 tiles in it: 1,024 bytes per position,
- * kv head and layer (plus the window's), at most 640 MiB asked for at a time; a call that needs more, or more than the
+ * kv head and layer (plus the window's), at most 640 MiB asked for at a time (more only for one kv head past 600,000 positions); a call that needs more, or more than the
  * device has, runs its layers, and past that its kv heads, one after another.  It holds its whole workspace before it
  * stores anything: one that cannot have the least of it (one kv head's tiles, and the partials of 640 tokens of one kv
  * head: 30 MiB past 40,960 positions) is refused and changes nothing.  A prefill call may grow it inside a stream capture

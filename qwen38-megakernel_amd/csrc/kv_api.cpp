@@ -212,6 +212,7 @@ struct Store {
         void ** p;
         size_t * have;
         size_t need;
+        size_t ahead = SIZE_MAX; // growth past the need (1.5 times) stays within this
     };
     // every buffer of w at least as large as needed, or none of them touched: a buffer allocated before another one's
     // allocation failed is given back (no work knows it yet).  in_capture: also while a stream of the program is being
@@ -226,7 +227,7 @@ struct Store {
             e = hipSuccess;
             for (size_t i = 0; i < N && e == hipSuccess; i++) {
                 if (w[i].need <= *w[i].have) continue;
-                got[i] = ahead ? std::max(w[i].need, *w[i].have + *w[i].have / 2) : w[i].need;
+                got[i] = ahead ? std::max(w[i].need, std::min(*w[i].have + *w[i].have / 2, w[i].ahead)) : w[i].need;
                 e = hipMalloc(&q[i], got[i]);
             }
             if (e == hipSuccess) {
@@ -917,7 +918,7 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
             // (in_capture: the tiles grow with the context, so a program that captures its chunks one after another, warmed up on
             // the first, allocates inside every capture that goes further than any call before it)
             const hipError_t e = s.try_hold<3>(
-                {{&s.kv16, &s.kv16_bytes, kv16_need}, {&s.part, &s.part_bytes, part_need}, {&s.ml, &s.ml_bytes, ml_need}}, true);
+                {{&s.kv16, &s.kv16_bytes, kv16_need, PREFILL_KV16_MAX}, {&s.part, &s.part_bytes, part_need}, {&s.ml, &s.ml_bytes, ml_need}}, true);
             held = e == hipSuccess;
             if (!held && e != hipErrorOutOfMemory) throw HipError(std::string("prefill workspace: ") + hipGetErrorString(e));
         }

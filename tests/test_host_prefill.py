@@ -143,3 +143,17 @@ def test_a_short_prompt_with_a_large_window(lib):
     assert r[1:4] == (2, 1, 16), r  # all layers' tiles in one launch, all layers in one attention
     assert lib.model_used() - used == 16 * 4 * (2 + 2) * 32768
     st.close()
+
+
+def test_the_tiles_grow_within_their_bound(lib):
+    # 586 MiB of tiles, then 601: asked for ahead of the need, but not past 640 MiB (the outgrown buffer is kept beside it)
+    st = Store(lib, "", 0, 4, 40000)
+    st.append(37500)
+    used = lib.model_used()
+    st.prefill(37500, 1)
+    first = lib.model_used() - used
+    assert 586 * MIB < first < 600 * MIB
+    st.append(38400)
+    st.prefill(38400, 1)
+    assert lib.model_used() - used - first <= 641 * MIB
+    st.close()
