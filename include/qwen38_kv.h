@@ -12,12 +12,12 @@
  * workspace grows on demand (by at least 1.5 times); a buffer it outgrows is kept, not freed, until mk_free, so a HIP
  * graph captured over an earlier call stays valid after a larger call (its replays keep using the old, smaller
  * buffer; a graph replay and an eager call of one handle must still not overlap).  The kept buffers together stay
- * below twice the live workspace.  The prefill calls also keep their keys as fp16 tiles in it: 1,024 bytes per position,
- * kv head and layer (plus the window's), at most 640 MiB asked for at a time (more only for one kv head past 600,000 positions); a call that needs more, or more than the
- * device has, runs its layers, and past that its kv heads, one after another.  It holds its whole workspace before it
- * stores anything: one that cannot have the least of it (one kv head's tiles, and the partials of 640 tokens of one kv
- * head: 30 MiB past 40,960 positions) is refused and changes nothing.  A prefill call may grow it inside a stream capture
- * (the attend calls may not: warm them up first).
+ * below twice the live workspace.  The prefill calls also keep their keys as fp16 tiles in it: 1,024 bytes per
+ * position, kv head and layer (plus the window's), at most 640 MiB asked for at a time (more only for one kv head past
+ * 600,000 positions); a call that needs more, or more than the device has, runs its layers, and past that its kv heads,
+ * one after another.  It holds its whole workspace before it stores anything: one that cannot have the least of it (one
+ * kv head's tiles, and the partials of 640 tokens of one kv head: 30 MiB past 40,960 positions) is refused and changes
+ * nothing.  A prefill call may grow it inside a stream capture (the attend calls may not: warm them up first).
  *
  * Shapes: NKV = 4 kv heads, NH = 24 query heads (GQA 6), head dim 256, up to 17 attention slots (layers), up to 8
  * query tokens per attend call, up to 8 sequences per attend call.

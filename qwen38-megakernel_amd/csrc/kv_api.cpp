@@ -246,7 +246,9 @@ struct Store {
         }
         return e;
     }
-    void grow(void *& p, size_t & have, size_t need) { HCK(try_hold<1>({{&p, &have, need}})); }
+    void grow(void *& p, size_t & have, size_t need) {
+        if (need > have) HCK(try_hold<1>({{&p, &have, need}}));
+    }
     size_t main_row(int seq, int g, int p) const {
         const int lp = p / page;
         return (size_t) (g * n_pages + ptab[(size_t) seq * pt_stride + lp]) * page + (p - lp * page);
