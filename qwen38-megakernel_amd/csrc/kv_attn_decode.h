@@ -129,10 +129,10 @@ __device__ __forceinline__ unsigned hi_dword(const unsigned * h, int ks) {
 template <int HB>
 __device__ __forceinline__ constexpr int hi_part(int ks) { return HB == 1 ? ks & 3 : ks & 1; }
 
-// where a K / V format's masks go (code_pairs)
-template <int KB, int VB>
+// where a K / V format's masks go (code_pairs) in a kernel of NP row groups
+template <int NP, int KB, int VB>
 __device__ __forceinline__ constexpr bool mask_sc() {
-    return KB != 6 && VB != 6;
+    return NP > 1 || (KB != 6 && VB != 6);
 }
 
 // fp16 A fragment of K step ks: values 8 ks .. 8 ks + 7 of the lane's row quarter, in pair order (pair_at)
@@ -504,8 +504,8 @@ __device__ __forceinline__ void compute_tile(WaveState<NP> & st, const half8 * s
     for (int h = 0; h < NP; h++) s[h][0] = s[h][1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < 8; ks++) {
-        const half8 a0 = kfrag<KB, mask_sc<KB, VB>()>(raw.k0, ks);
-        const half8 a1 = kfrag<KB, mask_sc<KB, VB>()>(raw.k1, ks);
+        const half8 a0 = kfrag<KB, mask_sc<NP, KB, VB>()>(raw.k0, ks);
+        const half8 a1 = kfrag<KB, mask_sc<NP, KB, VB>()>(raw.k1, ks);
 #pragma unroll
         for (int h = 0; h < NP; h++) {
             const half8 b = NP == 1 ? st.qf[ks] : sQ[qchunk(8 * h + (n >> 1), 8 * q + ks)];
@@ -593,7 +593,7 @@ __device__ __forceinline__ void compute_tile(WaveState<NP> & st, const half8 * s
         lds_drain();
         after_v();
     }
-    tile_pv<NP, VB, mask_sc<KB, VB>()>(st.acc, raw.v, pb);
+    tile_pv<NP, VB, mask_sc<NP, KB, VB>()>(st.acc, raw.v, pb);
 }
 
 // one row group's accumulators of a lane (odd: its dim parity) times e into the row's LDS buffer at its quarter's first
@@ -649,8 +649,8 @@ __device__ __forceinline__ void tile_scores(f32x4 (&s)[(NP + 1) / 2][2], const R
     for (int H = 0; H < NB; H++) s[H][0] = s[H][1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < 8; ks++) {
-        const half8 a0 = kfrag<KB, mask_sc<KB, VB>()>(raw.k0, ks);
-        const half8 a1 = kfrag<KB, mask_sc<KB, VB>()>(raw.k1, ks);
+        const half8 a0 = kfrag<KB, mask_sc<NP, KB, VB>()>(raw.k0, ks);
+        const half8 a1 = kfrag<KB, mask_sc<NP, KB, VB>()>(raw.k1, ks);
 #pragma unroll
         for (int H = 0; H < NB; H++) {
             const half8 b = qf(H, ks);
@@ -760,7 +760,7 @@ __device__ __forceinline__ void compute_tile_v(RowState<NP> & st, const half8 * 
     load_v(raw, n, q);
     lds_drain();
     after_v();
-    tile_pv<NP, VB, mask_sc<KB, VB>()>(st.acc, raw.v, pb);
+    tile_pv<NP, VB, mask_sc<NP, KB, VB>()>(st.acc, raw.v, pb);
 }
 
 // The fused append's rows of one workgroup (mk_kv_append_attend): positions pa .. pb - 1 of its segment, both sides,

@@ -53,7 +53,8 @@ QKV_HD uint32_t and_or(uint32_t x, uint32_t m, uint32_t c) {
 // B = 7 the low 24 bits (idx unused, the bits above them ignored)
 // SC: the high bits' masks in scalar registers.  The three-per-CU kernels have a few of each kind to spare: with 6-bit
 // sides (two masks more) all-scalar masks spill scalars into the tile loop (5 + 6 bits: 2% slower), and with 5-bit sides
-// alone masks in VGPRs spill those (5 + 5 bits: 2% slower).
+// alone masks in VGPRs spill those (5 + 5 bits: 2% slower).  The 16- and 24-row kernels have no VGPR to spare (5 + 6 bits,
+// T = 4, masks in VGPRs: two more spilled; eight short sequences 144.8 us over four layers, in scalars 137.9)
 template <int B, bool SC = true>
 QKV_HD void code_pairs(uint32_t W, uint32_t hd, int idx, uint32_t (&p)[4]) {
     constexpr uint32_t M64 = 0x64006400u, M54 = 0x54005400u, N0 = 0x000f000fu, N4 = 0x00f000f0u;
