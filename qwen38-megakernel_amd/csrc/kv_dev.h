@@ -313,10 +313,7 @@ __device__ __forceinline__ half2v pair_operand(unsigned p, float bias, half2v d2
 __device__ __forceinline__ void q8_pairs(unsigned d0, unsigned d1, unsigned (&p)[4]) {
     d0 ^= 0x80808080u; // signed q -> q + 128
     d1 ^= 0x80808080u;
-    p[0] = perm_b32(d0, 0x64646464u, 0x00060004u);
-    p[1] = perm_b32(d0, 0x64646464u, 0x00070005u);
-    p[2] = perm_b32(d1, 0x64646464u, 0x00060004u);
-    p[3] = perm_b32(d1, 0x64646464u, 0x00070005u);
+    byte_pairs(d0, d1, p);
 }
 
 } // namespace qkv
