@@ -1159,6 +1159,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SMALL ? 3 :
         }
         __syncthreads();
         const int RB = min(RP, R - row0); // rows of this batch
+        // the thread by the opaque lane: threadIdx.x would be held, spilled, across the tile loop.  (q8 on both sides has the
+        // register, and loses 3-6% to spilled scalars without it)
+        const int tid = KB == 8 && VB == 8 ? (int) threadIdx.x : 64 * wv + lane;
         constexpr int NPASS = (NP + 1) / 2;
 #pragma unroll
         for (int ps = 0; ps < NPASS; ps++) {
@@ -1175,7 +1178,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SMALL ? 3 :
             }
             __syncthreads();
             const int nrow = min(16, RB - 16 * ps);
-            for (int idx = threadIdx.x; idx < nrow * (HD / 4); idx += 256) {
+            for (int idx = tid; idx < nrow * (HD / 4); idx += 256) {
                 const int r16 = idx / (HD / 4), c4 = idx % (HD / 4);
                 const float * src = reinterpret_cast<const float *>(smem) + r16 * OLD + 4 * c4;
                 float4 y = *reinterpret_cast<const float4 *>(src);
@@ -1191,8 +1194,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SMALL ? 3 :
             }
             if (ps + 1 < NPASS) __syncthreads();
         }
-        if (threadIdx.x < RB) {
-            const int row = threadIdx.x;
+        if (tid < RB) {
+            const int row = tid;
             const float M = fmaxf(fmaxf(s_m[row], s_m[RP + row]), fmaxf(s_m[2 * RP + row], s_m[3 * RP + row]));
             float lsum = 0.f;
 #pragma unroll
@@ -1412,7 +1415,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 s_l[wv * RP + block_row<NP>(H, n)] = st.l[H];
             }
         }
-        const int th = threadIdx.x / 256, tl = threadIdx.x - 256 * th, wb = AWAVES * th;
+        const int th = hf, tl = 64 * sl + lane, wb = AWAVES * th; // (thread tl of half th, by the opaque lane)
         const int trow0 = RP * th, RB = min(RP, R - trow0);
         const float * const s_mh = s_m + wb * RP, * const s_mw = s_m + hf * AWAVES * RP;
         lds_barrier();
