@@ -157,3 +157,16 @@ def test_the_tiles_grow_within_their_bound(lib):
     st.prefill(38400, 1)
     assert lib.model_used() - used - first <= 641 * MIB
     st.close()
+
+
+@pytest.mark.parametrize("pos,T,groups,own", [(500, 16, 1, 0), (1072, 128, 1, 0), (3199, 1, 1, 0), (6001, 399, 1, 0), (6400, 640, 1, 0),
+                                              (600, 2600, 2, 0), (6001, 400, 1, 0), (6001, 440, 1, 1), (6001, 1000, 1, 1), (2000, 4000, 2, 1)])
+def test_window_rows_with_the_first_group(lib, pos, T, groups, own):
+    # the window's rows before the call take a launch of their own only where the first group's rows replace some of them in
+    # the ring of 3,232 (6,001 positions: the window starts at 3,200); otherwise a group is one launch over the tiles and one of
+    # the attention.  (That no row is read after it was replaced: as in test_every_shape_covers_the_call.)
+    st = Store(lib, F, 2048, 1, pos + T)
+    st.append(pos)
+    r = st.prefill(pos, T)
+    assert r[:2] == (groups, 2 * groups + own), r
+    st.close()
