@@ -952,6 +952,7 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
                 HCK(launch_prefill_kv(p, bits(l, 0), bits(l, 1), st));
             }
         }
+        int main_done = 0; // tiles of main rows that the call's groups have unpacked
         walk(
             [&](int a0, int b) {
                 const int n0 = pos + a0, L = pos + b;
@@ -960,10 +961,14 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
                 s.top[seq] = std::max(s.top[seq], L);
                 s.n[seq] = std::max(s.n[seq], L);
                 p.L = L;
-                p.p0 = sh.keep && a0 > 0 ? n0 / ATP_ : 0; // (the rows before the call with the first group's)
-                p.p1 = (L + ATP_ - 1) / ATP_;
+                // main rows up to the last piece's window, past whose start no piece reads them (the rows before the call with the
+                // first group's); the others once a later group's window has passed them
+                const int tiles = (L + ATP_ - 1) / ATP_;
+                p.p0 = sh.keep ? main_done : 0;
+                p.p1 = s.kvrc > 0 ? std::max(p.p0, window_start(L, s.win) / ATP_) : tiles;
+                main_done = s.kvrc > 0 ? p.p1 : L / ATP_; // (a last tile whose rows are not all stored: again)
                 p.q0 = s.kvrc == 0 ? 0 : !sh.keep ? window_start(L, s.win) / ATP_ : (a0 == 0 && window_kept ? win0 : n0) / ATP_;
-                p.q1 = s.kvrc == 0 ? 0 : p.p1;
+                p.q1 = s.kvrc == 0 ? 0 : tiles;
             },
             [&](int l, int, int a0, size_t n) {
                 set_tiles(l);

@@ -19,6 +19,7 @@ bool capturing_ = false;                       // a stream is being captured: hi
 hipStreamCaptureMode mode_ = hipStreamCaptureModeGlobal;
 std::map<size_t, size_t> live_;                // address -> bytes
 std::string bad_;
+int unread_ = 0; // tiles that no attention has read
 int appends_ = 0, launches_ = 0, most_pieces_ = 0, most_layers_ = 0, least_heads_ = 4;
 
 void fail(const char * what, long long a = 0, long long b = 0) {
@@ -36,6 +37,7 @@ void inside(const void * p, size_t n, const char * what) {
 }
 struct Tile {
     int layer, g, t, rows; // rows: positions 32 t .. 32 t + rows - 1 of the layer's head
+    bool read = false;
 };
 std::map<size_t, Tile> tiles_;
 std::map<std::pair<int, int>, int> ring_; // (layer, ring row) -> position
@@ -68,7 +70,9 @@ hipError_t launch_prefill_kv(const PrefillArgs & a, int kb, int vb, hipStream_t)
                 if (rows < 1 || ATP * t + rows > stored_[l]) fail("tile of rows that are not stored", t, stored_[l]);
                 for (int p = ATP * t; w && p < ATP * t + rows; p++)
                     if (ring_[{l, p % a.S.kvrc}] != p) fail("window row replaced in the ring", l, p);
-                tiles_[(size_t) at] = Tile{l, g, w ? -1 - t : t, rows};
+                Tile & x = tiles_[(size_t) at];
+                if (x.rows && !x.read) unread_++;
+                x = Tile{l, g, w ? -1 - t : t, rows};
             }
     }
     inside(a.q16, (size_t) a.nl * a.ng * a.q_blocks * Q16_BLOCK, "query operands");
@@ -88,6 +92,7 @@ hipError_t launch_prefill(PrefillArgs & a, hipStream_t) {
                 const bool w = ATP * t >= P.ws;
                 const uint8_t * at = w ? a.kq16 + ((size_t) u * a.q_tiles + t % a.q_tiles) * KV16_TILE : a.kv16 + ((size_t) u * a.kv_tiles + t) * KV16_TILE;
                 const auto x = tiles_.find((size_t) at);
+                if (x != tiles_.end()) x->second.read = true;
                 if (x == tiles_.end() || x->second.layer != l || x->second.g != g || x->second.t != (w ? -1 - t : t) ||
                     x->second.rows < std::min(ATP, pmax + 1 - ATP * t))
                     fail("tile read before it is written", l, t);
@@ -160,6 +165,7 @@ void model_begin(const float * out) {
     done_.clear();
     bad_.clear();
     tiles_.clear(); // (a call reads nothing that an earlier one unpacked)
+    unread_ = 0;
     appends_ = launches_ = most_pieces_ = most_layers_ = 0;
     least_heads_ = 4;
 }
@@ -174,6 +180,12 @@ const char * model_faults(long long rows) {
 void model_counts(int * c) {
     const int v[5] = {appends_, launches_, most_pieces_, most_layers_, least_heads_};
     for (int i = 0; i < 5; i++) c[i] = v[i];
+}
+// tiles unpacked for nothing
+int model_unread(void) {
+    int n = unread_;
+    for (const auto & x : tiles_) n += !x.second.read;
+    return n;
 }
 int model_stored(void * h, int seq) { return static_cast<Store *>(h)->n[seq]; }
 }

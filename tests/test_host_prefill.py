@@ -170,3 +170,15 @@ def test_window_rows_with_the_first_group(lib, pos, T, groups, own):
     r = st.prefill(pos, T)
     assert r[:2] == (groups, 2 * groups + own), r
     st.close()
+
+
+@pytest.mark.parametrize("spec,win,nl,pos,T", [(F, 2048, 1, 0, 2000), (F, 2048, 2, 0, 9000), (F, 2048, 1, 30000, 100), (F, 2048, 1, 6001, 4000),
+                                               (F, 640, 1, 650, 1300), ("", 0, 4, 1000, 3000), (F, 2048, 16, 12000, 700)])
+def test_every_unpacked_tile_is_read(lib, spec, win, nl, pos, T):
+    # a window's rows are read from its own tiles: no main tiles are unpacked for them.  (One tile of window rows per layer and
+    # head is unpacked twice where those before the call come first: the one that the call's first rows complete.)
+    st = Store(lib, spec, win, nl, pos + T)
+    st.append(pos)
+    assert isinstance(st.prefill(pos, T), tuple)
+    assert lib.model_unread() <= 4 * nl * (win > 0 and pos % 32 != 0)
+    st.close()
