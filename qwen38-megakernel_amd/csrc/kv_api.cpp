@@ -887,7 +887,10 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
                     p.layer = layer0 + l;
                     p.nl = e - l;
                     const unsigned slots = ((1u << p.nl) - 1u) << p.layer;
-                    p.q_blocks = sh.q_once && p.pc[0].nseg > 1 && (qnw || (p.krot & slots)) ? q_blocks : 0;
+                    int wgs = 0; // workgroups of the attention
+                    for (int i = 0; i < p.np; i++) wgs += (p.pc[i].R + PF2_ROWS - 1) / PF2_ROWS * p.pc[i].nseg * p.nl * sh.ng;
+                    const bool prep = qnw || (p.krot & slots);
+                    p.q_blocks = sh.q_once && ((prep && p.pc[0].nseg > 1) || wgs <= (prep ? PF_FEW_PREP : PF_FEW)) ? q_blocks : 0;
                     run(l, e, a0, (size_t) p.nl * sh.ng * part_rows);
                 }
                 a0 = b;

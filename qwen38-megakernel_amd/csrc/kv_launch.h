@@ -146,10 +146,14 @@ struct PrefillArgs {
     int kv_tiles, q_tiles; // tiles per unit of kv16 (main rows) and kq16 (window rows, tile t at t % q_tiles)
     unsigned krot, vrot; // per-slot bit masks: K / V stored rotated
     // 32-row blocks of the group's pieces per unit, and [nl ng][q_blocks][Q16_BLOCK] fp16 operands (kv_attn.hip) of the query
-    // rows, for groups with several segments per row whose queries get the prep or the FWHT: done once per row beside the
-    // tiles' conversion, not by every segment's workgroup (16,384 positions, rotated K: 3,838 -> 3,780 us; a prepped
-    // 433-token chunk at 60,188 over two layers 1,524 -> 1,455).  0 otherwise: the extra pass over the queries then costs
-    // more than it saves (a 1,111-token prompt without either over four layers 285 -> 300)
+    // rows: done once per row beside the tiles' conversion, not by every segment's workgroup.  For groups with several segments per
+    // row whose queries get the prep or the FWHT (16,384 positions, rotated K: 3,838 -> 3,780 us; a prepped 433-token chunk at
+    // 60,188 over two layers 1,524 -> 1,455), and for launches of few workgroups, which leave the CUs idle that would share the
+    // work: PF_FEW_PREP with the prep or the FWHT (one layer, rotated K: 16 tokens after 500 positions 37.2 -> 32.0 us, 640 after
+    // 640, 120 workgroups, 60.0 -> 57.3; prepped 49.5 -> 40.6 and 74.5 -> 69.5; 240 workgroups 65.5 -> 66.0), PF_FEW without
+    // (128 after 1,072 46.7 -> 45.4; over four layers, 96 workgroups, 54.3 -> 51.8 but 128 alone 24.4 -> 25.3; 640 alone, 120,
+    // 36.5 -> 37.7).  0 otherwise: the extra pass over the queries then costs more than it saves (a 1,111-token prompt without
+    // either over four layers 285 -> 300)
     int q_blocks;
     uint8_t * q16;
     const float * q;   // [nl][T][NH][qs] from the group's first token
@@ -176,14 +180,17 @@ constexpr int Q16_BLOCK = 32 * HD * 2;      // 32 query rows as fp16
 // segments pay there (60,000 positions, 2 / 4 / 8 segments: 16 tokens 731 / 412 / 252 us, 256 tokens 706 / 474 / 506, 512
 // tokens 830 / 862 / 811, 640 tokens 946 / 962 / 1,003), and up to 20,480 positions whole prompts decide (16,384 with
 // four segments: 9% slower).  Rows of one segment need neither partials nor the combine, which were over half of a short
-// prompt's time: up to 1,280 positions one segment (two / one: 1,111 tokens over four layers 296 / 128 us, over one 80 / 53,
-// 640 tokens 44 / 38, 640 after 640 60 / 54; 128 after 1,072 38 / 47, whose one workgroup per row block walks all keys).
+// prompt's time (640 tokens 44 / 38 us with two / one): one segment up to 1,280 positions.  Where the line lies is a trade between
+// prompts and short chunks, whose few workgroups then walk all keys one after another.  One q8 layer with the line at 640 /
+// 1,280 / 1,920 positions: 1,111 tokens 68 / 52 / 52 us, 640 after 640 55 / 52 / 52 (over four layers 183 / 102 / 101), 128 after
+// 1,072 36 / 47 / 46; 1,920 tokens 130 / 107 / 87, 640 after 1,280 65 / 64 / 66, 128 after 1,700 45 / 45 / 61.
 inline int pf_seg(int L) {
     const int lb = (L + ATT_BUCKET - 1) / ATT_BUCKET * ATT_BUCKET;
     const int n = lb > 64 * ATT_BUCKET ? 8 : lb > 32 * ATT_BUCKET ? 4 : lb > 2 * ATT_BUCKET ? 2 : 1;
     return 128 * ((lb + 128 * n - 1) / (128 * n));
 }
 constexpr int PF2_ROWS = 128; // query rows per prefill workgroup (32 per wave)
+constexpr int PF_FEW_PREP = 128, PF_FEW = 64; // prefill workgroups of a launch: PrefillArgs::q_blocks
 
 // canonical segment length: 128 ceil(Lb / 16384) positions with Lb = L rounded up to a 640 bucket: a multiple of 4 tiles,
 // so the 4 waves of a workgroup stream the same number of tiles; at most 128 segments per kv head (one layer's 4 heads

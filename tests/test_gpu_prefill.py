@@ -355,3 +355,32 @@ def test_prefill_in_less_workspace(qkv, torch_gpu, spec, win, pos):
             outs.append(o)
             assert torch.isfinite(o).all() and torch.equal(o, outs[0]), room
         st.close()
+
+
+@pytest.mark.parametrize("spec,win,T,prep", [("", 0, 342, False), ("K*=5r,V*=6r", 2048, 683, False), ("K*=6,V*=5", 640, 683, True)])
+def test_prefill_queries_beside_the_tiles(qkv, torch_gpu, spec, win, T, prep):
+    # launches of up to 64 workgroups (128 with prep or rotated K) take queries prepared with the tiles, larger ones prepare
+    # their own: the call of one token less is the last of the first kind (4 x 16 workgroups; 4 x (30 + 2)).  The same bits
+    torch = torch_gpu
+    g = torch.Generator(device="cuda")
+    g.manual_seed(T)
+    k, v = (torch.randn(T, 1, NKV, HD, device="cuda", generator=g) for _ in range(2))
+    q = torch.randn(1, T, NH, (2 if prep else 1) * HD, device="cuda", generator=g)
+    kn, qn = (1 + 0.1 * torch.randn(1, HD, device="cuda", generator=g) for _ in range(2))
+    outs = []
+    for chunks in ([T], [T - 1, 1]):
+        st = qkv.KVStore(spec, win=win, n_layers=1, ctx=T)
+        st.set_rope()
+        o, p = torch.full((1, T, NH, HD), float("nan"), device="cuda"), 0
+        for c in chunks:
+            oc, qc = torch.empty(1, c, NH, HD, device="cuda"), q[:, p:p + c].contiguous()
+            if prep:
+                st.prefill_prep(0, 0, 1, p, c, k[p:].data_ptr(), v[p:].data_ptr(), kn.data_ptr(), qc.data_ptr(), qn.data_ptr(), oc.data_ptr())
+            else:
+                st.prefill(0, 0, 1, p, c, k[p:].data_ptr(), v[p:].data_ptr(), 0, qc.data_ptr(), oc.data_ptr())
+            torch.cuda.synchronize()
+            o[:, p:p + c] = oc
+            p += c
+        outs.append(o)
+        st.close()
+    assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1])
