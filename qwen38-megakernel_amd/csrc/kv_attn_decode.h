@@ -1159,12 +1159,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SMALL ? 3 :
         }
         __syncthreads();
         const int RB = min(RP, R - row0); // rows of this batch
-        // the thread by the opaque lane: threadIdx.x would be held, spilled, across the tile loop.  (The kernels that have a register
-        // for it lose to spilled scalars without it: q8 on both sides 3-6%; the fused append's of one and two row groups up to 5%
-        // (preset F, 16 layers of 9,001 positions 261 us with it, 276 without; T = 2 on 4 + 4 bits 243 / 251), and those of three
-        // without a 6- or 7-bit side (T = 8 on 5 + 5 bits 596 / 611; on preset F 598 / 577, with three spilled registers more))
-        constexpr bool roomy = NP < 3 || !(KB == 6 || KB == 7 || VB == 6 || VB == 7);
-        const int tid = (KB == 8 && VB == 8) || (APPEND && roomy) ? (int) threadIdx.x : 64 * wv + lane;
+        // the thread by the opaque lane: threadIdx.x would be held, spilled, across the tile loop.  The kernels that have a register
+        // for it lose to spilled scalars without it: q8 on both sides 3-6%; one and two row groups, two workgroups per CU, 1% (T =
+        // 2, 16 layers of 9,001 positions, 6 + 5 bits 236 us with it, 239 without) and up to 5% with the fused append (preset F
+        // 261 / 276); of the fused ones of three groups those without a 6- or 7-bit side (T = 8 on 5 + 5 bits 596 / 611; on preset F
+        // 598 / 577, with three spilled registers more)
+        constexpr bool roomy = NP < 3 ? !SMALL : APPEND && !(KB == 6 || KB == 7 || VB == 6 || VB == 7);
+        const int tid = (KB == 8 && VB == 8) || roomy ? (int) threadIdx.x : 64 * wv + lane;
         constexpr int NPASS = (NP + 1) / 2;
 #pragma unroll
         for (int ps = 0; ps < NPASS; ps++) {
