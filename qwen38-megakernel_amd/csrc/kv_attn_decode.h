@@ -336,8 +336,7 @@ __device__ __forceinline__ TileSrc tile_src(const Geo & S, const SideLayout & SK
 // copies of one tile into the stage at LDS address `lds` (KB + VB + 1 copy instructions per lane).
 // Full tiles copy contiguous bytes (one address add per instruction); the last, partial tile of a context clamps each
 // 16-byte chunk to the last valid row.
-// PART: 0 = the whole tile, 1 = the K rows and scales, 2 = the V rows and scales (two waves sharing one stage, each
-// copying what it stores in a fused append)
+// PART: 0 = the whole tile, 1 = the K rows and scales, 2 = the V rows and scales (two waves sharing one stage)
 template <int KB, int VB, int PART = 0, bool NT = true>
 __device__ __forceinline__ void issue_tile(const TileSrc & t, int nv, unsigned lds, int lane) {
     constexpr int KR = 2 * KB, VR = 2 * VB; // 16-byte chunks per row
@@ -1162,8 +1161,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SMALL ? 3 :
         // the thread by the opaque lane: threadIdx.x would be held, spilled, across the tile loop.  The kernels that have a register
         // for it lose to spilled scalars without it: q8 on both sides 3-6%; one and two row groups, two workgroups per CU, 1% (T =
         // 2, 16 layers of 9,001 positions, 6 + 5 bits 236 us with it, 239 without) and up to 5% with the fused append (preset F
-        // 261 / 276); of the fused ones of three groups those without a 6- or 7-bit side (T = 8 on 5 + 5 bits 596 / 611; on preset F
-        // 598 / 577, with three spilled registers more)
+        // 261 / 276).  The fused ones of three groups spill four or five registers with it: without a 6- or 7-bit side that still
+        // costs less than the scalars (T = 8 on 5 + 5 bits 596 with it, 611 without; on preset F 598 / 577)
         constexpr bool roomy = NP < 3 ? !SMALL : APPEND && !(KB == 6 || KB == 7 || VB == 6 || VB == 7);
         const int tid = (KB == 8 && VB == 8) || roomy ? (int) threadIdx.x : 64 * wv + lane;
         constexpr int NPASS = (NP + 1) / 2;

@@ -1,5 +1,5 @@
-"""The unpack step of the packed formats (csrc/kv_codes.h, compiled for the host): for every B = 4..7, nibbles and high
-bits of every value position, the magic pair read as fp16 plus its bias is the signed code exactly, in the order
+"""The unpack step of the packed formats (csrc/kv_codes.h, compiled for the host): for every B = 4..7 and every code
+at every value position (between random neighbours), the magic pair read as fp16 plus its bias is the signed code exactly, in the order
 pair_at states, whatever the bits around the word's high field."""
 import ctypes
 import os
