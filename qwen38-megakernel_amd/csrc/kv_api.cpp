@@ -899,7 +899,7 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
         // The whole workspace is held before anything is stored: a call that cannot have it changes nothing.  What does not
         // fit the device (or the scratch knob) is tried in the next smaller shape: one piece and one layer per launch, then
         // one layer's tiles at a time, then fewer kv heads' -- the same bits in all.
-        size_t part_need = 0, ml_need = 0;
+        size_t part_need = 0, ml_need = 0, q_tail = 0; // q_tail: query operands behind the tiles
         auto units = [&]() { return sh.keep ? (size_t) n_layers * NKV : (size_t) sh.ng; };
         bool held = false;
         for (int step = 0; !held; step++) {
@@ -910,15 +910,21 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
             else if (sh.keep) sh.keep = false;
             else if (sh.ng > 1) sh.ng /= 2;
             else
-                throw std::runtime_error("no device memory for the prefill's workspace of " + std::to_string(units() * (unit + qunit) + part_need + ml_need) +
+                throw std::runtime_error("no device memory for the prefill's workspace of " + std::to_string(units() * (unit + qunit) + q_tail + part_need + ml_need) +
                                          " bytes");
-            part_need = ml_need = 0;
+            part_need = ml_need = q_tail = 0;
             walk([](int, int) {},
                  [&](int, int, int, size_t n) {
-                     part_need = std::max(part_need, n * HD * sizeof(float) + (size_t) p.nl * sh.ng * p.q_blocks * Q16_BLOCK);
+                     const size_t q16 = (size_t) p.nl * sh.ng * p.q_blocks * Q16_BLOCK;
+                     part_need = std::max(part_need, n * HD * sizeof(float) + q16);
                      ml_need = std::max(ml_need, n * sizeof(float2));
+                     q_tail = std::max(q_tail, q16);
                  });
-            const size_t kv16_need = units() * (unit + qunit);
+            // (the queries go behind the partials; a call without partials takes no buffer for them alone, whose allocation would
+            // cost a first call 25 us)
+            if (ml_need) q_tail = 0;
+            else part_need = 0;
+            const size_t kv16_need = units() * (unit + qunit) + q_tail;
             if (s.prefill_scratch && kv16_need + part_need + ml_need > s.prefill_scratch) continue;
             // (in_capture: the tiles grow with the context, so a program that captures its chunks one after another, warmed up on
             // the first, allocates inside every capture that goes further than any call before it)
@@ -975,7 +981,7 @@ static int prefill_impl(void * h, int seq, int layer0, int n_layers, int pos, in
             },
             [&](int l, int, int a0, size_t n) {
                 set_tiles(l);
-                p.q16 = static_cast<uint8_t *>(s.part) + n * HD * sizeof(float); // (the queries after the partials)
+                p.q16 = ml_need ? static_cast<uint8_t *>(s.part) + n * HD * sizeof(float) : kv16 + units() * (unit + qunit);
                 const size_t trow = (size_t) l * T + a0; // first token row of the group in this run's block
                 p.q = q + trow * NH * qs;
                 p.qnw = qnw ? qnw + (size_t) l * HD : nullptr;

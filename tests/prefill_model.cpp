@@ -107,7 +107,10 @@ hipError_t launch_prefill(PrefillArgs & a, hipStream_t) {
     }
     inside(a.part, part * HD * 4, "partials");
     inside(a.ml, part * sizeof(float2), "partial sums");
-    if (a.q_blocks && (const uint8_t *) (a.part + part * HD) > a.q16) fail("query operands inside the partials");
+    const uint8_t * const q0 = a.q16, * const q1 = q0 + (size_t) a.nl * a.ng * a.q_blocks * Q16_BLOCK;
+    if (q0 != q1 && part && q0 < (const uint8_t *) (a.part + part * HD) && q1 > (const uint8_t *) a.part) fail("query operands inside the partials");
+    for (const auto & x : tiles_)
+        if (q0 != q1 && (size_t) q1 > x.first && (size_t) q0 < x.first + KV16_TILE) fail("query operands inside the tiles");
     return hipSuccess;
 }
 hipError_t launch_ring_refill(const StoreLayout & S, int, int nl, int p0, int p1, hipStream_t) {
@@ -160,6 +163,7 @@ int model_capture(int on) {
     return mode_ == hipStreamCaptureModeGlobal;
 }
 size_t model_used(void) { return used_; }
+int model_allocations(void) { return (int) live_.size(); }
 void model_begin(const float * out) {
     out0_ = out;
     done_.clear();

@@ -183,3 +183,12 @@ def test_every_unpacked_tile_is_read(lib, spec, win, nl, pos, T):
     assert isinstance(st.prefill(pos, T), tuple)
     assert lib.model_unread() <= 4 * nl * (win > 0 and pos % 32 != 0)
     st.close()
+
+
+def test_a_short_prompt_takes_one_buffer(lib):
+    # rows of one key segment have no partials: their prepared queries take room behind the tiles, not a buffer of their own
+    st = Store(lib, F, 2048, 2, 1280)
+    n = lib.model_allocations()
+    assert isinstance(st.prefill(0, 100), tuple)
+    assert lib.model_allocations() - n == 1
+    st.close()
